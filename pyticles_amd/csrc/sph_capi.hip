@@ -210,6 +210,7 @@ struct Arena {
     std::vector<BoxDesc> boxes;
     std::vector<int> box_live;
     std::vector<SegDesc> segs;
+    std::vector<BoxDesc> sent;  // what d_boxes holds (send_boxes)
     BoxDesc *d_boxes = nullptr;
     BoxDyn *d_dyn = nullptr;
     SegDesc *d_segs = nullptr;
@@ -287,6 +288,8 @@ struct Arena {
     bool graph_sig_set = false;
     int use_graph = 1;
     int always_build = 0;  // arenas: build stage every step (per-box schedule on device)
+    int one_box = -1;          // the box owning every slot in use, or -1 (set by relayout)
+    int sums = SUMS_MIXED;     // the live boxes' summation orders (set by relayout)
     bool small_boxes = false;  // all live boxes fit the per-box sort (set by relayout)
     int unroll = 0;        // list entries in flight per lane in the pair passes (0 = default)
     int pass_block = 256;  // work-items per block of the pair passes (128, 256, 512)
@@ -317,6 +320,8 @@ struct Arena {
         A.nkeys = nkeys;
         A.cap = cap;
         A.lcap = lcap;
+        A.one_box = one_box;
+        A.sums = sums;
         A.pass_block = pass_block;
         return A;
     }
@@ -326,7 +331,8 @@ struct Arena {
         cap = capacity;
         precision = prec;
         lcap = list_entries;
-        if (lcap <= 0 || lcap % 8) return fail(SPH_ERR_ARG, "list entries must be a positive multiple of 8");
+        // 32: the four lanes that may share a list read whole 8-entry groups
+        if (lcap < 64 || lcap % 32) return fail(SPH_ERR_ARG, "list entries must be a multiple of 32, at least 64");
         // the pair walks gather neighbour records (up to 32 bytes) through
         // 32-bit byte offsets
         if (cap > (1 << 27)) return fail(SPH_ERR_ARG, "arena capacity above 2^27 slots");
@@ -434,6 +440,7 @@ struct Arena {
             dfree(d_dyn);
             dfree(box_coff);
             d_boxes = nb;
+            sent.clear();
             d_dyn = nd;
             box_coff = nco;
             BoxDyn *nh = nullptr;
@@ -562,6 +569,26 @@ struct Arena {
         return SPH_OK;
     }
 
+    // Bring the device's box table up to date: the range of entries that
+    // differ from what was last sent (adding a box to an arena changes one
+    // entry; the whole table of a large arena is a slow pageable copy).
+    int send_boxes()
+    {
+        size_t lo = 0, hi = boxes.size();
+        if (sent.size() == hi) {
+            while (lo < hi && memcmp(&boxes[lo], &sent[lo], sizeof(BoxDesc)) == 0) ++lo;
+            while (hi > lo && memcmp(&boxes[hi - 1], &sent[hi - 1], sizeof(BoxDesc)) == 0) --hi;
+        } else if (sent.size() < hi) {
+            while (lo < sent.size() && memcmp(&boxes[lo], &sent[lo], sizeof(BoxDesc)) == 0) ++lo;
+        }
+        if (lo >= hi) return SPH_OK;
+        sent.clear();  // until the copy is queued
+        HIPCHK(hipMemcpyAsync(d_boxes + lo, boxes.data() + lo, sizeof(BoxDesc) * (hi - lo), hipMemcpyHostToDevice,
+                              ctx->stream));
+        sent = boxes;
+        return SPH_OK;
+    }
+
     // Recompute key bases in slot order, the high-water mark, and upload the
     // box and segment tables.
     int relayout()
@@ -584,8 +611,14 @@ struct Arena {
         nkeys = key;
         // every live box small enough for the per-box sort: no global sort
         small_boxes = true;
-        for (size_t i = 0; i < boxes.size(); ++i)
-            if (box_live[i] && !box_sort_fits(boxes[i].ncx * boxes[i].ncy, boxes[i].n)) small_boxes = false;
+        bool any_groups = false, any_plain = false;
+        for (size_t i = 0; i < boxes.size(); ++i) {
+            if (!box_live[i]) continue;
+            if (!box_sort_fits(boxes[i].ncx * boxes[i].ncy, boxes[i].n)) small_boxes = false;
+            (boxes[i].n > SUM_GROUP_MAX ? any_plain : any_groups) = true;
+        }
+        one_box = !segs.empty() && segs[0].box >= 0 && segs[0].len == hwm ? segs[0].box : -1;
+        sums = any_groups && any_plain ? SUMS_MIXED : (any_plain ? SUMS_PLAIN : SUMS_GROUPS);
         if (nkeys + 1 > cell_cap) {
             int nc = std::max(nkeys + 1, cell_cap * 2);
             dfree(cell_start);
@@ -601,9 +634,7 @@ struct Arena {
             invalidate_graph();
         }
         if (ensure_tables((int)boxes.size())) return SPH_ERR_NOMEM;
-        if (!boxes.empty())
-            HIPCHK(hipMemcpyAsync(d_boxes, boxes.data(), sizeof(BoxDesc) * boxes.size(), hipMemcpyHostToDevice,
-                                  ctx->stream));
+        if (int rc = send_boxes()) return rc;
         HIPCHK(hipMemcpyAsync(d_segs, segs.data(), sizeof(SegDesc) * segs.size(), hipMemcpyHostToDevice,
                               ctx->stream));
         launch_slot_box(view(), ctx->stream);
@@ -960,7 +991,7 @@ struct Arena {
             if (!box_live[b] || !h_dyn[b].relist) continue;
             host_dyn_ok = false;
             boxes[b].build16 = 0;
-            HIPCHK(hipMemcpyAsync(d_boxes + b, &boxes[b], sizeof(BoxDesc), hipMemcpyHostToDevice, ctx->stream));
+            if (int rc = send_boxes()) return rc;
             HIPCHK(hipMemcpyAsync((char *)(d_dyn + b) + offsetof(BoxDyn, relist), &zero, sizeof(int),
                                   hipMemcpyHostToDevice, ctx->stream));
             h_dyn[b].relist = 0;
@@ -1043,6 +1074,16 @@ int fill_desc(const sph_params *p, int64_t n, BoxDesc &B)
     B.qhl = 5.0 / (PI * p->hl * p->hl);
     B.fh = -12.0 * B.qh / (p->h * p->h);    // spkernel.py:112-113, factored
     B.fhl = -12.0 * B.qhl / (p->hl * p->hl);
+    B.cutl = std::min(B.cut2, B.hl2); B.cuth = std::min(B.cut2, B.h2);
+    B.iLx = 1.0 / B.Lx; B.iLy = 1.0 / B.Ly;
+    B.ih3 = 3.0 * B.ih; B.ihl3 = 3.0 * B.ihl;
+    const double FIX48 = 281474976710656.0, FIX32 = 4294967296.0;  // 2^48, 2^32
+    B.fx48 = FIX48 / B.Lx; B.fy48 = FIX48 / B.Ly;
+    B.sclx = B.Lx / FIX32; B.scly = B.Ly / FIX32;
+    B.s48x = B.Lx / FIX48; B.s48y = B.Ly / FIX48;
+    B.cutsd = std::min(B.R2list, B.h2);
+    B.cutlf = (float)B.cutl; B.ihlf = (float)B.ihl; B.qhlf = (float)B.qhl; B.fhlf = (float)B.fhl;
+    B.ihl3f = (float)B.ihl3;
     B.a = p->a; B.b = p->b; B.kB = p->kB; B.eta = p->eta; B.zeta = p->zeta; B.kcond = p->kcond;
     B.dt = p->dt;
     B.n = (int)n;
@@ -1151,7 +1192,7 @@ int Arena::upload(int b, int field, const double *host, int ncomp)
         bool uni = n > 0 && host[0] > 0.0 && std::isfinite(host[0]);
         for (int i = 1; uni && i < n; ++i) uni = host[i] == host[0];
         boxes[b].munif = uni ? host[0] : 0.0;
-        HIPCHK(hipMemcpyAsync(d_boxes + b, &boxes[b], sizeof(BoxDesc), hipMemcpyHostToDevice, ctx->stream));
+        if (int rc = send_boxes()) return rc;
     }
     // the pageable source is staged before the copy call returns and the
     // staging buffer is reused in stream order: no wait
@@ -1804,7 +1845,7 @@ int sph_arena_add(sph_arena *ar, int64_t n, const sph_params *prm, const double 
     int b = -1;
     if (int rc = A.add_box(n, prm, &b)) return rc;
     A.boxes[b].T0 = T0;
-    HIPCHK(hipMemcpyAsync(A.d_boxes + b, &A.boxes[b], sizeof(BoxDesc), hipMemcpyHostToDevice, A.ctx->stream));
+    if (int rc = A.send_boxes()) return rc;
     if (int rc = A.upload(b, 0, r, 2)) return rc;
     if (int rc = A.upload(b, 1, v, 2)) return rc;
     if (int rc = A.upload(b, 2, m, 1)) return rc;
@@ -2175,9 +2216,7 @@ static int set_list_bits(Arena &A, int bits)
     A.list_bits = bits;
     for (size_t b = 0; b < A.boxes.size(); ++b)
         if (A.box_live[b]) A.boxes[b].build16 = bits == 16 ? 1 : 0;
-    if (!A.boxes.empty())
-        HIPCHK(hipMemcpyAsync(A.d_boxes, A.boxes.data(), sizeof(BoxDesc) * A.boxes.size(), hipMemcpyHostToDevice,
-                              A.ctx->stream));
+    if (int rc = A.send_boxes()) return rc;
     return SPH_OK;
 }
 

@@ -54,6 +54,12 @@ enum Health : int {
 // bits too, as the short-range terms always do.
 constexpr double FP32C_HI_ONLY_MAX_L = 1024.0;
 
+// Summation order of a box's pair passes: boxes of up to SUM_GROUP_MAX slots
+// sum in groups of eight entries (so that lanes may share a list), larger
+// ones in plain running order.  What a launch's boxes take:
+constexpr int SUM_GROUP_MAX = 98304;
+enum : int { SUMS_PLAIN = 0, SUMS_GROUPS = 1, SUMS_MIXED = 2 };
+
 // Static description of one box (host-owned, uploaded when it changes).
 struct BoxDesc {
     double Lx, Ly, hLx, hLy;       // sides and half sides (minimum image)
@@ -68,6 +74,14 @@ struct BoxDesc {
     double munif;                  // the common mass when all masses are equal, else 0
     double rin;                    // interior margin 2 (r_cut + skin): a particle at least this far
                                    // from every side has no listed neighbour across a side
+    // derived once here, read as they are by the passes
+    double cutl, cuth, iLx, iLy;   // min(cut2, hl2), min(cut2, h2), 1 / sides
+    double ih3, ihl3;              // 3 / h, 3 / h_l: 1 + 3q = fma(r, 3 / h, 1)
+    double fx48, fy48;             // FP32C: 2^48 / sides (fix_rec)
+    double sclx, scly, s48x, s48y; // FP32C: sides / 2^32 and / 2^48, the units of its separations
+    double cutsd;                  // FP32C: short-range cut min(R2list, h2)
+    float cutlf, ihlf, qhlf, fhlf, ihl3f;  // FP32C: cutl, ihl, qhl, fhl, ihl3
+    float padf;
     int ncx, ncy, sx, sy;          // cell grid and stencil half widths (0/1)
     int key_base, part_off, n, terms;
     int precision;
@@ -191,6 +205,8 @@ struct ArenaView {
     int nkeys;           // total keys
     int cap;             // slot capacity
     int lcap;            // list entries per slot
+    int one_box;         // the box that owns every slot in use, or -1 (several, or free slots)
+    int sums;            // summation orders of the live boxes (SUMS_*)
     int pass_block;      // work-items per block of the pair passes (128, 256 or 512)
 };
 

@@ -50,6 +50,17 @@ __device__ __forceinline__ int xcd_block()
 
 __device__ __forceinline__ int wrapi(int c, int n) { return c < 0 ? c + n : (c >= n ? c - n : c); }
 
+// A box's constants and state through the scalar path: a pass reads them by a
+// wave-uniform box index and no launch that does changes them (but for the
+// health bits, which it only sets), so they load into scalar registers, all
+// at once and beside the wave's vector loads.  (Read lane by lane, test by
+// test, they were a chain of dependent loads, about nine memory latencies
+// from a wave's start to its first gather.)
+using CBox = const __attribute__((address_space(4))) BoxDesc;
+using CDyn = const __attribute__((address_space(4))) BoxDyn;
+__device__ __forceinline__ CBox &cbox(const ArenaView &A, int bu) { return *(CBox *)(A.boxes + bu); }
+__device__ __forceinline__ CDyn &cdyn(const ArenaView &A, int bu) { return *(CDyn *)(A.dyn + bu); }
+
 // Wave-uniform values: a value the lanes agree on, moved to a scalar
 // register (readfirstlane).
 __device__ __forceinline__ double wave_uniform(double x)
@@ -133,22 +144,6 @@ __device__ __forceinline__ void load_entries(const unsigned *base, int P0, unsig
     }
 }
 
-// 16-bit form: entry i of the U in the low (i even) or high (i odd) half
-// of w[i / 2].
-template <int U>
-__device__ __forceinline__ void load_entries16(const unsigned short *base, int P0, unsigned (&w)[U])
-{
-    const unsigned short *p = base + pos16(P0);
-    if constexpr (U == 4) {
-        const uint2 g = *(const uint2 *)p;
-        w[0] = g.x; w[1] = g.y;
-    } else if constexpr (U == 2) {
-        w[0] = *(const unsigned *)p;
-    } else {
-        w[0] = *p;
-    }
-}
-
 // Entry form of a wave's lists, one of
 //   LF32: 32-bit slots;
 //   LF16: 16-bit offsets whose plain sum with the slot is the neighbour;
@@ -162,16 +157,24 @@ struct ListFmt {
     int form;
 };
 
-// The lists of the box bu that the wave's active lanes belong to.
-__device__ __forceinline__ ListFmt list_fmt(const ArenaView &A, int bu, int s)
+// The lists of the box bu that the wave's active lanes belong to (cx: the
+// lane's short count word).
+__device__ __forceinline__ ListFmt list_fmt(const CBox &B, const CDyn &D, int cx)
 {
     ListFmt f;
-    f.lo = wave_uniform(A.boxes[bu].part_off);
-    f.nb = wave_uniform(A.boxes[bu].n);
+    f.lo = B.part_off;
+    f.nb = B.n;
     f.hi = f.lo + f.nb;
-    const bool w16 = wave_uniform(A.dyn[bu].list16) != 0;
-    f.form = !w16 ? LF32 : (__ballot(A.cnt[s].x < 0) != 0ull ? LF16W : LF16);
+    f.form = D.list16 == 0 ? LF32 : (__ballot(cx < 0) != 0ull ? LF16W : LF16);
     return f;
+}
+
+// A slot's first cell of short (or, LONG, long) entries in the 16-bit form,
+// for the lane's first group of a shared list: its address needs nothing but
+// the slot, so a pass issues it before it knows the slot's box.
+__device__ __forceinline__ uint4 first_cell(const ArenaView &A, int s, bool LONG, int group)
+{
+    return *(const uint4 *)(list_base16(A, s) + (size_t)(LONG ? (A.lcap >> 3) - 1 - group : group) * CELL16);
 }
 
 // Calls f with the wave's form as a compile-time constant.
@@ -185,34 +188,40 @@ __device__ __forceinline__ void with_form(const ListFmt &L, Fn f)
 
 // A slot's short (LONG = false) or long entries, U per round (k0 a multiple
 // of U; long entry k sits at position lcap - 1 - k), in list form LF.
-// take(k0, t) gives the slots of round k0.  With AHEAD, next(k0) issues the
-// load of the next round's group, so that list fetch is in flight while
-// round k0's neighbour records are gathered and summed; at the last round it
-// re-reads the current group, so every load stays inside the slot's list
-// rows.  Without AHEAD, take() loads its own round's group.  Entries past the
-// count read as s (a valid record whose terms the callers mask off), so the
-// gathers need no branch.  AHEAD pays on the density walks (~15 rounds per
-// slot); on the short walks of the gradient and rate passes (3-4 rounds) its
-// extra load and registers cost more than the overlap gains.
-template <int U, bool LONG, bool AHEAD, int LF>
+// take(k0, t) gives the slots of round k0.  16-bit entries come a 16-byte
+// cell (eight entries) at a time, the first cell given (first_cell).  With
+// AHEAD, next(k0) issues the load of the next cell (32-bit form: the next
+// round's group), so that list fetch is in flight while this cell's
+// neighbour records are gathered and summed; at the last one it re-reads the
+// current cell, so every load stays inside the slot's list rows.  Without
+// AHEAD, take() loads its own cell or group.  Entries past the count read as
+// s (a valid record whose terms the callers mask off), so the gathers need no
+// branch.  AHEAD pays on the density walks (~15 rounds per slot); on the
+// short walks of the gradient and rate passes (3-4 rounds) its extra load and
+// registers cost more than the overlap gains.
+//
+// With S > 1 the S lanes of a particle take its groups of eight entries in
+// turn (lane i the groups i, i + S, ...): first is the lane's own first entry
+// and next() steps from one of its groups to the next.
+template <int U, bool LONG, bool AHEAD, int LF, int S = 1>
 struct ListRounds {
-    // 16-bit entries four per round: one 16-byte cell (8 entries) serves a
-    // pair of rounds, so a cell load every other round (issued, with AHEAD,
-    // two rounds before its use); c holds the current cell
-    static constexpr bool PAIRS = LF != LF32 && U == 4;
+    static constexpr bool CELLS = LF != LF32;
     const unsigned *base;
     const unsigned short *base16;
     int lcap, n, s, lo, hi, nb;
-    unsigned w[U];
-    unsigned c[PAIRS ? 4 : 1];
-    __device__ __forceinline__ ListRounds(const ArenaView &A, int s_, int n_, const ListFmt &L)
-        : lcap(A.lcap), n(n_), s(s_), lo(L.lo), hi(L.hi), nb(L.nb)
+    unsigned w[CELLS ? 4 : U];  // the next cell or group
+    unsigned c[CELLS ? 4 : 1];  // the current cell
+    bool given;                 // w is the first cell, not yet taken (without AHEAD)
+    // first < 8 S <= 32 entries: inside the slot's rows (lcap >= 64)
+    __device__ __forceinline__ ListRounds(const ArenaView &A, int s_, int n_, const ListFmt &L, uint4 g, int first = 0)
+        : lcap(A.lcap), n(n_), s(s_), lo(L.lo), hi(L.hi), nb(L.nb), given(true)
     {
-        if (LF == LF32) base = list_base(A, s_);
-        else base16 = list_base16(A, s_);
-        if (AHEAD) {
-            if constexpr (PAIRS) load_cell(cell(0), w);
-            else load(pos(0));
+        if constexpr (CELLS) {
+            base16 = list_base16(A, s_);
+            w[0] = g.x; w[1] = g.y; w[2] = g.z; w[3] = g.w;
+        } else {
+            base = list_base(A, s_);
+            if (AHEAD) load(pos(first));
         }
     }
     __device__ __forceinline__ int pos(int k0) const { return LONG ? lcap - k0 - U : k0; }
@@ -223,11 +232,7 @@ struct ListRounds {
         const uint4 g = *(const uint4 *)(base16 + (size_t)q * CELL16);
         d[0] = g.x; d[1] = g.y; d[2] = g.z; d[3] = g.w;
     }
-    __device__ __forceinline__ void load(int P0)
-    {
-        if constexpr (LF == LF32) load_entries<U>(base, P0, w);
-        else load_entries16<U>(base16, P0, w);
-    }
+    __device__ __forceinline__ void load(int P0) { load_entries<U>(base, P0, w); }
     __device__ __forceinline__ int decode(unsigned x, int half) const
     {
         int e = s + (half ? ((int)x >> 16) : ((int)(x << 16) >> 16));
@@ -239,52 +244,147 @@ struct ListRounds {
     }
     __device__ __forceinline__ void take(int k0, int (&t)[U])
     {
-        if constexpr (PAIRS) {
-            if ((k0 & 4) == 0) {  // first round of a cell
-                if constexpr (AHEAD) {
+        if constexpr (CELLS) {
+            if ((k0 & 7) == 0) {  // first round of a cell
+                if (AHEAD || given) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i) c[i] = w[i];
+                    given = false;
                 } else {
-                    load_cell(cell(k0), c);
+                    load_cell(cell(S == 1 || k0 < n ? k0 : 0), c);
                 }
             }
-            // short rounds take offsets 0-3 then 4-7 of the cell, long
-            // rounds 7-4 then 3-0 (the half picked by selects: a register
-            // array indexed at run time would live in scratch memory)
-            const bool hi4 = LONG ? ((k0 & 4) == 0) : ((k0 & 4) != 0);
-            const unsigned x0 = hi4 ? c[2] : c[0], x1 = hi4 ? c[3] : c[1];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int o = LONG ? 3 - u : u;  // offset within the half
-                t[u] = k0 + u < n ? decode(o < 2 ? x0 : x1, o & 1) : s;
+            // the round's words, picked by selects (a register array indexed
+            // at run time would live in scratch memory): short rounds go up
+            // the cell, long ones down
+            const int o0 = LONG ? 8 - U - (k0 & 7) : (k0 & 7);  // lowest offset of the round
+            unsigned x[2];
+            if constexpr (U == 4) {
+                x[0] = o0 ? c[2] : c[0];
+                x[1] = o0 ? c[3] : c[1];
+            } else {
+                const unsigned a = (o0 & 2) ? c[1] : c[0], b = (o0 & 2) ? c[3] : c[2];
+                x[0] = x[1] = (o0 & 4) ? b : a;
+                if (U == 1) x[0] = (o0 & 1) ? x[0] >> 16 : x[0];
             }
-            return;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int o = LONG ? U - 1 - u : u;  // offset within the round
+                t[u] = k0 + u < n ? decode(x[o >> 1], o & 1) : s;
+            }
         } else {
-            if (!AHEAD) load(pos(k0));
+            if (!AHEAD) load(pos(S == 1 || k0 < n ? k0 : 0));
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int i = LONG ? U - 1 - u : u;
-                int e;
-                if constexpr (LF == LF32) e = (int)w[i];
-                else e = decode(w[i >> 1], i & 1);
-                t[u] = k0 + u < n ? e : s;
+                t[u] = k0 + u < n ? (int)w[i] : s;
             }
         }
     }
     // issued after round k0's gathers, so waiting for them does not wait for
-    // this load too (loads retire in order); at the last round it re-reads
-    // the current group or cell, so every load stays inside the slot's rows
+    // this load too (loads retire in order)
     __device__ __forceinline__ void next(int k0)
     {
         if constexpr (AHEAD) {
-            if constexpr (PAIRS) {
-                if ((k0 & 4) == 0) load_cell(cell(k0 + 8 < n ? k0 + 8 : k0), w);
+            if constexpr (CELLS) {
+                if ((k0 & 7) == 0) load_cell(cell(k0 + 8 * S < n ? k0 + 8 * S : k0), w);
             } else {
-                load(pos(k0 + U < n ? k0 + U : k0));
+                const int kn = S == 1 || ((k0 + U) & 7) != 0 ? k0 + U : k0 + U + 8 * (S - 1);
+                load(pos(kn < n ? kn : k0));
             }
         }
     }
 };
+
+// The FP64 sums over a list run in groups of eight entries: a group's terms
+// add into partial sums from zero, and the groups' partial sums add to the
+// totals in group order.  The order does not depend on who takes the groups,
+// so a particle's list may be walked by one lane or shared by S neighbouring
+// lanes (1, 2 or 4) with the same bits; every lane of a particle ends with
+// the totals.  (A group past the count adds +0, which changes no total: the
+// totals start at +0 and never become -0.)
+//
+// Lane l of the particle's S lanes to all of them.
+template <int S>
+__device__ __forceinline__ int lane_bcast(int x, int l)
+{
+    // DPP quad permutations (the S lanes of a particle are neighbours)
+    if constexpr (S == 2) return l == 0 ? __builtin_amdgcn_mov_dpp(x, 0xA0, 0xf, 0xf, true) : __builtin_amdgcn_mov_dpp(x, 0xF5, 0xf, 0xf, true);
+    else if constexpr (S == 4)
+        return l == 0 ? __builtin_amdgcn_mov_dpp(x, 0x00, 0xf, 0xf, true)
+             : l == 1 ? __builtin_amdgcn_mov_dpp(x, 0x55, 0xf, 0xf, true)
+             : l == 2 ? __builtin_amdgcn_mov_dpp(x, 0xAA, 0xf, 0xf, true)
+                      : __builtin_amdgcn_mov_dpp(x, 0xFF, 0xf, 0xf, true);
+    else return x;
+}
+
+template <int S>
+__device__ __forceinline__ float lane_bcast(float x, int l) { return __int_as_float(lane_bcast<S>(__float_as_int(x), l)); }
+
+template <int S>
+__device__ __forceinline__ double lane_bcast(double x, int l)
+{
+    const long long v = __double_as_longlong(x);
+    const unsigned lo = (unsigned)lane_bcast<S>((int)(v & 0xffffffffll), l);
+    const unsigned hi = (unsigned)lane_bcast<S>((int)(v >> 32), l);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// Adds the lanes' group sums p to the totals d in group order and clears p.
+template <int S, int N>
+__device__ __forceinline__ void fold_groups(double (&d)[N], double (&p)[N])
+{
+#pragma unroll
+    for (int l = 0; l < S; ++l)
+#pragma unroll
+        for (int i = 0; i < N; ++i) d[i] += lane_bcast<S>(p[i], l);
+#pragma unroll
+    for (int i = 0; i < N; ++i) p[i] = 0.0;
+}
+
+// Walks n list entries in rounds of U, eight-entry groups dealt to the S
+// lanes of the particle: round(k0) takes entries k0 .. k0 + U - 1 of the
+// lane's group (some or all past n for the later lanes), fold() follows each
+// group.  Without GROUPS (one lane) the rounds follow each other and the
+// partial sums, folded once, are the plain running sums.
+template <int U, int S, bool GROUPS, class Round, class Fold>
+__device__ __forceinline__ void for_rounds(int n, int sub, Round round, Fold fold)
+{
+    static_assert(GROUPS || S == 1, "shared lists sum in groups");
+    if constexpr (!GROUPS) {
+        for (int k0 = 0; k0 < n; k0 += U) round(k0);
+    } else {
+        int c = 0;
+        for (;;) {
+            const int g = S == 1 ? c : (c >> 3) * (8 * S) + (c & 7);
+            if (g >= n) break;
+            round(S == 1 ? g : g + 8 * sub);
+            c += U;
+            if ((c & 7) == 0) fold();
+        }
+        if ((c & 7) != 0) fold();
+    }
+}
+
+// Boxes of up to SUM_GROUP_MAX slots sum in groups, whatever lanes their
+// launch gives a list (lanes_per_slot shares lists only among so many slots);
+// larger ones, which are never shared, keep plain running sums: the group
+// sums' extra adds and registers cost their density pass 2 %.  A launch knows
+// which sums its boxes take (ArenaView::sums), so that the common launches
+// hold the code of one form.
+//
+// Calls f with whether the wave's box sums in groups, and its lists' form, as
+// compile-time constants.
+template <int SUMS, class Fn>
+__device__ __forceinline__ void with_walk(const ListFmt &L, Fn f)
+{
+    with_form(L, [&](auto lf) {
+        if constexpr (SUMS == SUMS_PLAIN) f(lf, std::integral_constant<bool, false>());
+        else if constexpr (SUMS == SUMS_GROUPS) f(lf, std::integral_constant<bool, true>());
+        else if (L.nb > SUM_GROUP_MAX) f(lf, std::integral_constant<bool, false>());
+        else f(lf, std::integral_constant<bool, true>());
+    });
+}
 
 // Record j of array p through a 32-bit byte offset from the array's base,
 // which the walks hold in scalar registers: the gather is then a
@@ -347,7 +447,8 @@ __device__ __forceinline__ void flag_health(BoxDyn *dyn, int b, int bits) { atom
 // A box rebuilds its cell order and neighbour list in this launch when it is
 // initialising, when its running schedule says so, or when forced (the
 // stand-alone passes build every box whose state is in force_mask).
-__device__ __forceinline__ bool building(const BoxDyn &D, int force_mask)
+template <class Dyn>
+__device__ __forceinline__ bool building(const Dyn &D, int force_mask)
 {
     if (state_in(D.state, force_mask)) return true;
     return D.state == BOX_INIT || (D.state == BOX_RUN && D.k >= D.next_rebuild);
@@ -372,35 +473,34 @@ __device__ __forceinline__ void max_bits(unsigned long long *addr, double x)
 // recorded positions exactly (units of side / 2^48: 1.8e-12 at 512), which
 // the short-range terms take in FP64.  Coordinates are in [0, L); one that
 // rounds up to L wraps to 0, as the box does.
-static constexpr double FIX48 = 281474976710656.0;  // 2^48
-static constexpr double FIX32 = 4294967296.0;       // 2^32
-
-__device__ __forceinline__ void fix_rec(double2 r, double2 v, const BoxDesc &B, float4 &hi, unsigned &lo)
+template <class Box>
+__device__ __forceinline__ void fix_rec(double2 r, double2 v, const Box &B, float4 &hi, unsigned &lo)
 {
     const unsigned long long M = (1ull << 48) - 1ull;
-    const unsigned long long X = (unsigned long long)fmax(rint(r.x * (FIX48 / B.Lx)), 0.0) & M;
-    const unsigned long long Y = (unsigned long long)fmax(rint(r.y * (FIX48 / B.Ly)), 0.0) & M;
+    const unsigned long long X = (unsigned long long)fmax(rint(r.x * B.fx48), 0.0) & M;
+    const unsigned long long Y = (unsigned long long)fmax(rint(r.y * B.fy48), 0.0) & M;
     hi = make_float4(__uint_as_float((unsigned)(X >> 16)), __uint_as_float((unsigned)(Y >> 16)), (float)v.x,
                      (float)v.y);
     lo = (unsigned)(X & 0xffffull) | ((unsigned)(Y & 0xffffull) << 16);
 }
 
 // Runs f(bu) once for each distinct box bu among the active lanes, on the
-// lanes of that box, with bu wave-uniform (a waterfall over the boxes of the
+// lanes of that box (b >= 0), with bu wave-uniform (a waterfall over the boxes of the
 // wave: one round for all waves but those straddling a box boundary).
 template <class F>
 __device__ __forceinline__ void per_box(int b, F &&f)
 {
-    bool done = false;
-    for (;;) {
+    bool done = b < 0;
+    while (__ballot(!done) != 0ull) {
         if (!done) {
-            const int bu = __builtin_amdgcn_readfirstlane(b);
-            if (b == bu) {
-                f(bu);
+            if (b == __builtin_amdgcn_readfirstlane(b)) {
+                // read again: of the value compared above the compiler knows
+                // that it equals the lanes' b, which it would put in its
+                // place, and load per lane what the box index selects
+                f(__builtin_amdgcn_readfirstlane(b));
                 done = true;
             }
         }
-        if (__ballot(!done) == 0ull) break;
     }
 }
 
@@ -1071,39 +1171,61 @@ __global__ __launch_bounds__(NT) void k_build_lists(ArenaView A, int force_mask,
 // the loop issues no loads but the neighbour records.
 // ---------------------------------------------------------------------------
 struct BoxK {
-    double Lx, Ly, hLx, hLy;
+    double Lx, Ly;
     double cut2, h2, hl2, cutl, cuth;  // cutl = min(cut2, hl2), cuth = min(cut2, h2)
     double ih, ihl, qh, qhl, fh, fhl, munif, rin, iLx, iLy;
     double ih3, ihl3;  // 3/h, 3/h_l: 1 + 3q = fma(r, 3/h, 1)
     int terms;
 };
 
-__device__ __forceinline__ BoxK box_k(const BoxDesc &B, bool uniform)
+__device__ __forceinline__ BoxK box_k(const CBox &B)
 {
     BoxK k;
-    k.Lx = B.Lx; k.Ly = B.Ly; k.hLx = B.hLx; k.hLy = B.hLy;
+    k.Lx = B.Lx; k.Ly = B.Ly;
     k.cut2 = B.cut2; k.h2 = B.h2; k.hl2 = B.hl2;
-    k.cutl = B.cut2 < B.hl2 ? B.cut2 : B.hl2;
-    k.cuth = B.cut2 < B.h2 ? B.cut2 : B.h2;
+    k.cutl = B.cutl; k.cuth = B.cuth;
     k.ih = B.ih; k.ihl = B.ihl; k.qh = B.qh; k.qhl = B.qhl; k.fh = B.fh; k.fhl = B.fhl;
     k.munif = B.munif;
-    k.ih3 = 3.0 * B.ih; k.ihl3 = 3.0 * B.ihl;
+    k.ih3 = B.ih3; k.ihl3 = B.ihl3;
     k.rin = B.rin;
-    k.iLx = 1.0 / B.Lx;
-    k.iLy = 1.0 / B.Ly;
+    k.iLx = B.iLx; k.iLy = B.iLy;
     k.terms = B.terms;
-    if (uniform) {
-        k.Lx = wave_uniform(k.Lx); k.Ly = wave_uniform(k.Ly); k.hLx = wave_uniform(k.hLx); k.hLy = wave_uniform(k.hLy);
-        k.cut2 = wave_uniform(k.cut2); k.h2 = wave_uniform(k.h2); k.hl2 = wave_uniform(k.hl2);
-        k.cutl = wave_uniform(k.cutl); k.cuth = wave_uniform(k.cuth);
-        k.ih = wave_uniform(k.ih); k.ihl = wave_uniform(k.ihl); k.qh = wave_uniform(k.qh); k.qhl = wave_uniform(k.qhl);
-        k.fh = wave_uniform(k.fh); k.fhl = wave_uniform(k.fhl); k.munif = wave_uniform(k.munif);
-        k.rin = wave_uniform(k.rin); k.iLx = wave_uniform(k.iLx); k.iLy = wave_uniform(k.iLy);
-        k.ih3 = wave_uniform(k.ih3); k.ihl3 = wave_uniform(k.ihl3);
-        k.terms = wave_uniform(k.terms);
-    }
     return k;
 }
+
+using true_t = std::integral_constant<bool, true>;
+using false_t = std::integral_constant<bool, false>;
+
+// Slot and lane-of-slot of a pair pass that shares each list among S lanes
+// (shared lists run in blocks of NT).
+template <int S>
+__device__ __forceinline__ int pass_slot(const ArenaView &A, int &sub)
+{
+    const int g = xcd_block() * (S > 1 ? NT : A.pass_block) + threadIdx.x;
+    sub = g & (S - 1);
+    return g / S;
+}
+
+// Box of slot s, -1 past the slots in use or where it has none.  A single
+// box's arena needs no look-up.
+__device__ __forceinline__ int slot_owner(const ArenaView &A, int s)
+{
+    if (s >= A.n) return -1;
+    return A.one_box >= 0 ? A.one_box : A.slot_box[s];
+}
+
+__device__ __forceinline__ bool takes_part(const CDyn &D, int state_mask)
+{
+    return (((1 << D.state) & state_mask) != 0) & (D.relist == 0);
+}
+
+// What a pass reads of its own slot before it knows the box: issued together
+// at the wave's start (slots past the end read slot 0).
+struct Own64 {
+    double2 r, v;
+    int2 c;
+    uint4 g0, g1;  // first cells of short and of long entries
+};
 
 // ===========================================================================
 // FP64 form
@@ -1146,108 +1268,84 @@ __device__ __forceinline__ double sqrt_pair(double x)
     return x >= 1e-280 ? g : 0.0;
 }
 
-__device__ __forceinline__ double vdw_p(double rho, double T, const BoxDesc &B)
+template <class Box>
+__device__ __forceinline__ double vdw_p(double rho, double T, const Box &B)
 {
     return (rho * B.kB * T) / (1.0 - rho * B.b);  // properties.py:41
 }
 
+enum : int { D_RHO = 0, D_RHOL, D_GX, D_GY, D_EV, D_N };
 struct Dens64 {
     double rho, rhol, gx, gy, ev;
 };
 
 // P1 list walk.  COH: accumulate the cohesive terms (needs velocities);
 // UNIM: all masses equal (no mass fetch).
-template <int U64, bool COH, bool UNIM, bool WRAP, int LF>
-__device__ __forceinline__ Dens64 density64_walk(const ArenaView &A, const BoxK &K, const ListFmt &L, int s)
+template <int U64, int S, bool GRP, bool COH, bool UNIM, bool WRAP, int LF>
+__device__ __forceinline__ Dens64 density64_walk(const ArenaView &A, const BoxK &K, const ListFmt &L, int s, int sub, const Own64 &own)
 {
-    const double2 ri = A.r[s], vi = A.vp[s];
-    const int2 cr = A.cnt[s];
-    const int2 c = make_int2(cr.x & CNT_MASK, cr.y);
+    const double2 ri = own.r, vi = own.v;
+    const int2 c = make_int2(own.c.x & CNT_MASK, own.c.y);
     // the sums leave out the kernel constants (and, with UNIM, the mass);
     // they scale the totals at the end
-    Dens64 d;
-    d.rho = d.rhol = d.gx = d.gy = d.ev = 0.0;
-    // U64 entries per round: all their loads are issued before any use so
+    double t5[D_N] = {}, p[D_N] = {};
+    // one round: U64 entries, all their loads issued before any use so
     // several neighbour fetches are in flight per wavefront; one load brings
-    // a round's list entries.
-    ListRounds<U64, false, true, LF> rounds(A, s, c.x, L);
-    for (int k0 = 0; k0 < c.x; k0 += U64) {
-        int t[U64];
-        double2 rj[U64], vv[U64];
-        double mj[U64];
-        rounds.take(k0, t);
+    // a round's list entries.  Long entries lie past the short range.
+    auto walk = [&](auto &rounds, int n, auto long_t) {
+        constexpr bool LONG = decltype(long_t)::value;
+        for_rounds<U64, S, GRP>(n, sub, [&](int k0) {
+            int t[U64];
+            double2 rj[U64], vv[U64];
+            double mj[U64];
+            rounds.take(k0, t);
 #pragma unroll
-        for (int u = 0; u < U64; ++u) {
-            rj[u] = at32(A.r, t[u]);
-            if (!UNIM) mj[u] = at32(A.m, t[u]);
-            if (COH) vv[u] = at32(A.vp, t[u]);
-        }
-        rounds.next(k0);
+            for (int u = 0; u < U64; ++u) {
+                rj[u] = at32(A.r, t[u]);
+                if (!UNIM) mj[u] = at32(A.m, t[u]);
+                if (COH) vv[u] = at32(A.vp, t[u]);
+            }
+            rounds.next(k0);
 #pragma unroll
-        for (int u = 0; u < U64; ++u) {
-            double dx = rj[u].x - ri.x, dy = rj[u].y - ri.y;
-            if (WRAP) min_image_listed(dx, dy, K);
-            const double r2 = rsq_exact(dx, dy);
-            if (k0 + u < c.x && r2 < K.cut2) {
-                const double m = UNIM ? 1.0 : mj[u];
-                const double rr = sqrt_pair(r2);
-                if (r2 < K.hl2) {
-                    const double w = fma(-rr, K.ihl, 1.0), w2 = w * w;
-                    d.rhol = fma(m * fma(rr, K.ihl3, 1.0), w2 * w, d.rhol);
-                    if (COH) {
-                        const double g = m * w2;
-                        d.gx = fma(g, dx, d.gx);
-                        d.gy = fma(g, dy, d.gy);
-                        d.ev = fma(g, (vv[u].x - vi.x) * dx + (vv[u].y - vi.y) * dy, d.ev);
+            for (int u = 0; u < U64; ++u) {
+                double dx = rj[u].x - ri.x, dy = rj[u].y - ri.y;
+                if (WRAP) min_image_listed(dx, dy, K);
+                const double r2 = rsq_exact(dx, dy);
+                if (k0 + u < n && r2 < (LONG ? K.cutl : K.cut2)) {
+                    const double m = UNIM ? 1.0 : mj[u];
+                    const double rr = sqrt_pair(r2);
+                    if (LONG || r2 < K.hl2) {
+                        const double w = fma(-rr, K.ihl, 1.0), w2 = w * w;
+                        p[D_RHOL] = fma(m * fma(rr, K.ihl3, 1.0), w2 * w, p[D_RHOL]);
+                        if (COH) {
+                            const double g = m * w2;
+                            p[D_GX] = fma(g, dx, p[D_GX]);
+                            p[D_GY] = fma(g, dy, p[D_GY]);
+                            p[D_EV] = fma(g, (vv[u].x - vi.x) * dx + (vv[u].y - vi.y) * dy, p[D_EV]);
+                        }
+                    }
+                    if (!LONG && r2 < K.h2) {
+                        const double w = fma(-rr, K.ih, 1.0);
+                        p[D_RHO] = fma(m * fma(rr, K.ih3, 1.0), w * w * w, p[D_RHO]);
                     }
                 }
-                if (r2 < K.h2) {
-                    const double w = fma(-rr, K.ih, 1.0);
-                    d.rho = fma(m * fma(rr, K.ih3, 1.0), w * w * w, d.rho);
-                }
             }
-        }
-    }
+        }, [&] { fold_groups<S>(t5, p); });
+    };
+    ListRounds<U64, false, true, LF, S> rounds(A, s, c.x, L, own.g0, 8 * sub);
+    walk(rounds, c.x, false_t{});
     // long entries: row lcap-1-k holds the k-th, so all lanes of a wave
     // read the same row at step k (coalesced), whatever their counts
-    ListRounds<U64, true, true, LF> lrounds(A, s, c.y, L);
-    for (int k0 = 0; k0 < c.y; k0 += U64) {
-        int t[U64];
-        double2 rj[U64], vv[U64];
-        double mj[U64];
-        lrounds.take(k0, t);
-#pragma unroll
-        for (int u = 0; u < U64; ++u) {
-            rj[u] = at32(A.r, t[u]);
-            if (!UNIM) mj[u] = at32(A.m, t[u]);
-            if (COH) vv[u] = at32(A.vp, t[u]);
-        }
-        lrounds.next(k0);
-#pragma unroll
-        for (int u = 0; u < U64; ++u) {
-            double dx = rj[u].x - ri.x, dy = rj[u].y - ri.y;
-            if (WRAP) min_image_listed(dx, dy, K);
-            const double r2 = rsq_exact(dx, dy);
-            if (k0 + u < c.y && r2 < K.cutl) {
-                const double m = UNIM ? 1.0 : mj[u];
-                const double rr = sqrt_pair(r2);
-                const double w = fma(-rr, K.ihl, 1.0), w2 = w * w;
-                d.rhol = fma(m * fma(rr, K.ihl3, 1.0), w2 * w, d.rhol);
-                if (COH) {
-                    const double g = m * w2;
-                    d.gx = fma(g, dx, d.gx);
-                    d.gy = fma(g, dy, d.gy);
-                    d.ev = fma(g, (vv[u].x - vi.x) * dx + (vv[u].y - vi.y) * dy, d.ev);
-                }
-            }
-        }
-    }
+    ListRounds<U64, true, true, LF, S> lrounds(A, s, c.y, L, own.g1, 8 * sub);
+    walk(lrounds, c.y, true_t{});
+    if constexpr (!GRP) fold_groups<1>(t5, p);
+    Dens64 d;
     const double mu = UNIM ? K.munif : 1.0, cf = K.fhl * mu;
-    d.rho = fma(K.qh * mu, d.rho, K.qh);
-    d.rhol = fma(K.qhl * mu, d.rhol, K.qhl);
-    d.gx *= cf;
-    d.gy *= cf;
-    d.ev *= cf;
+    d.rho = fma(K.qh * mu, t5[D_RHO], K.qh);
+    d.rhol = fma(K.qhl * mu, t5[D_RHOL], K.qhl);
+    d.gx = t5[D_GX] * cf;
+    d.gy = t5[D_GY] * cf;
+    d.ev = t5[D_EV] * cf;
     return d;
 }
 
@@ -1261,74 +1359,87 @@ __device__ __forceinline__ Dens64 density64_walk(const ArenaView &A, const BoxK 
 //   a_co,i  = -2a sum_j m_j dwdx_hl,ij
 //   du_co,i = -a  sum_j m_j (v_j - v_i) . dwdx_hl,ij      (dv . f / 2)
 // and the rate pass only walks the short entries (r < h + skin).
-template <int U64>
-__global__ __launch_bounds__(PASS_NT_MAX) void k_density64(ArenaView A, int state_mask)
+template <int U64, int S, int SUMS>
+__global__ __launch_bounds__(PASS_NT_MAX, 4) void k_density64(ArenaView A, int state_mask)
 {
-    const int s = xcd_block() * (int)blockDim.x + threadIdx.x;
-    if (s >= A.n) return;
-    const int b = A.slot_box[s];
-    if (b < 0) return;
-    const int st = A.dyn[b].state;
-    if (!state_in(st, state_mask) || A.dyn[b].relist) return;
-    Dens64 d;
-    per_box(b, [&](int bu) {
-        const BoxK K = box_k(A.boxes[bu], true);
-        const ListFmt L = list_fmt(A, bu, s);
-        const bool coh = (K.terms & 2) != 0, unim = K.munif > 0.0, inner = wave_interior(A.r[s], K);
-        with_form(L, [&](auto lf) {
+    int sub;
+    const int s = pass_slot<S>(A, sub), sl = s < A.n ? s : 0;
+    Own64 own;
+    const int bs = slot_owner(A, s);
+    own.c = A.cnt[sl];
+    own.r = A.r[sl];
+    own.v = A.vp[sl];
+    own.g0 = first_cell(A, sl, false, sub);
+    own.g1 = first_cell(A, sl, true, sub);
+    const double mi = A.m[sl];
+    double ui = A.up[sl];
+    per_box(bs, [&](int bu) {
+        CBox &B = cbox(A, bu);
+        CDyn &D = cdyn(A, bu);
+        const BoxK K = box_k(B);
+        const int st = D.state;
+        if (!takes_part(D, state_mask)) return;
+        const ListFmt L = list_fmt(B, D, own.c.x);
+        // shared lists walk with the image test always (the same bits)
+        const bool coh = (K.terms & 2) != 0, unim = K.munif > 0.0, inner = S == 1 && wave_interior(own.r, K);
+        Dens64 d;
+        with_walk<SUMS>(L, [&](auto lf, auto grp) {
             constexpr int F = decltype(lf)::value;
-            if (inner) {
-                if (coh) d = unim ? density64_walk<U64, true, true, false, F>(A, K, L, s) : density64_walk<U64, true, false, false, F>(A, K, L, s);
-                else d = unim ? density64_walk<U64, false, true, false, F>(A, K, L, s) : density64_walk<U64, false, false, false, F>(A, K, L, s);
-            } else {
-                if (coh) d = unim ? density64_walk<U64, true, true, true, F>(A, K, L, s) : density64_walk<U64, true, false, true, F>(A, K, L, s);
-                else d = unim ? density64_walk<U64, false, true, true, F>(A, K, L, s) : density64_walk<U64, false, false, true, F>(A, K, L, s);
+            constexpr bool G = decltype(grp)::value;
+            auto walk = [&](auto wrap_t) {
+                constexpr bool W = decltype(wrap_t)::value;
+                if (coh) d = unim ? density64_walk<U64, S, G, true, true, W, F>(A, K, L, s, sub, own) : density64_walk<U64, S, G, true, false, W, F>(A, K, L, s, sub, own);
+                else d = unim ? density64_walk<U64, S, G, false, true, W, F>(A, K, L, s, sub, own) : density64_walk<U64, S, G, false, false, W, F>(A, K, L, s, sub, own);
+            };
+            if constexpr (S == 1) {
+                if (inner) {
+                    walk(false_t{});
+                    return;
+                }
             }
+            walk(true_t{});
         });
+        if (S > 1 && sub != 0) return;  // one lane stores
+        const double rho = d.rho, rhol = d.rhol;
+        if (st == BOX_INIT) {  // u = kB T0 - a rho (properties.py:44-46,119)
+            ui = B.kB * B.T0 - B.a * rho;
+            A.u[s] = ui;
+            A.up[s] = ui;
+        }
+        double T = (ui + B.a * rho) / B.kB;  // properties.py:48-49
+        T = T < 0.0 ? 0.0 : T;               // spam_complete_force.py:152
+        const double p = vdw_p(rho, T, B);
+        A.rho[s] = make_double2(rho, rhol);
+        A.T[s] = T;
+        // the stress record (m in .w for the rate pass) only when the gradient
+        // pass will not write it; q/rho^2 is read only with conduction, when the
+        // gradient pass writes it
+        if (!(B.terms & 4)) {
+            const double ps = (B.terms & 1) ? p / (rho * rho) : 0.0;
+            A.S[s] = make_double4(ps, 0.0, ps, mi);
+        }
+        A.vt[s] = make_double2(mi / rho, T);
+        A.aco[s] = coh ? make_double2(-2.0 * B.a * d.gx, -2.0 * B.a * d.gy) : make_double2(0.0, 0.0);
+        A.uco[s] = coh ? -B.a * d.ev : 0.0;
+        if (!(rho * B.b < 1.0)) flag_health(A.dyn, bu, HEALTH_EOS_POLE);
+        if (!isfinite(rho) || !isfinite(rhol) || !isfinite(ui)) flag_health(A.dyn, bu, HEALTH_NONFINITE);
     });
-    const BoxDesc &B = A.boxes[b];
-    const bool coh = (B.terms & 2u) != 0;
-    const double rho = d.rho, rhol = d.rhol;
-    const double mi = A.m[s];
-    double ui = A.up[s];
-    if (st == BOX_INIT) {  // u = kB T0 - a rho (properties.py:44-46,119)
-        ui = B.kB * B.T0 - B.a * rho;
-        A.u[s] = ui;
-        A.up[s] = ui;
-    }
-    double T = (ui + B.a * rho) / B.kB;  // properties.py:48-49
-    T = T < 0.0 ? 0.0 : T;               // spam_complete_force.py:152
-    const double p = vdw_p(rho, T, B);
-    A.rho[s] = make_double2(rho, rhol);
-    A.T[s] = T;
-    // the stress record (m in .w for the rate pass) only when the gradient
-    // pass will not write it; q/rho^2 is read only with conduction, when the
-    // gradient pass writes it
-    if (!(B.terms & 4u)) {
-        const double ps = (B.terms & 1u) ? p / (rho * rho) : 0.0;
-        A.S[s] = make_double4(ps, 0.0, ps, mi);
-    }
-    A.vt[s] = make_double2(mi / rho, T);
-    A.aco[s] = coh ? make_double2(-2.0 * B.a * d.gx, -2.0 * B.a * d.gy) : make_double2(0.0, 0.0);
-    A.uco[s] = coh ? -B.a * d.ev : 0.0;
-    if (!(rho * B.b < 1.0)) flag_health(A.dyn, b, HEALTH_EOS_POLE);
-    if (!isfinite(rho) || !isfinite(rhol) || !isfinite(ui)) flag_health(A.dyn, b, HEALTH_NONFINITE);
 }
 
+enum : int { G_00 = 0, G_01, G_10, G_11, G_T0, G_T1, G_N };
 struct Grad64 {
     double g00, g01, g10, g11, gt0, gt1;
 };
 
-template <int U64, bool WRAP, int LF>
-__device__ __forceinline__ Grad64 grad64_walk(const ArenaView &A, const BoxK &K, const ListFmt &L, int s)
+template <int U64, int S, bool GRP, bool WRAP, int LF>
+__device__ __forceinline__ Grad64 grad64_walk(const ArenaView &A, const BoxK &K, const ListFmt &L, int s, int sub, const Own64 &own,
+                                              double Ti)
 {
-    const double2 ri = A.r[s], vi = A.vp[s];
-    const double Ti = A.T[s];
-    const int ns = A.cnt[s].x & CNT_MASK;
-    Grad64 g;
-    g.g00 = g.g01 = g.g10 = g.g11 = g.gt0 = g.gt1 = 0.0;
-    ListRounds<U64, false, false, LF> rounds(A, s, ns, L);
-    for (int k0 = 0; k0 < ns; k0 += U64) {
+    const double2 ri = own.r, vi = own.v;
+    const int ns = own.c.x & CNT_MASK;
+    double d[G_N] = {}, p[G_N] = {};
+    ListRounds<U64, false, false, LF, S> rounds(A, s, ns, L, own.g0, 8 * sub);
+    for_rounds<U64, S, GRP>(ns, sub, [&](int k0) {
         int t[U64];
         double2 rj[U64], vv[U64], vt[U64];
         rounds.take(k0, t);
@@ -1352,79 +1463,91 @@ __device__ __forceinline__ Grad64 grad64_walk(const ArenaView &A, const BoxK &K,
                 const double vj = vt[u].x;
                 const double dvx = vv[u].x - vi.x, dvy = vv[u].y - vi.y;
                 const double dT = vt[u].y - Ti;
-                g.g00 += vj * dvx * gx;
-                g.g01 += vj * dvx * gy;
-                g.g10 += vj * dvy * gx;
-                g.g11 += vj * dvy * gy;
-                g.gt0 += vj * dT * gx;
-                g.gt1 += vj * dT * gy;
+                p[G_00] += vj * dvx * gx;
+                p[G_01] += vj * dvx * gy;
+                p[G_10] += vj * dvy * gx;
+                p[G_11] += vj * dvy * gy;
+                p[G_T0] += vj * dT * gx;
+                p[G_T1] += vj * dT * gy;
             }
         }
-    }
-    return g;
+    }, [&] { fold_groups<S>(d, p); });
+    if constexpr (!GRP) fold_groups<1>(d, p);
+    return Grad64{d[G_00], d[G_01], d[G_10], d[G_11], d[G_T0], d[G_T1]};
 }
 
 // P2: grad v and grad T with grad_i W_ij = -dwdx_ij (dwdx from r_j - r_i);
 // viscous stress Pi = -eta (G + G^T - tr G I) - zeta tr G I (2-D) and heat
 // flux q = -k grad T.  diag != 0 also stores grad v and q for download.
 // Neighbour record: position, velocity, (m/rho, T) from P1.
-template <int U64>
-__global__ __launch_bounds__(PASS_NT_MAX) void k_grad64(ArenaView A, int state_mask, int diag)
+template <int U64, int S, int SUMS>
+__global__ __launch_bounds__(PASS_NT_MAX, 4) void k_grad64(ArenaView A, int state_mask, int diag)
 {
-    const int s = xcd_block() * (int)blockDim.x + threadIdx.x;
-    if (s >= A.n) return;
-    const int b = A.slot_box[s];
-    if (b < 0) return;
-    if (!state_in(A.dyn[b].state, state_mask) || A.dyn[b].relist) return;
-    const BoxDesc &B = A.boxes[b];
-    if (!diag && !(B.terms & 12u)) return;
-    Grad64 g;
-    per_box(b, [&](int bu) {
-        const BoxK K = box_k(A.boxes[bu], true);
-        const ListFmt L = list_fmt(A, bu, s);
-        const bool inner = wave_interior(A.r[s], K);
-        with_form(L, [&](auto lf) {
+    int sub;
+    const int s = pass_slot<S>(A, sub), sl = s < A.n ? s : 0;
+    Own64 own;
+    const int bs = slot_owner(A, s);
+    own.c = A.cnt[sl];
+    own.r = A.r[sl];
+    own.v = A.vp[sl];
+    own.g0 = first_cell(A, sl, false, sub);
+    const double Ti = A.T[sl], rho = A.rho[sl].x, mi = A.m[sl];
+    per_box(bs, [&](int bu) {
+        CBox &B = cbox(A, bu);
+        CDyn &D = cdyn(A, bu);
+        const BoxK K = box_k(B);
+        if (!takes_part(D, state_mask)) return;
+        if (!diag && !(B.terms & 12)) return;
+        const ListFmt L = list_fmt(B, D, own.c.x);
+        const bool inner = S == 1 && wave_interior(own.r, K);
+        Grad64 g;
+        with_walk<SUMS>(L, [&](auto lf, auto grp) {
             constexpr int F = decltype(lf)::value;
-            g = inner ? grad64_walk<U64, false, F>(A, K, L, s) : grad64_walk<U64, true, F>(A, K, L, s);
+            constexpr bool G = decltype(grp)::value;
+            if constexpr (S == 1) {
+                if (inner) {
+                    g = grad64_walk<U64, S, G, false, F>(A, K, L, s, sub, own, Ti);
+                    return;
+                }
+            }
+            g = grad64_walk<U64, S, G, true, F>(A, K, L, s, sub, own, Ti);
         });
+        if (S > 1 && sub != 0) return;  // one lane stores
+        const double r2i = rho * rho;
+        double pxx = 0, pxy = 0, pyy = 0;
+        if (B.terms & 4) {
+            const double tr = g.g00 + g.g11;
+            pxx = -B.eta * (2.0 * g.g00 - tr) - B.zeta * tr;
+            pyy = -B.eta * (2.0 * g.g11 - tr) - B.zeta * tr;
+            pxy = -B.eta * (g.g01 + g.g10);
+            const double pr = (B.terms & 1) ? vdw_p(rho, Ti, B) : 0.0;
+            A.S[s] = make_double4((pr + pxx) / r2i, pxy / r2i, (pr + pyy) / r2i, mi);
+        }
+        double qx = 0, qy = 0;
+        if (B.terms & 8) {
+            qx = -B.kcond * g.gt0;
+            qy = -B.kcond * g.gt1;
+            A.Q[s] = make_double2(qx / r2i, qy / r2i);
+        }
+        if (diag) {
+            A.gradv[s] = make_double4(g.g00, g.g01, g.g10, g.g11);
+            A.jq[s] = make_double2(qx, qy);
+        }
     });
-    const double Ti = A.T[s];
-    const double rho = A.rho[s].x, r2i = rho * rho;
-    double pxx = 0, pxy = 0, pyy = 0;
-    if (B.terms & 4u) {
-        const double tr = g.g00 + g.g11;
-        pxx = -B.eta * (2.0 * g.g00 - tr) - B.zeta * tr;
-        pyy = -B.eta * (2.0 * g.g11 - tr) - B.zeta * tr;
-        pxy = -B.eta * (g.g01 + g.g10);
-        const double pr = (B.terms & 1u) ? vdw_p(rho, Ti, B) : 0.0;
-        A.S[s] = make_double4((pr + pxx) / r2i, pxy / r2i, (pr + pyy) / r2i, A.m[s]);
-    }
-    double qx = 0, qy = 0;
-    if (B.terms & 8u) {
-        qx = -B.kcond * g.gt0;
-        qy = -B.kcond * g.gt1;
-        A.Q[s] = make_double2(qx / r2i, qy / r2i);
-    }
-    if (diag) {
-        A.gradv[s] = make_double4(g.g00, g.g01, g.g10, g.g11);
-        A.jq[s] = make_double2(qx, qy);
-    }
 }
 
 struct Rate64 {
     double ax, ay, ud;
 };
 
-template <int U64, bool COND, bool WRAP, int LF>
-__device__ __forceinline__ Rate64 rates64_walk(const ArenaView &A, const BoxK &K, const ListFmt &L, int s, int ns)
+template <int U64, int S, bool GRP, bool COND, bool WRAP, int LF>
+__device__ __forceinline__ Rate64 rates64_walk(const ArenaView &A, const BoxK &K, const ListFmt &L, int s, int sub,
+                                               int ns, const Own64 &own, const double4 &Si, const double2 &Qi)
 {
-    const double2 ri = A.r[s], vi = A.vp[s];
-    const double4 Si = A.S[s];
-    const double2 Qi = COND ? A.Q[s] : make_double2(0.0, 0.0);
-    Rate64 o;
-    o.ax = o.ay = o.ud = 0.0;
-    ListRounds<U64, false, false, LF> rounds(A, s, ns, L);
-    for (int k0 = 0; k0 < ns; k0 += U64) {
+    const double2 ri = own.r, vi = own.v;
+    double d[3] = {}, p[3] = {};
+    ListRounds<U64, false, false, LF, S> rounds(A, s, ns, L, own.g0, 8 * sub);
+    for_rounds<U64, S, GRP>(ns, sub, [&](int k0) {
         int t[U64];
         double2 rj[U64], vv[U64], Qj[U64];
         double4 Sj[U64];
@@ -1453,13 +1576,14 @@ __device__ __forceinline__ Rate64 rates64_walk(const ArenaView &A, const BoxK &K
                 const double cc = COND ? (Qi.x + Qj[u].x) * wx + (Qi.y + Qj[u].y) * wy : 0.0;
                 const double e = 0.5 * ((vv[u].x - vi.x) * fx + (vv[u].y - vi.y) * fy);
                 const double mj = Sj[u].w;
-                o.ax += mj * fx;
-                o.ay += mj * fy;
-                o.ud += mj * (e + cc);
+                p[0] += mj * fx;
+                p[1] += mj * fy;
+                p[2] += mj * (e + cc);
             }
         }
-    }
-    return o;
+    }, [&] { fold_groups<S>(d, p); });
+    if constexpr (!GRP) fold_groups<1>(d, p);
+    return Rate64{d[0], d[1], d[2]};
 }
 
 // ===========================================================================
@@ -1467,9 +1591,6 @@ __device__ __forceinline__ Rate64 rates64_walk(const ArenaView &A, const BoxK &K
 // point positions), FP32 long-range pair arithmetic with Kahan-compensated
 // sums, FP64 short-range terms, EOS, integration and energy.
 // ===========================================================================
-
-using true_t = std::integral_constant<bool, true>;
-using false_t = std::integral_constant<bool, false>;
 
 struct Kahan {
     float s, c;
@@ -1514,42 +1635,39 @@ struct BoxF {
     // FP64 constants of the short-range terms (short density, gradients,
     // rates), which take FP64 arithmetic on exact separations
     double h2d, cutsd, ihd, ih3d, fhd;
-    float cut2, cutl;
+    float cutl;
     float ihl, qhl, fhl, munif;
     float ihl3;  // 3/h_l: 1 + 3q = fma(r, 3/h_l, 1)
     int terms;
 };
 
-__device__ __forceinline__ BoxF boxf(const BoxDesc &B, bool uniform)
+__device__ __forceinline__ BoxF boxf(const CBox &B)
 {
     BoxF f;
-    f.sclx = B.Lx / FIX32;
-    f.scly = B.Ly / FIX32;
-    f.s48x = B.Lx / FIX48;
-    f.s48y = B.Ly / FIX48;
+    f.sclx = B.sclx;
+    f.scly = B.scly;
+    f.s48x = B.s48x;
+    f.s48y = B.s48y;
     f.h2d = B.h2;
-    f.cutsd = B.R2list < B.h2 ? B.R2list : B.h2;
+    f.cutsd = B.cutsd;
     f.ihd = B.ih;
-    f.ih3d = 3.0 * B.ih;
+    f.ih3d = B.ih3;
     f.fhd = B.fh;
-    f.munif = (float)B.munif;
-    f.cut2 = (float)B.cut2;
-    f.cutl = (float)(B.cut2 < B.hl2 ? B.cut2 : B.hl2);
-    f.ihl = (float)B.ihl; f.qhl = (float)B.qhl; f.fhl = (float)B.fhl;
-    f.ihl3 = (float)(3.0 * B.ihl);
+    f.munif = wave_uniform((float)B.munif);
+    f.cutl = B.cutlf;
+    f.ihl = B.ihlf; f.qhl = B.qhlf; f.fhl = B.fhlf;
+    f.ihl3 = B.ihl3f;
     f.terms = B.terms;
-    if (uniform) {
-        f.sclx = wave_uniform(f.sclx); f.scly = wave_uniform(f.scly);
-        f.s48x = wave_uniform(f.s48x); f.s48y = wave_uniform(f.s48y);
-        f.h2d = wave_uniform(f.h2d); f.cutsd = wave_uniform(f.cutsd); f.ihd = wave_uniform(f.ihd);
-        f.ih3d = wave_uniform(f.ih3d); f.fhd = wave_uniform(f.fhd);
-        f.cut2 = wave_uniform(f.cut2); f.cutl = wave_uniform(f.cutl);
-        f.ihl = wave_uniform(f.ihl); f.qhl = wave_uniform(f.qhl); f.fhl = wave_uniform(f.fhl);
-        f.ihl3 = wave_uniform(f.ihl3); f.munif = wave_uniform(f.munif);
-        f.terms = wave_uniform(f.terms);
-    }
     return f;
 }
+
+// What an FP32C pass reads of its own slot (as Own64).
+struct Own32 {
+    float4 r;
+    unsigned lo;
+    int2 c;
+    uint4 g0, g1;
+};
 
 // Minimum-image separation of record j from record i (fix_rec): the signed
 // 32-bit difference of the high words (wrapping at the box side), with LO
@@ -1592,174 +1710,211 @@ struct Dens32 {
 // long entry rf alone (16), or rf and rlo in boxes wider than the side
 // up to which the high words keep the long-range terms within FP32 rounding
 // (LOLONG).  UNIM: all masses equal, none fetched.
-template <int U32, bool COH, bool UNIM, bool LOLONG, int LF>
-__device__ __forceinline__ void density32_walk(const ArenaView &A, const BoxF &F, const ListFmt &L, int s, Dens32 &d)
+//
+// A round's partial sums depend on its entries alone, so the S lanes that
+// share a list compute their groups' rounds apart; then each of the four
+// sums is taken by one of the lanes (4 / S sums a lane), which adds every
+// round's part of it in round order: the bits of the walk by one lane.
+template <int U32, int S, bool GRP, bool COH, bool UNIM, bool LOLONG, int LF>
+__device__ __forceinline__ void density32_walk(const ArenaView &A, const BoxF &F, const ListFmt &L, int s, int sub,
+                                               const Own32 &own, Dens32 &d)
 {
+    static_assert(S == 1 || U32 == 4, "shared lists take rounds of four entries");
     // the kernel constants (and, with UNIM, the mass) scale each round's
     // partial sums instead of every term
     const float cqhl = UNIM ? F.qhl * F.munif : F.qhl;
     const float cfhl = UNIM ? F.fhl * F.munif : F.fhl;
-    const float4 ri = A.rf[s];
-    const unsigned loi = A.rlo[s];
-    const int2 cr = A.cnt[s];
-    const int2 c = make_int2(cr.x & CNT_MASK, cr.y);
-    ListRounds<U32, false, true, LF> rounds(A, s, c.x, L);
-    for (int k0 = 0; k0 < c.x; k0 += U32) {
-        int t[U32];
-        float4 rj[U32];
-        unsigned lj[U32];
-        float mm[U32];
-        rounds.take(k0, t);
-#pragma unroll
-        for (int u = 0; u < U32; ++u) {
-            rj[u] = at32(A.rf, t[u]);
-            lj[u] = at32(A.rlo, t[u]);
-            if (!UNIM) mm[u] = (float)at32(A.m, t[u]);
+    const float4 ri = own.r;
+    const unsigned loi = own.lo;
+    const int2 c = make_int2(own.c.x & CNT_MASK, own.c.y);
+    double rho[1] = {}, prho[1] = {};
+    // shared lists: this lane's sums, of rhol, gx, gy, ev the (4 / S) sub on
+    constexpr int NK = S > 1 ? 4 / S : 1;
+    Kahan kk[NK];
+    if (S > 1 && sub == 0) kk[0] = d.rhol;
+    const float sc0 = S > 1 && sub == 0 ? cqhl : cfhl;
+    auto add = [&](float rhol, float gx, float gy, float ev) {
+        d.rhol.add(cqhl * rhol);
+        if (COH) {
+            d.gx.add(cfhl * gx);
+            d.gy.add(cfhl * gy);
+            d.ev.add(cfhl * ev);
         }
-        rounds.next(k0);
-        float grhol = 0.f, ggx = 0.f, ggy = 0.f, gev = 0.f;
+    };
+    auto walk = [&](auto &rounds, int n, auto long_t) {
+        constexpr bool LONG = decltype(long_t)::value;
+        float qa[4] = {}, qb[4] = {};  // the group's two rounds
+        int base = 0;  // first entry of the lanes' current groups
+        for_rounds<U32, S, GRP>(n, sub, [&](int k0) {
+            int t[U32];
+            float4 rj[U32];
+            unsigned lj[U32];
+            float mm[U32];
+            rounds.take(k0, t);
 #pragma unroll
-        for (int u = 0; u < U32; ++u) {
-            double dxd, dyd;
-            sep_fix<true>(ri, loi, rj[u], lj[u], F, dxd, dyd);
-            const float dx = (float)dxd, dy = (float)dyd;
-            const float r2 = dx * dx + dy * dy;
-            const float mj = UNIM ? 1.f : mm[u];
-            if (k0 + u < c.x && r2 < F.cutl) {
-                const float rr = __builtin_amdgcn_sqrtf(r2);
-                const float w = fmaf(-rr, F.ihl, 1.f), w2 = w * w;
-                grhol = fmaf(mj * fmaf(rr, F.ihl3, 1.f), w2 * w, grhol);
-                if (COH) {
-                    const float g = mj * w2;
-                    ggx = fmaf(g, dx, ggx);
-                    ggy = fmaf(g, dy, ggy);
-                    gev = fmaf(g, (rj[u].z - ri.z) * dx + (rj[u].w - ri.w) * dy, gev);
+            for (int u = 0; u < U32; ++u) {
+                rj[u] = at32(A.rf, t[u]);
+                if (!LONG || LOLONG) lj[u] = at32(A.rlo, t[u]);
+                if (!UNIM) mm[u] = (float)at32(A.m, t[u]);
+            }
+            rounds.next(k0);
+            float grhol = 0.f, ggx = 0.f, ggy = 0.f, gev = 0.f;
+#pragma unroll
+            for (int u = 0; u < U32; ++u) {
+                double dxd, dyd;
+                sep_fix<!LONG || LOLONG>(ri, loi, rj[u], !LONG || LOLONG ? lj[u] : 0u, F, dxd, dyd);
+                const float dx = (float)dxd, dy = (float)dyd;
+                const float r2 = dx * dx + dy * dy;
+                const float mj = UNIM ? 1.f : mm[u];
+                if (k0 + u < n && r2 < F.cutl) {
+                    const float rr = __builtin_amdgcn_sqrtf(r2);
+                    const float w = fmaf(-rr, F.ihl, 1.f), w2 = w * w;
+                    grhol = fmaf(mj * fmaf(rr, F.ihl3, 1.f), w2 * w, grhol);
+                    if (COH) {
+                        const float g = mj * w2;
+                        ggx = fmaf(g, dx, ggx);
+                        ggy = fmaf(g, dy, ggy);
+                        gev = fmaf(g, (rj[u].z - ri.z) * dx + (rj[u].w - ri.w) * dy, gev);
+                    }
+                }
+                if constexpr (!LONG) {
+                    const double r2d = rsq_exact(dxd, dyd);
+                    if (k0 + u < n && r2d < F.h2d) {
+                        const double rr = sqrt_pair(r2d), w = fma(-rr, F.ihd, 1.0);
+                        prho[0] = fma((double)mj * fma(rr, F.ih3d, 1.0), w * w * w, prho[0]);
+                    }
                 }
             }
-            const double r2d = rsq_exact(dxd, dyd);
-            if (k0 + u < c.x && r2d < F.h2d) {
-                const double rr = sqrt_pair(r2d), w = fma(-rr, F.ihd, 1.0);
-                d.rho = fma((double)mj * fma(rr, F.ih3d, 1.0), w * w * w, d.rho);
+            if constexpr (S == 1) {
+                add(grhol, ggx, ggy, gev);
+            } else {
+                const bool second = (k0 & 4) != 0;
+                const float x[4] = {grhol, ggx, ggy, gev};
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    qa[i] = second ? qa[i] : x[i];
+                    qb[i] = second ? x[i] : qb[i];
+                }
             }
-        }
-        d.rhol.add(cqhl * grhol);
-        if (COH) {
-            d.gx.add(cfhl * ggx);
-            d.gy.add(cfhl * ggy);
-            d.ev.add(cfhl * gev);
-        }
-    }
+        }, [&] {
+            if constexpr (!LONG) fold_groups<S>(rho, prho);
+            if constexpr (S > 1) {
+#pragma unroll
+                for (int l = 0; l < S; ++l)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        float x[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) x[i] = lane_bcast<S>(h ? qb[i] : qa[i], l);
+                        const bool on = base + 8 * l + 4 * h < n;
+#pragma unroll
+                        for (int i = 0; i < NK; ++i) {
+                            float v = x[i];
+#pragma unroll
+                            for (int o = 1; o < S; ++o) v = sub == o ? x[o * NK + i] : v;
+                            Kahan nk = kk[i];
+                            nk.add((i == 0 ? sc0 : cfhl) * v);
+                            kk[i].s = on ? nk.s : kk[i].s;
+                            kk[i].c = on ? nk.c : kk[i].c;
+                        }
+                    }
+                base += 8 * S;
+            }
+        });
+    };
+    ListRounds<U32, false, true, LF, S> rounds(A, s, c.x, L, own.g0, 8 * sub);
+    walk(rounds, c.x, false_t{});
     // long entries: row lcap-1-k holds the k-th, so all lanes of a wave
     // read the same row at step k (coalesced), whatever their counts
-    ListRounds<U32, true, true, LF> lrounds(A, s, c.y, L);
-    for (int k0 = 0; k0 < c.y; k0 += U32) {
-        int t[U32];
-        float4 rj[U32];
-        unsigned lj[U32];
-        float mm[U32];
-        lrounds.take(k0, t);
-#pragma unroll
-        for (int u = 0; u < U32; ++u) {
-            rj[u] = at32(A.rf, t[u]);
-            if (LOLONG) lj[u] = at32(A.rlo, t[u]);
-            if (!UNIM) mm[u] = (float)at32(A.m, t[u]);
-        }
-        lrounds.next(k0);
-        float grhol = 0.f, ggx = 0.f, ggy = 0.f, gev = 0.f;
-#pragma unroll
-        for (int u = 0; u < U32; ++u) {
-            double dxd, dyd;
-            sep_fix<LOLONG>(ri, loi, rj[u], LOLONG ? lj[u] : 0u, F, dxd, dyd);
-            const float dx = (float)dxd, dy = (float)dyd;
-            const float r2 = dx * dx + dy * dy;
-            const float mj = UNIM ? 1.f : mm[u];
-            if (k0 + u < c.y && r2 < F.cutl) {
-                const float rr = __builtin_amdgcn_sqrtf(r2);
-                const float w = fmaf(-rr, F.ihl, 1.f), w2 = w * w;
-                grhol = fmaf(mj * fmaf(rr, F.ihl3, 1.f), w2 * w, grhol);
-                if (COH) {
-                    const float g = mj * w2;
-                    ggx = fmaf(g, dx, ggx);
-                    ggy = fmaf(g, dy, ggy);
-                    gev = fmaf(g, (rj[u].z - ri.z) * dx + (rj[u].w - ri.w) * dy, gev);
-                }
-            }
-        }
-        d.rhol.add(cqhl * grhol);
+    ListRounds<U32, true, true, LF, S> lrounds(A, s, c.y, L, own.g1, 8 * sub);
+    walk(lrounds, c.y, true_t{});
+    if constexpr (!GRP) fold_groups<1>(rho, prho);
+    d.rho = rho[0];
+    if constexpr (S > 1) {
+        auto take = [&](Kahan &k, int q) {
+            k.s = lane_bcast<S>(kk[q % NK].s, q / NK);
+            k.c = lane_bcast<S>(kk[q % NK].c, q / NK);
+        };
+        take(d.rhol, 0);
         if (COH) {
-            d.gx.add(cfhl * ggx);
-            d.gy.add(cfhl * ggy);
-            d.ev.add(cfhl * gev);
+            take(d.gx, 1);
+            take(d.gy, 2);
+            take(d.ev, 3);
         }
     }
 }
 
 // P1 of the FP32C form: rf carries position and predicted velocity; the
 // cohesive rate part (see k_density64) is accumulated with the densities.
-template <int U32>
-__global__ __launch_bounds__(PASS_NT_MAX) void k_density32(ArenaView A, int state_mask)
+template <int U32, int S, int SUMS>
+__global__ __launch_bounds__(PASS_NT_MAX, 4) void k_density32(ArenaView A, int state_mask)
 {
-    const int s = xcd_block() * (int)blockDim.x + threadIdx.x;
-    if (s >= A.n) return;
-    const int b = A.slot_box[s];
-    if (b < 0) return;
-    const int st = A.dyn[b].state;
-    if (!state_in(st, state_mask) || A.dyn[b].relist) return;
-    const BoxDesc &B = A.boxes[b];
-    const bool coh = (B.terms & 2u) != 0;
-    Dens32 d;
-    per_box(b, [&](int bu) {
-        const BoxDesc &Bu = A.boxes[bu];
-        const BoxF F = boxf(Bu, true);
-        const ListFmt L = list_fmt(A, bu, s);
-        const bool lolong = wave_uniform(Bu.lolong) != 0;
+    int sub;
+    const int s = pass_slot<S>(A, sub), sl = s < A.n ? s : 0;
+    Own32 own;
+    const int bs = slot_owner(A, s);
+    own.c = A.cnt[sl];
+    own.r = A.rf[sl];
+    own.lo = A.rlo[sl];
+    own.g0 = first_cell(A, sl, false, sub);
+    own.g1 = first_cell(A, sl, true, sub);
+    const double mi = A.m[sl];
+    double ui = A.up[sl];
+    per_box(bs, [&](int bu) {
+        CBox &B = cbox(A, bu);
+        CDyn &D = cdyn(A, bu);
+        const BoxF F = boxf(B);
+        const int st = D.state;
+        if (!takes_part(D, state_mask)) return;
+        const ListFmt L = list_fmt(B, D, own.c.x);
+        const bool lolong = B.lolong != 0, coh = (B.terms & 2) != 0;
+        Dens32 d;
         d.rho = 0.0;
         d.rhol = Kahan(F.qhl);
         auto walk = [&](auto coh_t, auto unim_t) {
             constexpr bool C = decltype(coh_t)::value, M = decltype(unim_t)::value;
-            with_form(L, [&](auto lf) {
+            with_walk<SUMS>(L, [&](auto lf, auto grp) {
                 constexpr int LF = decltype(lf)::value;
-                if (lolong) density32_walk<U32, C, M, true, LF>(A, F, L, s, d);
-                else density32_walk<U32, C, M, false, LF>(A, F, L, s, d);
+                constexpr bool G = decltype(grp)::value;
+                if (lolong) density32_walk<U32, S, G, C, M, true, LF>(A, F, L, s, sub, own, d);
+                else density32_walk<U32, S, G, C, M, false, LF>(A, F, L, s, sub, own, d);
             });
         };
         const bool unim = F.munif > 0.f;
-        if (F.terms & 2) {
+        if (coh) {
             if (unim) walk(true_t{}, true_t{});
             else walk(true_t{}, false_t{});
         } else {
             if (unim) walk(false_t{}, true_t{});
             else walk(false_t{}, false_t{});
         }
+        if (S > 1 && sub != 0) return;  // one lane stores
+        // the short-range sum leaves out q_h (and the common mass)
+        const double rd = fma(B.qh * (B.munif > 0.0 ? B.munif : 1.0), d.rho, B.qh), rl = d.rhol.value();
+        if (st == BOX_INIT) {
+            ui = B.kB * B.T0 - B.a * rd;
+            A.u[s] = ui;
+            A.up[s] = ui;
+        }
+        double T = (ui + B.a * rd) / B.kB;
+        T = T < 0.0 ? 0.0 : T;
+        const double p = vdw_p(rd, T, B);
+        A.rho[s] = make_double2(rd, rl);
+        A.T[s] = T;
+        // records the gradient pass rewrites are written here only when it will
+        // not run (stress without viscosity; q/rho^2 without viscosity and
+        // conduction)
+        if (!(B.terms & 4)) {
+            const double ps = (B.terms & 1) ? p / (rd * rd) : 0.0;
+            A.S32[s] = make_float4((float)ps, 0.f, (float)ps, (float)mi);
+        }
+        if (!(B.terms & 12)) A.q32[s] = QRec32{own.lo, 0.f, 0.f, 0.f};
+        A.g32[s] = GRec32{own.lo, (float)(mi / rd), T};
+        A.aco[s] = coh ? make_double2(-2.0 * B.a * d.gx.value(), -2.0 * B.a * d.gy.value()) : make_double2(0.0, 0.0);
+        A.uco[s] = coh ? -B.a * d.ev.value() : 0.0;
+        if (!(rd * B.b < 1.0)) flag_health(A.dyn, bu, HEALTH_EOS_POLE);
+        if (!isfinite(rd) || !isfinite(rl) || !isfinite(ui)) flag_health(A.dyn, bu, HEALTH_NONFINITE);
     });
-    // the short-range sum leaves out q_h (and the common mass)
-    const double rd = fma(B.qh * (B.munif > 0.0 ? B.munif : 1.0), d.rho, B.qh), rl = d.rhol.value();
-    const double mi = A.m[s];
-    double ui = A.up[s];
-    if (st == BOX_INIT) {
-        ui = B.kB * B.T0 - B.a * rd;
-        A.u[s] = ui;
-        A.up[s] = ui;
-    }
-    double T = (ui + B.a * rd) / B.kB;
-    T = T < 0.0 ? 0.0 : T;
-    const double p = vdw_p(rd, T, B);
-    A.rho[s] = make_double2(rd, rl);
-    A.T[s] = T;
-    // records the gradient pass rewrites are written here only when it will
-    // not run (stress without viscosity; q/rho^2 without viscosity and
-    // conduction)
-    if (!(B.terms & 4u)) {
-        const double ps = (B.terms & 1u) ? p / (rd * rd) : 0.0;
-        A.S32[s] = make_float4((float)ps, 0.f, (float)ps, (float)mi);
-    }
-    const unsigned lo = A.rlo[s];
-    if (!(B.terms & 12u)) A.q32[s] = QRec32{lo, 0.f, 0.f, 0.f};
-    A.g32[s] = GRec32{lo, (float)(mi / rd), T};
-    A.aco[s] = coh ? make_double2(-2.0 * B.a * d.gx.value(), -2.0 * B.a * d.gy.value()) : make_double2(0.0, 0.0);
-    A.uco[s] = coh ? -B.a * d.ev.value() : 0.0;
-    if (!(rd * B.b < 1.0)) flag_health(A.dyn, b, HEALTH_EOS_POLE);
-    if (!isfinite(rd) || !isfinite(rl) || !isfinite(ui)) flag_health(A.dyn, b, HEALTH_NONFINITE);
 }
 
 struct Grad32 {
@@ -1777,16 +1932,17 @@ struct Grad32 {
 // m/rho with a float T, the FP64 T) the pass was no faster than the FP64
 // form's, every gather costing the same texture-path time whatever its
 // width.
-template <int U32, int LF>
-__device__ __forceinline__ void grad32_walk(const ArenaView &A, const BoxF &F, const ListFmt &L, int s, Grad32 &g)
+template <int U32, int S, bool GRP, int LF>
+__device__ __forceinline__ void grad32_walk(const ArenaView &A, const BoxF &F, const ListFmt &L, int s, int sub,
+                                            const Own32 &own, double Ti, Grad32 &g)
 {
-    const float4 ri = A.rf[s];
-    const unsigned loi = A.rlo[s];
+    const float4 ri = own.r;
+    const unsigned loi = own.lo;
     const double vix = ri.z, viy = ri.w;
-    const double Ti = A.T[s];
-    const int ns = A.cnt[s].x & CNT_MASK;
-    ListRounds<U32, false, false, LF> rounds(A, s, ns, L);
-    for (int k0 = 0; k0 < ns; k0 += U32) {
+    const int ns = own.c.x & CNT_MASK;
+    double d[G_N] = {}, p[G_N] = {};
+    ListRounds<U32, false, false, LF, S> rounds(A, s, ns, L, own.g0, 8 * sub);
+    for_rounds<U32, S, GRP>(ns, sub, [&](int k0) {
         int t[U32];
         float4 rj[U32];
         GRec32 gj[U32];
@@ -1809,56 +1965,64 @@ __device__ __forceinline__ void grad32_walk(const ArenaView &A, const BoxF &F, c
                 const double vj = gj[u].v;
                 const double dvx = (double)rj[u].z - vix, dvy = (double)rj[u].w - viy;
                 const double dT = gj[u].T - Ti;
-                g.g00 += vj * dvx * gx;
-                g.g01 += vj * dvx * gy;
-                g.g10 += vj * dvy * gx;
-                g.g11 += vj * dvy * gy;
-                g.gt0 += vj * dT * gx;
-                g.gt1 += vj * dT * gy;
+                p[G_00] += vj * dvx * gx;
+                p[G_01] += vj * dvx * gy;
+                p[G_10] += vj * dvy * gx;
+                p[G_11] += vj * dvy * gy;
+                p[G_T0] += vj * dT * gx;
+                p[G_T1] += vj * dT * gy;
             }
         }
-    }
+    }, [&] { fold_groups<S>(d, p); });
+    if constexpr (!GRP) fold_groups<1>(d, p);
+    g = Grad32{d[G_00], d[G_01], d[G_10], d[G_11], d[G_T0], d[G_T1]};
 }
 
 // P2 of the FP32C form.  Writes the stress record (S32, with viscosity) and
 // the rate pass's q/rho^2 record.
-template <int U32>
-__global__ __launch_bounds__(PASS_NT_MAX) void k_grad32(ArenaView A, int state_mask, int diag)
+template <int U32, int S, int SUMS>
+__global__ __launch_bounds__(PASS_NT_MAX, 4) void k_grad32(ArenaView A, int state_mask, int diag)
 {
-    const int s = xcd_block() * (int)blockDim.x + threadIdx.x;
-    if (s >= A.n) return;
-    const int b = A.slot_box[s];
-    if (b < 0) return;
-    if (!state_in(A.dyn[b].state, state_mask) || A.dyn[b].relist) return;
-    const BoxDesc &B = A.boxes[b];
-    if (!diag && !(B.terms & 12u)) return;
-    Grad32 g = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    per_box(b, [&](int bu) {
-        const BoxF F = boxf(A.boxes[bu], true);
-        const ListFmt L = list_fmt(A, bu, s);
-        with_form(L, [&](auto lf) { grad32_walk<U32, decltype(lf)::value>(A, F, L, s, g); });
+    int sub;
+    const int s = pass_slot<S>(A, sub), sl = s < A.n ? s : 0;
+    Own32 own;
+    const int bs = slot_owner(A, s);
+    own.c = A.cnt[sl];
+    own.r = A.rf[sl];
+    own.lo = A.rlo[sl];
+    own.g0 = first_cell(A, sl, false, sub);
+    const double Ti = A.T[sl], rho = A.rho[sl].x, mi = A.m[sl];
+    per_box(bs, [&](int bu) {
+        CBox &B = cbox(A, bu);
+        CDyn &D = cdyn(A, bu);
+        const BoxF F = boxf(B);
+        if (!takes_part(D, state_mask)) return;
+        if (!diag && !(B.terms & 12)) return;
+        const ListFmt L = list_fmt(B, D, own.c.x);
+        Grad32 g = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+        with_walk<SUMS>(L, [&](auto lf, auto grp) { grad32_walk<U32, S, decltype(grp)::value, decltype(lf)::value>(A, F, L, s, sub, own, Ti, g); });
+        if (S > 1 && sub != 0) return;  // one lane stores
+        const double G00 = g.g00, G01 = g.g01, G10 = g.g10, G11 = g.g11;
+        const double r2i = rho * rho;
+        double qx = 0, qy = 0;
+        if (B.terms & 4) {
+            const double tr = G00 + G11;
+            const double pxx = -B.eta * (2.0 * G00 - tr) - B.zeta * tr;
+            const double pyy = -B.eta * (2.0 * G11 - tr) - B.zeta * tr;
+            const double pxy = -B.eta * (G01 + G10);
+            const double pr = (B.terms & 1) ? vdw_p(rho, Ti, B) : 0.0;
+            A.S32[s] = make_float4((float)((pr + pxx) / r2i), (float)(pxy / r2i), (float)((pr + pyy) / r2i), (float)mi);
+        }
+        if (B.terms & 8) {
+            qx = -B.kcond * g.gt0;
+            qy = -B.kcond * g.gt1;
+        }
+        A.q32[s] = QRec32{own.lo, (float)(qx / r2i), (float)(qy / r2i), 0.f};
+        if (diag) {
+            A.gradv[s] = make_double4(G00, G01, G10, G11);
+            A.jq[s] = make_double2(qx, qy);
+        }
     });
-    const double G00 = g.g00, G01 = g.g01, G10 = g.g10, G11 = g.g11;
-    const double rho = A.rho[s].x, r2i = rho * rho;
-    double qx = 0, qy = 0;
-    if (B.terms & 4u) {
-        const double tr = G00 + G11;
-        const double pxx = -B.eta * (2.0 * G00 - tr) - B.zeta * tr;
-        const double pyy = -B.eta * (2.0 * G11 - tr) - B.zeta * tr;
-        const double pxy = -B.eta * (G01 + G10);
-        const double pr = (B.terms & 1u) ? vdw_p(rho, A.T[s], B) : 0.0;
-        A.S32[s] = make_float4((float)((pr + pxx) / r2i), (float)(pxy / r2i), (float)((pr + pyy) / r2i),
-                               (float)A.m[s]);
-    }
-    if (B.terms & 8u) {
-        qx = -B.kcond * g.gt0;
-        qy = -B.kcond * g.gt1;
-    }
-    A.q32[s] = QRec32{A.rlo[s], (float)(qx / r2i), (float)(qy / r2i), 0.f};
-    if (diag) {
-        A.gradv[s] = make_double4(G00, G01, G10, G11);
-        A.jq[s] = make_double2(qx, qy);
-    }
 }
 
 struct Rate32 {
@@ -1868,20 +2032,15 @@ struct Rate32 {
 // P3 walk of the FP32C form: FP32 neighbour records, FP64 arithmetic on the
 // exact separations (see grad32_walk).  Per neighbour: rf, (S, m) and rlo,
 // the latter, with conduction, in one record with q/rho^2.
-template <int U32, bool COND, int LF>
-__device__ __forceinline__ void rates32_walk(const ArenaView &A, const BoxF &F, const ListFmt &L, int s, int ns,
-                                             Rate32 &o)
+template <int U32, int S, bool GRP, bool COND, int LF>
+__device__ __forceinline__ void rates32_walk(const ArenaView &A, const BoxF &F, const ListFmt &L, int s, int sub,
+                                             int ns, const Own32 &own, const float4 &Si, const float2 &qi, Rate32 &o)
 {
-    const float4 ri = A.rf[s];
-    const unsigned loi = A.rlo[s];
-    float2 qi = make_float2(0.f, 0.f);
-    if (COND) {
-        const QRec32 q = A.q32[s];
-        qi = make_float2(q.qx, q.qy);
-    }
-    const float4 Si = A.S32[s];
-    ListRounds<U32, false, false, LF> rounds(A, s, ns, L);
-    for (int k0 = 0; k0 < ns; k0 += U32) {
+    const float4 ri = own.r;
+    const unsigned loi = own.lo;
+    double d[3] = {}, p[3] = {};
+    ListRounds<U32, false, false, LF, S> rounds(A, s, ns, L, own.g0, 8 * sub);
+    for_rounds<U32, S, GRP>(ns, sub, [&](int k0) {
         int t[U32];
         float4 rj[U32], Sj[U32];
         unsigned lj[U32];
@@ -1918,12 +2077,14 @@ __device__ __forceinline__ void rates32_walk(const ArenaView &A, const BoxF &F, 
                                        : 0.0;
                 const double mj = Sj[u].w;
                 const double e = 0.5 * (((double)rj[u].z - (double)ri.z) * fx + ((double)rj[u].w - (double)ri.w) * fy);
-                o.ax += mj * fx;
-                o.ay += mj * fy;
-                o.ud += mj * (e + cc);
+                p[0] += mj * fx;
+                p[1] += mj * fy;
+                p[2] += mj * (e + cc);
             }
         }
-    }
+    }, [&] { fold_groups<S>(d, p); });
+    if constexpr (!GRP) fold_groups<1>(d, p);
+    o = Rate32{d[0], d[1], d[2]};
 }
 
 // ===========================================================================
@@ -1948,11 +2109,9 @@ __device__ __forceinline__ void rates32_walk(const ArenaView &A, const BoxF &F, 
 // (a, ud); returns the squared displacement since the box's last build (-1
 // at the closing half kick, which moves nothing).  On the box's first and
 // last step, cap is set and e holds the slot's energy.
-__device__ __forceinline__ double integrate_slot(const ArenaView &A, int fp32, int s, int b, double2 a, double ud,
-                                                 double &e, bool &cap)
+__device__ __forceinline__ double integrate_slot(const ArenaView &A, int fp32, int s, int b, const CBox &B, const CDyn &D,
+                                                 double2 a, double ud, double &e, bool &cap)
 {
-    const BoxDyn &D = A.dyn[b];
-    const BoxDesc &B = A.boxes[b];
     const int64_t k = D.k, K = D.nsteps;
     const double kick = (k == 0 || k == K) ? 0.5 * B.dt : B.dt;
     const double2 v = A.v[s];
@@ -2013,7 +2172,8 @@ __device__ __forceinline__ void carry_slot(const ArenaView &A, int fp32, int s)
 // (k_box_step, extend_steps); on that step the step pass gathers the largest
 // squared displacement of the box's slots: per wave in wdisp for the waves
 // wholly inside the box, in its dyn.dmax2 for the waves it shares.
-__device__ __forceinline__ bool list_review(const BoxDyn &D)
+template <class Dyn>
+__device__ __forceinline__ bool list_review(const Dyn &D)
 {
     // not at the closing half kick (k = nsteps), which moves nothing; the
     // step before it reviews as any other, so the schedule of a run does
@@ -2022,7 +2182,7 @@ __device__ __forceinline__ bool list_review(const BoxDyn &D)
 }
 
 // The step pass's tail for slot s of box b (-1: no box): the leapfrog step
-// (on: the box runs and took its rates in this launch) or the carry-over,
+// (a running box, with the rates a, ud of this launch) or the carry-over,
 // then, on a box's review step, the largest squared displacement of its
 // lanes.  A wave holds 64 consecutive slots and a box a contiguous slot
 // range, so a wave whose first and last lanes share a box lies wholly inside
@@ -2033,18 +2193,19 @@ __device__ __forceinline__ bool list_review(const BoxDyn &D)
 // (One atomic per wave into a box field made every review step of a large
 // box slow, the waves queueing on one address.)  Every lane of the wave
 // calls this (no early return before the shuffles).
-__device__ __forceinline__ void step_tail(const ArenaView &A, int fp32, int s, int b, bool on, double2 a, double ud)
+__device__ __forceinline__ void step_tail(const ArenaView &A, int fp32, int s, int b, double2 a, double ud)
 {
     double d2 = 0.0, e = 0.0;
     bool review = false, cap = false;
-    if (s < A.n && b >= 0) {
-        if (on) {
-            d2 = fmax(integrate_slot(A, fp32, s, b, a, ud, e, cap), 0.0);
-            review = list_review(A.dyn[b]);
+    per_box(b, [&](int bu) {
+        CDyn &D = cdyn(A, bu);
+        if (takes_part(D, 1 << BOX_RUN)) {
+            d2 = fmax(integrate_slot(A, fp32, s, bu, cbox(A, bu), D, a, ud, e, cap), 0.0);
+            review = list_review(D);
         } else {
             carry_slot(A, fp32, s);
         }
-    }
+    });
     const int lane = (int)(threadIdx.x & 63);
     const int bfirst = __shfl(b, 0);
     const bool whole = bfirst >= 0 && bfirst == __shfl(b, 63);  // wholly inside one box
@@ -2082,79 +2243,120 @@ __device__ __forceinline__ void step_tail(const ArenaView &A, int fp32, int s, i
 // Neighbour record: position, velocity, (Sxx, Sxy, Syy, m), Q.  step: the
 // stepping launch, which then takes the leapfrog step (step_tail); the
 // stand-alone evaluations only store the rates.
-template <int U64>
-__global__ __launch_bounds__(PASS_NT_MAX) void k_rates64(ArenaView A, int state_mask, int step)
+//
+// With shared lists (S > 1) a block's threads / S slots hand their rates to
+// its first waves through LDS, which store them and take the step tail: one
+// lane per slot over whole 64-slot waves, as with S = 1 (blocks of at least
+// 64 S threads).
+template <int S>
+__device__ __forceinline__ void rates_tail(const ArenaView &A, int fp32, int state_mask, int step, int s, int sub,
+                                           int b, double2 a, double ud)
 {
-    const int s = xcd_block() * (int)blockDim.x + threadIdx.x;
-    int b = -1;
-    bool on = false;
-    if (s < A.n) {
-        b = A.slot_box[s];
-        on = b >= 0 && state_in(A.dyn[b].state, state_mask) && !A.dyn[b].relist;
+    if constexpr (S > 1) {
+        constexpr int n = NT / S;
+        __shared__ double xch[3][n];
+        const int i = (int)threadIdx.x / S, j = (int)threadIdx.x;
+        if (sub == 0) {
+            xch[0][i] = a.x;
+            xch[1][i] = a.y;
+            xch[2][i] = ud;
+        }
+        __syncthreads();
+        if (j >= n) return;
+        s = xcd_block() * n + j;
+        b = slot_owner(A, s);
+        a = make_double2(xch[0][j], xch[1][j]);
+        ud = xch[2][j];
     }
-    double2 a = make_double2(0.0, 0.0);
-    double ud = 0.0;
-    if (on) {
-        const BoxDesc &B = A.boxes[b];
-        const int ns = (B.terms & 13u) ? (A.cnt[s].x & CNT_MASK) : 0;
-        Rate64 o;
-        per_box(b, [&](int bu) {
-            const BoxK K = box_k(A.boxes[bu], true);
-            const ListFmt L = list_fmt(A, bu, s);
-            const bool inner = wave_interior(A.r[s], K), cond = (K.terms & 8) != 0;
-            with_form(L, [&](auto lf) {
-                constexpr int F = decltype(lf)::value;
-                if (inner)
-                    o = cond ? rates64_walk<U64, true, false, F>(A, K, L, s, ns) : rates64_walk<U64, false, false, F>(A, K, L, s, ns);
-                else
-                    o = cond ? rates64_walk<U64, true, true, F>(A, K, L, s, ns) : rates64_walk<U64, false, true, F>(A, K, L, s, ns);
-            });
-        });
+    per_box(b, [&](int bu) {
+        if (!takes_part(cdyn(A, bu), state_mask)) return;
         const double2 ac = A.aco[s];
-        a = make_double2(o.ax + ac.x, o.ay + ac.y);
-        ud = o.ud + A.uco[s];
-        if (!isfinite(a.x) || !isfinite(a.y) || !isfinite(ud)) flag_health(A.dyn, b, HEALTH_NONFINITE);
+        a = make_double2(a.x + ac.x, a.y + ac.y);
+        ud += A.uco[s];
+        if (!isfinite(a.x) || !isfinite(a.y) || !isfinite(ud)) flag_health(A.dyn, bu, HEALTH_NONFINITE);
         A.acc[s] = a;
         A.udot[s] = ud;
-    }
-    if (step) step_tail(A, 0, s, b, on, a, ud);
+    });
+    if (step) step_tail(A, fp32, s, b, a, ud);
+}
+
+template <int U64, int S, int SUMS>
+__global__ __launch_bounds__(PASS_NT_MAX, U64 == 4 ? 3 : 4) void k_rates64(ArenaView A, int state_mask, int step)
+{
+    int sub;
+    const int s = pass_slot<S>(A, sub), sl = s < A.n ? s : 0;
+    Own64 own;
+    const int bs = slot_owner(A, s);
+    own.c = A.cnt[sl];
+    own.r = A.r[sl];
+    own.v = A.vp[sl];
+    own.g0 = first_cell(A, sl, false, sub);
+    const double4 Si = A.S[sl];
+    const double2 Qi = A.Q[sl];
+    double2 a = make_double2(0.0, 0.0);
+    double ud = 0.0;
+    per_box(bs, [&](int bu) {
+        CBox &B = cbox(A, bu);
+        CDyn &D = cdyn(A, bu);
+        const BoxK K = box_k(B);
+        if (!takes_part(D, state_mask)) return;
+        const int ns = (B.terms & 13) ? (own.c.x & CNT_MASK) : 0;
+        const ListFmt L = list_fmt(B, D, own.c.x);
+        const bool inner = S == 1 && wave_interior(own.r, K), cond = (K.terms & 8) != 0;
+        Rate64 o;
+        with_walk<SUMS>(L, [&](auto lf, auto grp) {
+            constexpr int F = decltype(lf)::value;
+            constexpr bool G = decltype(grp)::value;
+            if constexpr (S == 1) {
+                if (inner) {
+                    o = cond ? rates64_walk<U64, S, G, true, false, F>(A, K, L, s, sub, ns, own, Si, Qi) : rates64_walk<U64, S, G, false, false, F>(A, K, L, s, sub, ns, own, Si, Qi);
+                    return;
+                }
+            }
+            o = cond ? rates64_walk<U64, S, G, true, true, F>(A, K, L, s, sub, ns, own, Si, Qi) : rates64_walk<U64, S, G, false, true, F>(A, K, L, s, sub, ns, own, Si, Qi);
+        });
+        a = make_double2(o.ax, o.ay);
+        ud = o.ud;
+    });
+    rates_tail<S>(A, 0, state_mask, step, s, sub, bs, a, ud);
 }
 
 // P3 of the FP32C form over the short entries; adds the cohesive part from
 // P1; step as in k_rates64.
-template <int U32>
-__global__ __launch_bounds__(PASS_NT_MAX) void k_rates32(ArenaView A, int state_mask, int step)
+template <int U32, int S, int SUMS>
+__global__ __launch_bounds__(PASS_NT_MAX, 4) void k_rates32(ArenaView A, int state_mask, int step)
 {
-    const int s = xcd_block() * (int)blockDim.x + threadIdx.x;
-    int b = -1;
-    bool on = false;
-    if (s < A.n) {
-        b = A.slot_box[s];
-        on = b >= 0 && state_in(A.dyn[b].state, state_mask) && !A.dyn[b].relist;
-    }
+    int sub;
+    const int s = pass_slot<S>(A, sub), sl = s < A.n ? s : 0;
+    Own32 own;
+    const int bs = slot_owner(A, s);
+    own.c = A.cnt[sl];
+    own.r = A.rf[sl];
+    own.lo = A.rlo[sl];
+    own.g0 = first_cell(A, sl, false, sub);
+    const float4 Si = A.S32[sl];
+    const QRec32 q = A.q32[sl];
+    const float2 qi = make_float2(q.qx, q.qy);
     double2 a = make_double2(0.0, 0.0);
     double ud = 0.0;
-    if (on) {
-        const BoxDesc &B = A.boxes[b];
-        const int ns = (B.terms & 13u) ? (A.cnt[s].x & CNT_MASK) : 0;
+    per_box(bs, [&](int bu) {
+        CBox &B = cbox(A, bu);
+        CDyn &D = cdyn(A, bu);
+        const BoxF F = boxf(B);
+        if (!takes_part(D, state_mask)) return;
+        const int ns = (B.terms & 13) ? (own.c.x & CNT_MASK) : 0;
+        const ListFmt L = list_fmt(B, D, own.c.x);
         Rate32 o = {0.0, 0.0, 0.0};
-        per_box(b, [&](int bu) {
-            const BoxF F = boxf(A.boxes[bu], true);
-            const ListFmt L = list_fmt(A, bu, s);
-            with_form(L, [&](auto lf) {
-                constexpr int LF = decltype(lf)::value;
-                if (F.terms & 8) rates32_walk<U32, true, LF>(A, F, L, s, ns, o);
-                else rates32_walk<U32, false, LF>(A, F, L, s, ns, o);
-            });
+        with_walk<SUMS>(L, [&](auto lf, auto grp) {
+            constexpr int LF = decltype(lf)::value;
+            constexpr bool G = decltype(grp)::value;
+            if (F.terms & 8) rates32_walk<U32, S, G, true, LF>(A, F, L, s, sub, ns, own, Si, qi, o);
+            else rates32_walk<U32, S, G, false, LF>(A, F, L, s, sub, ns, own, Si, qi, o);
         });
-        const double2 ac = A.aco[s];
-        a = make_double2(o.ax + ac.x, o.ay + ac.y);
-        ud = o.ud + A.uco[s];
-        if (!isfinite(a.x) || !isfinite(a.y) || !isfinite(ud)) flag_health(A.dyn, b, HEALTH_NONFINITE);
-        A.acc[s] = a;
-        A.udot[s] = ud;
-    }
-    if (step) step_tail(A, 1, s, b, on, a, ud);
+        a = make_double2(o.ax, o.ay);
+        ud = o.ud;
+    });
+    rates_tail<S>(A, 1, state_mask, step, s, sub, bs, a, ud);
 }
 
 // The step pass as a launch of its own (the schedule's unfused form): the
@@ -2162,20 +2364,10 @@ __global__ __launch_bounds__(PASS_NT_MAX) void k_rates32(ArenaView A, int state_
 // rates that pass stored.  The same bits either way.
 __global__ __launch_bounds__(NT) void k_leapfrog(ArenaView A, int fp32)
 {
-    const int s = xcd_block() * NT + threadIdx.x;
-    int b = -1;
-    bool on = false;
-    double2 a = make_double2(0.0, 0.0);
-    double ud = 0.0;
-    if (s < A.n) {
-        b = A.slot_box[s];
-        on = b >= 0 && A.dyn[b].state == BOX_RUN && !A.dyn[b].relist;
-        if (on) {
-            a = A.acc[s];
-            ud = A.udot[s];
-        }
-    }
-    step_tail(A, fp32, s, b, on, a, ud);
+    const int s = xcd_block() * NT + threadIdx.x, sl = s < A.n ? s : 0;
+    const double2 a = A.acc[sl];
+    const double ud = A.udot[sl];
+    step_tail(A, fp32, s, slot_owner(A, s), a, ud);
 }
 
 // ===========================================================================
@@ -2753,19 +2945,53 @@ void launch_build_lists(const ArenaView &A, int force_mask, int fp32, hipStream_
 {
     hipLaunchKernelGGL(k_build_lists, tile_grid(A), dim3(NT), 0, st, A, force_mask, fp32);
 }
+// Lanes that share a slot's list in the pair passes.  One lane per slot
+// leaves the chip's 1024 SIMDs with less than two waves each up to ~100k
+// slots, and a pass then lasts as long as one lane's serial walk of ~58
+// entries (about 200 cycles each), whatever the slot count: 14 us for the
+// density pass of 1,024 slots as of 32,768.  Sharing a list shortens the walk
+// while the waves it adds still find idle SIMDs; past that it only repeats
+// the per-slot work.  Measured step times with 1 / 2 / 4 lanes (us; FP64,
+// FP32C within 2 us of it): 1,024 slots 46.6 / 37.4 / 32.5, 12,345: 51.0 /
+// 41.4 / 36.0, 32,768: 50.5 / 40.8 / 40.8, 49,152: 53.5 / 48.7 / 48.9,
+// 65,536: 58.0 / 51.8 / 61.2, 98,304: 70.1 / 62.5 / 82.2, 131,072: 71.8 /
+// 78.1 / 99.8.  The lines lie where two waves a SIMD are reached with 4 lanes
+// and three with 2.  The bits do not depend on it (fold_groups).  Only rounds
+// of four entries share (FP64 also of two): the depths the tuned schedules
+// and the defaults use.
+static inline int lanes_per_slot(const ArenaView &A)
+{
+    static_assert(98304 <= SUM_GROUP_MAX, "shared lists sum in groups");
+    return A.n <= 32768 ? 4 : (A.n <= 98304 ? 2 : 1);
+}
+
 // unroll: entries in flight per lane (1, 2 or 4; anything else = default)
+#define SPH_LAUNCH(K, ...) hipLaunchKernelGGL(K, g, b, 0, st, __VA_ARGS__)
+#define SPH_SUMS(K, U, ...)                                                                      \
+    do {                                                                                         \
+        if (A.sums == SUMS_PLAIN) SPH_LAUNCH((K<U, 1, SUMS_PLAIN>), __VA_ARGS__);                \
+        else if (A.sums == SUMS_GROUPS) SPH_LAUNCH((K<U, 1, SUMS_GROUPS>), __VA_ARGS__);         \
+        else SPH_LAUNCH((K<U, 1, SUMS_MIXED>), __VA_ARGS__);                                     \
+    } while (0)
+#define SPH_LANES(K, U, ...)                                                                     \
+    do {                                                                                         \
+        if (S == 4) SPH_LAUNCH((K<U, 4, SUMS_GROUPS>), __VA_ARGS__);                             \
+        else if (S == 2) SPH_LAUNCH((K<U, 2, SUMS_GROUPS>), __VA_ARGS__);                        \
+        else SPH_SUMS(K, U, __VA_ARGS__);                                                        \
+    } while (0)
 #define SPH_DISPATCH(K64, K32, ...)                                                              \
     do {                                                                                         \
-        const int bs_ = pass_block_of(A);                                                        \
-        const dim3 g = grid_for_bs(A.n, bs_), b(bs_);                                            \
+        const int S = unroll == 1 || (fp32 && unroll == 2) ? 1 : lanes_per_slot(A);              \
+        const int bs_ = S > 1 ? NT : pass_block_of(A);                                           \
+        const dim3 g = grid_for_bs((long long)A.n * S, bs_), b(bs_);                             \
         if (fp32) {                                                                              \
-            if (unroll == 1) hipLaunchKernelGGL(K32<1>, g, b, 0, st, __VA_ARGS__);               \
-            else if (unroll == 2) hipLaunchKernelGGL(K32<2>, g, b, 0, st, __VA_ARGS__);          \
-            else hipLaunchKernelGGL(K32<4>, g, b, 0, st, __VA_ARGS__);                           \
+            if (unroll == 1) SPH_LAUNCH((K32<1, 1, SUMS_MIXED>), __VA_ARGS__);                   \
+            else if (unroll == 2) SPH_LAUNCH((K32<2, 1, SUMS_MIXED>), __VA_ARGS__);              \
+            else SPH_LANES(K32, 4, __VA_ARGS__);                                                 \
         } else {                                                                                 \
-            if (unroll == 1) hipLaunchKernelGGL(K64<1>, g, b, 0, st, __VA_ARGS__);               \
-            else if (unroll == 4) hipLaunchKernelGGL(K64<4>, g, b, 0, st, __VA_ARGS__);          \
-            else hipLaunchKernelGGL(K64<2>, g, b, 0, st, __VA_ARGS__);                           \
+            if (unroll == 1) SPH_LAUNCH((K64<1, 1, SUMS_MIXED>), __VA_ARGS__);                   \
+            else if (unroll == 4) SPH_LANES(K64, 4, __VA_ARGS__);                                \
+            else SPH_LANES(K64, 2, __VA_ARGS__);                                                 \
         }                                                                                        \
     } while (0)
 
