@@ -82,8 +82,8 @@ constexpr size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 constexpr size_t NOALLOC_REC_BYTES = align256(sizeof(double4) * NOALLOC_MAX_PARTICLES);
 constexpr size_t NOALLOC_KEY_BYTES = align256(sizeof(unsigned) * 5 * NOALLOC_MAX_PARTICLES);
 constexpr size_t NOALLOC_CS_BYTES = align256(sizeof(int) * (NOALLOC_MAX_CELLS + 1));
-constexpr size_t NOALLOC_SCRATCH_BYTES = 2 * NOALLOC_REC_BYTES + NOALLOC_KEY_BYTES + NOALLOC_CS_BYTES +
-                                         NOALLOC_SORT_BYTES;
+constexpr size_t NOALLOC_SCRATCH_BYTES = SPLASH_HEAD_BYTES + 2 * NOALLOC_REC_BYTES + NOALLOC_KEY_BYTES +
+                                         NOALLOC_CS_BYTES + NOALLOC_SORT_BYTES;
 constexpr int NOALLOC_MAX_DEVICES = 64;
 std::mutex g_noalloc_mu;
 void *g_noalloc_scratch[NOALLOC_MAX_DEVICES] = {};
@@ -112,6 +112,31 @@ struct sph_ctx {
     // scratch for the stateless helpers (kernel, minimum image)
     double *d_scratch = nullptr;
     size_t scratch_bytes = 0;
+
+    // workspace of sph_splash_map_2d, kept from call to call up to
+    // RENDER_KEEP bytes
+    static constexpr size_t RENDER_KEEP = (size_t)256 << 20;
+    std::mutex render_mu;
+    char *d_render = nullptr;
+    size_t render_bytes = 0;
+
+    int render_space(size_t bytes)
+    {
+        if (bytes <= render_bytes) return SPH_OK;
+        dfree(d_render);
+        render_bytes = 0;
+        if (int rc = dalloc(&d_render, bytes)) return rc;
+        render_bytes = bytes;
+        return SPH_OK;
+    }
+
+    void render_trim()
+    {
+        if (render_bytes <= RENDER_KEEP) return;
+        (void)hipStreamSynchronize(stream);
+        dfree(d_render);
+        render_bytes = 0;
+    }
 
     int scratch(size_t bytes)
     {
@@ -1288,6 +1313,7 @@ int sph_ctx_destroy(sph_ctx *ctx)
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     dfree(ctx->d_scratch);
+    dfree(ctx->d_render);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return SPH_OK;
@@ -2038,10 +2064,16 @@ int sph_box_snapshot(sph_box *box, double *r, double *v, double *u, double *m)
     return SPH_OK;
 }
 
+static constexpr int64_t SPLASH_FINE_CELLS = 65536;
+
 // Cell grid of the rendering: cells at least one cutoff wide, periods
 // (xmax, ymax) as interpolate.py:79 uses them.
-static int splash_grid(const double *bounds, double cutoff, SplashGrid &G)
+// Its cells are the coarsest a rendering takes; the device refines them to
+// the particles' reach (splash_fine) up to max_cells: about one particle a
+// cell, at most 65,536 (two passes of the cell sort).
+static int splash_grid(const double *bounds, double cutoff, int64_t n, SplashGrid &G)
 {
+    memset(&G, 0, sizeof(G));
     const double Lx = bounds[1], Ly = bounds[3];
     if (!(Lx > 0) || !(Ly > 0)) return fail(SPH_ERR_ARG, "bounds need xmax, ymax > 0");
     G.Lx = Lx; G.Ly = Ly; G.cutoff = cutoff;
@@ -2050,6 +2082,8 @@ static int splash_grid(const double *bounds, double cutoff, SplashGrid &G)
     G.ncx = G.ncx < 3 ? 1 : std::min(G.ncx, 4096);
     G.ncy = G.ncy < 3 ? 1 : std::min(G.ncy, 4096);
     G.cwx = Lx / G.ncx; G.cwy = Ly / G.ncy;
+    const int64_t fine = std::min<int64_t>(std::max<int64_t>(n, 256), SPLASH_FINE_CELLS);
+    G.max_cells = (int)std::max<int64_t>((int64_t)G.ncx * G.ncy, fine);
     return SPH_OK;
 }
 
@@ -2063,58 +2097,58 @@ int sph_splash_map_2d(sph_ctx *ctx, int64_t n, const double *r, const double *m,
     if (n > (1ll << 30) || (long long)nx * ny > (1ll << 31))
         return fail(SPH_ERR_ARG, "too many particles or pixels");
     SplashGrid G;
-    if (int rc = splash_grid(bounds, cutoff, G)) return rc;
+    if (int rc = splash_grid(bounds, cutoff, n, G)) return rc;
     HIPCHK(hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
-    const int ncell = G.ncx * G.ncy;
     const size_t np = (size_t)nx * ny;
-    double *d_in = nullptr, *d_xy = nullptr, *d_Z = nullptr;
-    double4 *d_rec = nullptr, *d_rec2 = nullptr;
-    unsigned *d_keys = nullptr;
-    int *d_cs = nullptr;
-    void *d_tmp = nullptr;
     const size_t N = (size_t)std::max<int64_t>(n, 1);
-    const size_t tmp_bytes = radix_sort_temp_bytes((int)N);
-    int rc = 0;
-    rc |= dalloc(&d_in, 6 * N);  // r (2n), m, rho, a, h
-    rc |= dalloc(&d_xy, (size_t)nx + ny);
-    rc |= dalloc(&d_Z, np);
-    rc |= dalloc(&d_rec, N);
-    rc |= dalloc(&d_rec2, N);
-    rc |= dalloc(&d_keys, 5 * N);
-    rc |= dalloc(&d_cs, (size_t)ncell + 1);
-    rc |= dalloc((char **)&d_tmp, tmp_bytes);
-    if (!rc) {
-        const size_t b = sizeof(double) * n;
-        if (n > 0) {
-            if (hipMemcpyAsync(d_in, r, 2 * b, hipMemcpyHostToDevice, st) ||
-                hipMemcpyAsync(d_in + 2 * n, m, b, hipMemcpyHostToDevice, st) ||
-                hipMemcpyAsync(d_in + 3 * n, rho, b, hipMemcpyHostToDevice, st) ||
-                hipMemcpyAsync(d_in + 4 * n, a, b, hipMemcpyHostToDevice, st) ||
-                hipMemcpyAsync(d_in + 5 * n, h, b, hipMemcpyHostToDevice, st))
-                rc = fail(SPH_ERR_HIP, "hipMemcpyAsync failed");
-        }
-        if (!rc && (hipMemcpyAsync(d_xy, x, sizeof(double) * nx, hipMemcpyHostToDevice, st) ||
-                    hipMemcpyAsync(d_xy + nx, y, sizeof(double) * ny, hipMemcpyHostToDevice, st)))
-            rc = fail(SPH_ERR_HIP, "hipMemcpyAsync failed");
-        if (!rc) {
-            unsigned *k_in = d_keys, *k_out = d_keys + N, *v_out = d_keys + 2 * N, *k_alt = d_keys + 3 * N,
-                     *v_alt = d_keys + 4 * N;
-            launch_splash(n, d_in, d_in + 2 * n, d_in + 3 * n, d_in + 4 * n, d_in + 5 * n, G, d_rec, d_rec2, k_in,
-                          k_out, v_out, k_alt, v_alt, d_tmp, bits_for(ncell), d_cs, nx, ny, d_xy, d_xy + nx, d_Z,
-                          st);
-            if (hipGetLastError() != hipSuccess) rc = fail(SPH_ERR_HIP, "splash launch failed");
-            if (!rc && hipMemcpyAsync(Z, d_Z, sizeof(double) * np, hipMemcpyDeviceToHost, st))
-                rc = fail(SPH_ERR_HIP, "hipMemcpyAsync failed");
-            if (!rc && hipStreamSynchronize(st)) rc = fail(SPH_ERR_HIP, "hipStreamSynchronize failed");
-        }
-    } else {
-        rc = fail(SPH_ERR_NOMEM, "device allocation failed");
+    // the context's rendering workspace (eight allocations and frees a call
+    // took most of a small image's time): inputs, pixel coordinates,
+    // the image and the launch's scratch
+    const size_t in_b = align256(sizeof(double) * 6 * N), xy_b = align256(sizeof(double) * ((size_t)nx + ny));
+    const size_t z_b = align256(sizeof(double) * np), rec_b = align256(sizeof(double4) * N);
+    const size_t key_b = align256(sizeof(unsigned) * N), cs_b = align256(sizeof(int) * ((size_t)G.max_cells + 1));
+    const size_t tmp_b = align256(radix_sort_temp_bytes((int)N));
+    std::lock_guard<std::mutex> lk(ctx->render_mu);  // calls of several threads take turns
+    if (ctx->render_space(in_b + xy_b + z_b + SPLASH_HEAD_BYTES + 2 * rec_b + 5 * key_b + cs_b + tmp_b))
+        return SPH_ERR_NOMEM;
+    struct Trim {
+        sph_ctx *c;
+        ~Trim() { c->render_trim(); }
+    } trim{ctx};
+    char *at = ctx->d_render;
+    auto take = [&](size_t b) {
+        char *p = at;
+        at += b;
+        return p;
+    };
+    double *d_in = (double *)take(in_b), *d_xy = (double *)take(xy_b), *d_Z = (double *)take(z_b);  // r (2n), m, rho, a, h
+    SplashScratch W;
+    W.head = take(SPLASH_HEAD_BYTES);
+    W.rec = (double4 *)take(rec_b);
+    W.rec_sorted = (double4 *)take(rec_b);
+    W.keys = (unsigned *)take(key_b);
+    W.k_out = (unsigned *)take(key_b);
+    W.v_out = (unsigned *)take(key_b);
+    W.k_alt = (unsigned *)take(key_b);
+    W.v_alt = (unsigned *)take(key_b);
+    W.cs = (int *)take(cs_b);
+    W.sort_tmp = take(tmp_b);
+    const size_t b = sizeof(double) * (size_t)n;
+    if (n > 0) {
+        HIPCHK(hipMemcpyAsync(d_in, r, 2 * b, hipMemcpyHostToDevice, st));
+        HIPCHK(hipMemcpyAsync(d_in + 2 * n, m, b, hipMemcpyHostToDevice, st));
+        HIPCHK(hipMemcpyAsync(d_in + 3 * n, rho, b, hipMemcpyHostToDevice, st));
+        HIPCHK(hipMemcpyAsync(d_in + 4 * n, a, b, hipMemcpyHostToDevice, st));
+        HIPCHK(hipMemcpyAsync(d_in + 5 * n, h, b, hipMemcpyHostToDevice, st));
     }
-    (void)hipStreamSynchronize(st);
-    dfree(d_in); dfree(d_xy); dfree(d_Z); dfree(d_rec); dfree(d_rec2); dfree(d_keys); dfree(d_cs);
-    if (d_tmp) (void)hipFree(d_tmp);
-    return rc;
+    HIPCHK(hipMemcpyAsync(d_xy, x, sizeof(double) * nx, hipMemcpyHostToDevice, st));
+    HIPCHK(hipMemcpyAsync(d_xy + nx, y, sizeof(double) * ny, hipMemcpyHostToDevice, st));
+    launch_splash(n, d_in, d_in + 2 * n, d_in + 3 * n, d_in + 4 * n, d_in + 5 * n, G, W, nx, d_xy, ny, d_xy + nx, d_Z, st);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(Z, d_Z, sizeof(double) * np, hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    return SPH_OK;
 }
 
 int sph_splash_map_2d_noalloc(sph_ctx *ctx, int64_t n, const double *r, const double *m, const double *rho,
@@ -2129,7 +2163,7 @@ int sph_splash_map_2d_noalloc(sph_ctx *ctx, int64_t n, const double *r, const do
                                      " particles (its fixed scratch); use sph_splash_map_2d");
     if ((long long)nx * ny > (1ll << 31)) return fail(SPH_ERR_ARG, "too many pixels");
     SplashGrid G;
-    if (int rc = splash_grid(bounds, cutoff, G)) return rc;
+    if (int rc = splash_grid(bounds, cutoff, n, G)) return rc;
     const int ncell = G.ncx * G.ncy;
     if (ncell > NOALLOC_MAX_CELLS)
         return fail(SPH_ERR_ARG, "sph_splash_map_2d_noalloc holds at most " + std::to_string(NOALLOC_MAX_CELLS) +
@@ -2139,16 +2173,23 @@ int sph_splash_map_2d_noalloc(sph_ctx *ctx, int64_t n, const double *r, const do
     unsigned char *base = (unsigned char *)g_noalloc_scratch[ctx->device];
     if (!base) return fail(SPH_ERR_STATE, "scratch address not set up for this device");
     HIPCHK(hipSetDevice(ctx->device));
-    double4 *d_rec = (double4 *)base;
-    double4 *d_rec2 = (double4 *)(base + NOALLOC_REC_BYTES);
-    unsigned *d_keys = (unsigned *)(base + 2 * NOALLOC_REC_BYTES);
-    int *d_cs = (int *)(base + 2 * NOALLOC_REC_BYTES + NOALLOC_KEY_BYTES);
-    void *d_tmp = base + 2 * NOALLOC_REC_BYTES + NOALLOC_KEY_BYTES + NOALLOC_CS_BYTES;
-    // every scratch word a launch reads it first writes (records, keys, the
-    // cell starts of all ncell + 1 cells, the counters of every tile), so
-    // nothing needs clearing between calls
-    launch_splash(n, r, m, rho, a, h, G, d_rec, d_rec2, d_keys, d_keys + N, d_keys + 2 * N, d_keys + 3 * N,
-                  d_keys + 4 * N, d_tmp, bits_for(ncell), d_cs, nx, ny, x, y, Z, ctx->stream);
+    G.max_cells = std::min(G.max_cells, NOALLOC_MAX_CELLS);
+    SplashScratch W;
+    W.head = base;
+    W.rec = (double4 *)(base + SPLASH_HEAD_BYTES);
+    W.rec_sorted = (double4 *)(base + SPLASH_HEAD_BYTES + NOALLOC_REC_BYTES);
+    unsigned char *rest = base + SPLASH_HEAD_BYTES + 2 * NOALLOC_REC_BYTES;
+    W.keys = (unsigned *)rest;
+    W.k_out = W.keys + N;
+    W.v_out = W.keys + 2 * N;
+    W.k_alt = W.keys + 3 * N;
+    W.v_alt = W.keys + 4 * N;
+    W.cs = (int *)(rest + NOALLOC_KEY_BYTES);
+    W.sort_tmp = rest + NOALLOC_KEY_BYTES + NOALLOC_CS_BYTES;
+    // every scratch word a launch reads it first writes (the head, records,
+    // keys, the cell starts of all cells and one more, the counters of every
+    // tile), so nothing needs clearing between calls
+    launch_splash(n, r, m, rho, a, h, G, W, nx, x, ny, y, Z, ctx->stream);
     HIPCHK(hipGetLastError());
     return SPH_OK;
 }

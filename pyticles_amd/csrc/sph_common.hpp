@@ -210,10 +210,13 @@ struct ArenaView {
     int pass_block;      // work-items per block of the pair passes (128, 256 or 512)
 };
 
-// Grid of the splash rendering: particle cells at least one cutoff wide.
+// Cell grid of the splash rendering: cells at least as wide as the largest
+// reach of a particle (the host's, one cutoff wide, is the coarsest).
 struct SplashGrid {
     double Lx, Ly, cwx, cwy, cutoff;
     int ncx, ncy;
+    int max_cells;  // cells there is room for
+    int pad;
 };
 
 }  // namespace sph

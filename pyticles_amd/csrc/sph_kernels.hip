@@ -2805,16 +2805,72 @@ __global__ __launch_bounds__(NT) void k_energy_now(ArenaView A, int box, double 
 // SPH scatter to a grid (interpolate.splash_map_2d) as a per-pixel gather
 // ===========================================================================
 
-// Particle record (x, y wrapped into the periods, w = a m / rho, h) and its
-// cell key.
+// Largest smoothing length per block (NaN and negative lengths reach nothing
+// and count as 0).
+static constexpr int SPLASH_HB = 64;  // blocks, and partial maxima, of k_splash_hmax
+
+__global__ __launch_bounds__(NT) void k_splash_hmax(long long n, const double *__restrict__ h,
+                                                     double *__restrict__ part)
+{
+    __shared__ double wmax[NT / 64];
+    double m = 0.0;
+    for (long long i = (long long)blockIdx.x * NT + threadIdx.x; i < n; i += (long long)SPLASH_HB * NT) m = fmax(m, h[i]);
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) m = fmax(m, __shfl_xor(m, off));
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < NT / 64; ++w) m = fmax(m, wmax[w]);
+        part[blockIdx.x] = m;
+    }
+}
+
+// Cell grid of a rendering.  A particle reaches min(cutoff, h_p), so cells
+// need only be as wide as the largest reach: at the usual cutoff of h plus
+// one or two pixels, cells one cutoff wide gave a pixel up to four times the
+// candidates (144 of them at h = 2, cutoff = 4, for 13 in reach).  C holds
+// the grid of cells one cutoff wide and the most cells there is room for; a
+// grid that would take more is coarsened, down to C's.
+__device__ __forceinline__ SplashGrid splash_fine(const SplashGrid &C, double hmax)
+{
+    SplashGrid G = C;
+    const double reach = (hmax < C.cutoff && hmax > 0.0 ? hmax : C.cutoff) * (1.0 + 1e-9);
+    double fx = fmin(floor(C.Lx / reach), 4096.0), fy = fmin(floor(C.Ly / reach), 4096.0);
+    const double over = fx * fy / (double)C.max_cells;
+    if (over > 1.0) {
+        const double f = 1.0 / sqrt(over);
+        fx = floor(fx * f);
+        fy = floor(fy * f);
+    }
+    int nx = (int)fx, ny = (int)fy;
+    nx = nx < 3 ? 1 : nx;
+    ny = ny < 3 ? 1 : ny;
+    if (nx < C.ncx || ny < C.ncy) return G;
+    G.ncx = nx;
+    G.ncy = ny;
+    G.cwx = C.Lx / nx;
+    G.cwy = C.Ly / ny;
+    return G;
+}
+
+// The grid (block 0 leaves it in *grid for the kernels that follow), and per
+// particle its record (x, y as given, a m / rho times the kernel norm
+// 5 / (pi h^2), 1 / h) and its cell key (of the position wrapped into the
+// periods).
 __global__ __launch_bounds__(NT) void k_splash_prep(long long n, const double *__restrict__ r,
                                                      const double *__restrict__ m,
                                                      const double *__restrict__ rho,
                                                      const double *__restrict__ a,
-                                                     const double *__restrict__ h, SplashGrid G,
+                                                     const double *__restrict__ h, SplashGrid C,
+                                                     const double *__restrict__ part, SplashGrid *grid,
                                                      double4 *__restrict__ rec, unsigned *__restrict__ keys)
 {
+    double hm = n > 0 ? part[threadIdx.x & (SPLASH_HB - 1)] : 0.0;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) hm = fmax(hm, __shfl_xor(hm, off));
+    const SplashGrid G = splash_fine(C, hm);
     const long long i = (long long)blockIdx.x * NT + threadIdx.x;
+    if (i == 0) *grid = G;
     if (i >= n) return;
     double x = r[2 * i], y = r[2 * i + 1];
     x -= G.Lx * floor(x / G.Lx);
@@ -2822,7 +2878,11 @@ __global__ __launch_bounds__(NT) void k_splash_prep(long long n, const double *_
     int cx = (int)(x / G.cwx), cy = (int)(y / G.cwy);
     cx = cx < 0 ? 0 : (cx >= G.ncx ? G.ncx - 1 : cx);
     cy = cy < 0 ? 0 : (cy >= G.ncy ? G.ncy - 1 : cy);
-    rec[i] = make_double4(r[2 * i], r[2 * i + 1], a[i] * m[i] / rho[i], h[i]);
+    const double hp = h[i];
+    // a length that is not positive reaches nothing (1 / h = inf: q >= 1 or NaN)
+    const bool on = hp > 0.0;
+    rec[i] = make_double4(r[2 * i], r[2 * i + 1], on ? a[i] * m[i] / rho[i] * (5.0 / (SPH_PI * hp * hp)) : 0.0,
+                          on ? 1.0 / hp : __longlong_as_double(0x7ff0000000000000ll));
     keys[i] = (unsigned)(cy * G.ncx + cx);
 }
 
@@ -2836,63 +2896,102 @@ __global__ __launch_bounds__(NT) void k_splash_gather(long long n, const unsigne
 }
 
 // cs[c] = first sorted particle with key >= c, c in [0, ncell]
-__global__ __launch_bounds__(NT) void k_splash_cells(long long n, const unsigned *__restrict__ keys, int ncell,
-                                                      int *__restrict__ cs)
+__global__ __launch_bounds__(NT) void k_splash_cells(long long n, const unsigned *__restrict__ keys,
+                                                      const SplashGrid *__restrict__ grid, int *__restrict__ cs)
 {
     const long long i = (long long)blockIdx.x * NT + threadIdx.x;
     if (i > n) return;
-    const int k = i == n ? ncell : (int)keys[i];
+    const int k = i == n ? grid->ncx * grid->ncy : (int)keys[i];
     const int kp = i == 0 ? -1 : (int)keys[i - 1];
     for (int c = kp + 1; c <= k; ++c) cs[c] = (int)i;
 }
 
+// Rows of a pixel block's tile, as a power of two, for waves of 2^li rows:
+// 16 x 16 pixels of 8 x 8 waves, or one line of 256 along a grid's long axis.
+__host__ __device__ inline int splash_block_bits(int li) { return li == 3 ? 4 : (li == 0 ? 0 : 8); }
+
 // One thread per pixel (i, j) at (x[i], y[j]); Z[i * ny + j] sums
 // w_p W(s, h_p) over particles within the cutoff (minimum image with periods
 // Lx, Ly, dr = (x_p - x, y - y_p) as interpolate.py:76).  Cells are at least
-// the cutoff wide, so the 3x3 stencil of the pixel's cell holds them all
-// (every cell when an axis has fewer than three).
-__global__ __launch_bounds__(NT) void k_splash_pixels(int nx, int ny, const double *__restrict__ x,
-                                                       const double *__restrict__ y, SplashGrid G,
+// the largest reach wide, so the 3x3 stencil of the pixel's cell holds them
+// all (every cell when an axis has fewer than three); a row of the stencil is
+// one run of sorted particles, two where it crosses the period.
+//
+// A block renders 16 x 16 pixels, a wave 8 x 8 (grids narrower than eight
+// pixels: lines): the lanes of a wave share
+// most of their cells, so a record's load touches a few cache lines and the
+// runs end together.  (Along a pixel row a wave's lanes spread over 64 pixels
+// and 17 cells.)  Four records are in flight.  The image test is a branch
+// taken only near the sides, the kernel's norm and 1 / h come with the
+// record.  At 40,000 particles on 512 x 512 pixels, h = 2, cutoff = 4: 25 us
+// (100 us along pixel rows with cells one cutoff wide, two divisions and a
+// correctly rounded root per pair in reach); what bounds it now is the FP64
+// arithmetic of the pairs some lane of a wave has in reach.  The root is
+// sqrt_pair's and the partial sums keep the total's error at the level of the
+// running sum it replaces (3.29e-16 against 3.35e-16 in long double).
+__global__ __launch_bounds__(NT) void k_splash_pixels(long long tiles, int li, int nx, int ny,
+                                                       const double *__restrict__ x,
+                                                       const double *__restrict__ y,
+                                                       const SplashGrid *__restrict__ grid,
                                                        const double4 *__restrict__ rec,
                                                        const int *__restrict__ cs, double *__restrict__ Z)
 {
-    const long long pix = (long long)blockIdx.x * NT + threadIdx.x;
-    if (pix >= (long long)nx * ny) return;
-    const int i = (int)(pix / ny), j = (int)(pix % ny);
-    const double px = x[i], py = y[j];
-    double wx = px - G.Lx * floor(px / G.Lx), wy = py - G.Ly * floor(py / G.Ly);
-    int cx = (int)(wx / G.cwx), cy = (int)(wy / G.cwy);
-    cx = cx < 0 ? 0 : (cx >= G.ncx ? G.ncx - 1 : cx);
-    cy = cy < 0 ? 0 : (cy >= G.ncy ? G.ncy - 1 : cy);
-    const int sx = G.ncx >= 3 ? 1 : 0, sy = G.ncy >= 3 ? 1 : 0;
-    const int x0 = sx ? -1 : 0, x1 = sx ? 1 : G.ncx - 1, y0 = sy ? -1 : 0, y1 = sy ? 1 : G.ncy - 1;
-    const double c2 = G.cutoff * G.cutoff;
-    const double hLx = G.Lx / 2., hLy = G.Ly / 2.;
-    double z = 0.0;
-    for (int oy = y0; oy <= y1; ++oy) {
-        const int yy = sy ? wrapi(cy + oy, G.ncy) : oy;
-        for (int ox = x0; ox <= x1; ++ox) {
-            const int xx = sx ? wrapi(cx + ox, G.ncx) : ox;
-            const int c = yy * G.ncx + xx;
-            for (int t = cs[c]; t < cs[c + 1]; ++t) {
-                const double4 p = rec[t];
-                double dx = p.x - px, dy = py - p.y;
-                dx = dx > hLx ? dx - G.Lx : dx;  // neighbour_list.py:110-123 order
-                dy = dy > hLy ? dy - G.Ly : dy;
-                dx = dx < -hLx ? dx + G.Lx : dx;
-                dy = dy < -hLy ? dy + G.Ly : dy;
-                const double rsq = rsq_exact(dx, dy);
-                if (rsq < c2) {
-                    const double sr = sqrt(rsq);
-                    if (sr < p.w) {  // spkernel.lucy_w, 2-D
-                        const double q = sr / p.w, tt = 1.0 - q;
-                        z += p.z * ((5.0 / (SPH_PI * p.w * p.w)) * (1.0 + 3.0 * q) * (tt * tt * tt));
+    const SplashGrid G = *grid;
+    // block tile of 2^bi x 2^(8 - bi) pixels in waves of 2^li x 2^(6 - li)
+    const int bi = splash_block_bits(li), lj = 6 - li, wj = 8 - bi - lj;  // 2^wj waves across the tile
+    const int nbj = (int)(((long long)ny + (1 << (8 - bi)) - 1) >> (8 - bi));
+    const int w = (int)threadIdx.x >> 6, l = (int)threadIdx.x & 63;
+    for (long long tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const int i = ((int)(tile / nbj) << bi) + ((w >> wj) << li) + (l >> lj);
+        const int j = ((int)(tile % nbj) << (8 - bi)) + ((w & ((1 << wj) - 1)) << lj) + (l & ((1 << lj) - 1));
+        if (i >= nx || j >= ny) continue;
+        const double px = x[i], py = y[j];
+        const double wx = px - G.Lx * floor(px / G.Lx), wy = py - G.Ly * floor(py / G.Ly);
+        int cx = (int)(wx / G.cwx), cy = (int)(wy / G.cwy);
+        cx = cx < 0 ? 0 : (cx >= G.ncx ? G.ncx - 1 : cx);
+        cy = cy < 0 ? 0 : (cy >= G.ncy ? G.ncy - 1 : cy);
+        const bool sx = G.ncx >= 3, sy = G.ncy >= 3;
+        const int y0 = sy ? -1 : 0, y1 = sy ? 1 : G.ncy - 1;
+        const double c2 = G.cutoff * G.cutoff;
+        const double hLx = G.Lx / 2., hLy = G.Ly / 2.;
+        double z = 0.0;
+        auto run = [&](int c0, int c1) {  // the particles of cells c0 .. c1
+            const int t1 = cs[c1 + 1];
+            double zr[2] = {};  // partial sums, so that the total's rounding stays below one running sum's
+            for (int t = cs[c0]; t < t1; t += 4) {
+                double4 p[4];
+    #pragma unroll
+                for (int u = 0; u < 4; ++u) p[u] = rec[min(t + u, t1 - 1)];
+    #pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    double dx = p[u].x - px, dy = py - p[u].y;
+                    if (fabs(dx) > hLx || fabs(dy) > hLy) {
+                        dx = dx > hLx ? dx - G.Lx : dx;  // neighbour_list.py:110-123 order
+                        dy = dy > hLy ? dy - G.Ly : dy;
+                        dx = dx < -hLx ? dx + G.Lx : dx;
+                        dy = dy < -hLy ? dy + G.Ly : dy;
+                    }
+                    const double rsq = rsq_exact(dx, dy);
+                    if (t + u < t1 && rsq < c2) {
+                        const double q = sqrt_pair(rsq) * p[u].w, tt = 1.0 - q;
+                        if (q < 1.0) zr[u & 1] += p[u].z * ((1.0 + 3.0 * q) * (tt * tt * tt));  // spkernel.lucy_w, 2-D
                     }
                 }
             }
+            z += zr[0] + zr[1];
+        };
+        for (int oy = y0; oy <= y1; ++oy) {
+            const int row = (sy ? wrapi(cy + oy, G.ncy) : oy) * G.ncx;
+            if (!sx) {
+                run(row, row + G.ncx - 1);
+            } else {
+                run(row + max(cx - 1, 0), row + min(cx + 1, G.ncx - 1));
+                if (cx == 0) run(row + G.ncx - 1, row + G.ncx - 1);
+                else if (cx == G.ncx - 1) run(row, row);
+            }
         }
+        Z[(long long)i * ny + j] = z;
     }
-    Z[pix] = z;
 }
 
 // ===========================================================================
@@ -3048,18 +3147,26 @@ void launch_separations(const ArenaView &A, int box, const int *inv, long long n
     hipLaunchKernelGGL(k_separations, grid_for(np), dim3(NT), 0, st, A, box, inv, np, iap, drij, rij, rsq, dv);
 }
 void launch_splash(long long n, const double *r, const double *m, const double *rho, const double *a,
-                   const double *h, const SplashGrid &G, double4 *rec, double4 *rec_sorted, unsigned *keys,
-                   unsigned *k_out, unsigned *v_out, unsigned *k_alt, unsigned *v_alt, void *sort_tmp, int key_bits,
-                   int *cs, int nx, int ny, const double *x, const double *y, double *Z, hipStream_t st)
+                   const double *h, const SplashGrid &C, const SplashScratch &W, int nx, const double *x, int ny,
+                   const double *y, double *Z, hipStream_t st)
 {
+    double *part = (double *)W.head;
+    SplashGrid *grid = (SplashGrid *)((char *)W.head + sizeof(double) * SPLASH_HB);
+    static_assert(sizeof(double) * SPLASH_HB + sizeof(SplashGrid) <= SPLASH_HEAD_BYTES, "splash head");
+    if (n > 0) hipLaunchKernelGGL(k_splash_hmax, dim3(SPLASH_HB), dim3(NT), 0, st, n, h, part);
+    hipLaunchKernelGGL(k_splash_prep, grid_for(n), dim3(NT), 0, st, n, r, m, rho, a, h, C, part, grid, W.rec, W.keys);
     if (n > 0) {
-        hipLaunchKernelGGL(k_splash_prep, grid_for(n), dim3(NT), 0, st, n, r, m, rho, a, h, G, rec, keys);
-        radix_sort_pairs(keys, k_out, v_out, k_alt, v_alt, (int)n, key_bits, sort_tmp, st);
-        hipLaunchKernelGGL(k_splash_gather, grid_for(n), dim3(NT), 0, st, n, v_out, rec, rec_sorted);
+        int bits = 1;  // of the largest key the grid may have
+        while ((1ll << bits) < C.max_cells) ++bits;
+        radix_sort_pairs(W.keys, W.k_out, W.v_out, W.k_alt, W.v_alt, (int)n, bits, W.sort_tmp, st);
+        hipLaunchKernelGGL(k_splash_gather, grid_for(n), dim3(NT), 0, st, n, W.v_out, W.rec, W.rec_sorted);
     }
-    hipLaunchKernelGGL(k_splash_cells, grid_for(n + 1), dim3(NT), 0, st, n, k_out, G.ncx * G.ncy, cs);
-    const long long np = (long long)nx * ny;
-    hipLaunchKernelGGL(k_splash_pixels, grid_for(np), dim3(NT), 0, st, nx, ny, x, y, G, rec_sorted, cs, Z);
+    hipLaunchKernelGGL(k_splash_cells, grid_for(n + 1), dim3(NT), 0, st, n, W.k_out, grid, W.cs);
+    const int li = nx < 8 ? 0 : (ny < 8 ? 6 : 3), bi = splash_block_bits(li);
+    const long long ti = ((long long)nx + (1 << bi) - 1) >> bi, tj = ((long long)ny + (1 << (8 - bi)) - 1) >> (8 - bi);
+    const long long tiles = ti * tj;
+    hipLaunchKernelGGL(k_splash_pixels, dim3((unsigned)(tiles < (1 << 20) ? tiles : (1 << 20))), dim3(NT), 0, st, tiles, li,
+                       nx, ny, x, y, grid, W.rec_sorted, W.cs, Z);
 }
 void launch_lucy(long long np, const double *r, const double *dx, double h, int dim, double *w,
                  double *dwdx, hipStream_t st)

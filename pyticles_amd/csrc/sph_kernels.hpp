@@ -49,9 +49,20 @@ void launch_min_image(long long np, double *dr, double Lx, double Ly, hipStream_
 void launch_set_u(const ArenaView &A, int box, int n, const double *T, double T0, hipStream_t st);
 void launch_energy_now(const ArenaView &A, int box, double *out3, hipStream_t st);
 void launch_fp32_accumulate(long long n, const double *x, int unroll, double *out2, hipStream_t st);
+// Device scratch of a rendering of n particles (n >= 1 counts; the arrays of
+// one call, nothing in them need be cleared): SPLASH_HEAD_BYTES of head, n
+// records twice, n keys and values, the sort's counters and C.max_cells + 1
+// cell starts.
+constexpr size_t SPLASH_HEAD_BYTES = 1024;
+struct SplashScratch {
+    void *head;
+    double4 *rec, *rec_sorted;
+    unsigned *keys, *k_out, *v_out, *k_alt, *v_alt;
+    void *sort_tmp;
+    int *cs;
+};
 void launch_splash(long long n, const double *r, const double *m, const double *rho, const double *a,
-                   const double *h, const SplashGrid &G, double4 *rec, double4 *rec_sorted, unsigned *keys,
-                   unsigned *k_out, unsigned *v_out, unsigned *k_alt, unsigned *v_alt, void *sort_tmp, int key_bits,
-                   int *cs, int nx, int ny, const double *x, const double *y, double *Z, hipStream_t st);
+                   const double *h, const SplashGrid &C, const SplashScratch &W, int nx, const double *x, int ny,
+                   const double *y, double *Z, hipStream_t st);
 
 }  // namespace sph
