@@ -1219,6 +1219,16 @@ __device__ __forceinline__ bool takes_part(const CDyn &D, int state_mask)
     return (((1 << D.state) & state_mask) != 0) & (D.relist == 0);
 }
 
+// The bookkeeping of the plain step before this one, which launched no
+// k_box_step (single boxes): the step is counted.  Only the density pass may
+// do it: it reads no step count, and every later launch sees the new one.
+__device__ __forceinline__ void advance_step(const ArenaView &A, int advance)
+{
+    if (!advance || blockIdx.x != 0 || threadIdx.x != 0 || A.one_box < 0) return;
+    BoxDyn &D = A.dyn[A.one_box];
+    if (D.state == BOX_RUN && !D.relist && D.k < D.nsteps) D.k += 1;
+}
+
 // What a pass reads of its own slot before it knows the box: issued together
 // at the wave's start (slots past the end read slot 0).
 struct Own64 {
@@ -1360,8 +1370,9 @@ __device__ __forceinline__ Dens64 density64_walk(const ArenaView &A, const BoxK 
 //   du_co,i = -a  sum_j m_j (v_j - v_i) . dwdx_hl,ij      (dv . f / 2)
 // and the rate pass only walks the short entries (r < h + skin).
 template <int U64, int S, int SUMS>
-__global__ __launch_bounds__(PASS_NT_MAX, 4) void k_density64(ArenaView A, int state_mask)
+__global__ __launch_bounds__(PASS_NT_MAX, 4) void k_density64(ArenaView A, int state_mask, int advance)
 {
+    advance_step(A, advance);
     int sub;
     const int s = pass_slot<S>(A, sub), sl = s < A.n ? s : 0;
     Own64 own;
@@ -1847,8 +1858,9 @@ __device__ __forceinline__ void density32_walk(const ArenaView &A, const BoxF &F
 // P1 of the FP32C form: rf carries position and predicted velocity; the
 // cohesive rate part (see k_density64) is accumulated with the densities.
 template <int U32, int S, int SUMS>
-__global__ __launch_bounds__(PASS_NT_MAX, 4) void k_density32(ArenaView A, int state_mask)
+__global__ __launch_bounds__(PASS_NT_MAX, 4) void k_density32(ArenaView A, int state_mask, int advance)
 {
+    advance_step(A, advance);
     int sub;
     const int s = pass_slot<S>(A, sub), sl = s < A.n ? s : 0;
     Own32 own;
@@ -3094,9 +3106,9 @@ static inline int lanes_per_slot(const ArenaView &A)
         }                                                                                        \
     } while (0)
 
-void launch_density(const ArenaView &A, int fp32, int state_mask, int unroll, hipStream_t st)
+void launch_density(const ArenaView &A, int fp32, int state_mask, int unroll, hipStream_t st, int advance)
 {
-    SPH_DISPATCH(k_density64, k_density32, A, state_mask);
+    SPH_DISPATCH(k_density64, k_density32, A, state_mask, advance);
 }
 void launch_grad(const ArenaView &A, int fp32, int state_mask, int diag, int unroll, hipStream_t st)
 {

@@ -23,7 +23,9 @@ void launch_permute(const ArenaView &A, int force_mask, int cells, hipStream_t s
 void launch_box_sort(const ArenaView &A, int force_mask, int nbox, hipStream_t st);
 bool box_sort_fits(int ncells, int n);
 void launch_build_lists(const ArenaView &A, int force_mask, int fp32, hipStream_t st);
-void launch_density(const ArenaView &A, int fp32, int state_mask, int unroll, hipStream_t st);
+// advance != 0: also counts the step before this one (a plain step of a single
+// box launched without k_box_step)
+void launch_density(const ArenaView &A, int fp32, int state_mask, int unroll, hipStream_t st, int advance = 0);
 void launch_grad(const ArenaView &A, int fp32, int state_mask, int diag, int unroll, hipStream_t st);
 // step != 0: the stepping launch, which also takes each running slot's
 // leapfrog step into the second state buffers (and carries the other live
