@@ -1759,7 +1759,9 @@ int sph_energy(sph_box *box, double *ke, double *ue, double *etot)
     Arena &A = box->ar;
     HIPCHK(hipSetDevice(A.ctx->device));
     double out[3];
-    launch_energy_now(A.view(), box->b, A.d_e3, A.ctx->stream);
+    const int n = A.boxes[box->b].n;
+    if (A.stage(sizeof(double2) * (size_t)energy_blocks(n))) return SPH_ERR_NOMEM;
+    launch_energy_now(A.view(), box->b, n, (double2 *)A.d_stage, A.d_e3, A.ctx->stream);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(out, A.d_e3, sizeof(out), hipMemcpyDeviceToHost, A.ctx->stream));
     HIPCHK(hipStreamSynchronize(A.ctx->stream));

@@ -785,13 +785,15 @@ __global__ __launch_bounds__(NT) void k_permute(ArenaView A, int force_mask, int
 // pipelines give identical lists.  Ranks come from wave ballots and per-wave
 // counters (each wave owns one counter row and walks its slice of the box in
 // order), so there are no atomics and the result is deterministic.  1024
-// threads and 1024 cells (40 KB of LDS): the block of the largest box sets
+// threads and 1024 cells (36 KB of LDS): the block of the largest box sets
 // the kernel's time, and with 512 threads and 2048 cells it took twice as
 // long per slot; boxes of up to 16,384 slots have at most 784 cells.
 static constexpr int BS_THREADS = 1024;
 static constexpr int BS_WAVES = BS_THREADS / 64;
 static constexpr int BS_CELL_BITS = 10;
 static constexpr int BS_MAX_CELLS = 1 << BS_CELL_BITS;
+static constexpr int BS_MAX_N = 16384;
+static_assert(BS_CELL_BITS + 6 <= 16, "cell and rank share a register's low half");
 
 __device__ __forceinline__ uint64_t lanes_below()
 {
@@ -825,7 +827,7 @@ __global__ __launch_bounds__(BS_THREADS) void k_box_sort(ArenaView A, int force_
 {
     __shared__ unsigned short cnt[BS_WAVES][BS_MAX_CELLS];
     __shared__ int start[BS_MAX_CELLS + 1];
-    __shared__ int part[BS_THREADS];
+    __shared__ int part[BS_WAVES];
     const int b = blockIdx.x;
     if (b >= nbox || !building(A.dyn[b], force_mask)) return;
     const BoxDesc &B = A.boxes[b];
@@ -834,59 +836,80 @@ __global__ __launch_bounds__(BS_THREADS) void k_box_sort(ArenaView A, int force_
     for (int c = tid; c < C; c += BS_THREADS)
         for (int v = 0; v < BS_WAVES; ++v) cnt[v][c] = 0;
     __syncthreads();
-    // wave w walks slots [s0, s1) of the box, 64 at a time, in order
+    // Wave w walks slots [s0, s1) of the box, 64 at a time, in order, the
+    // positions of four groups loaded before the first is counted.  A slot's
+    // cell, its rank among the group's lanes of that cell and (on the first
+    // of them) their number go to keys_in (which only the radix sort reads
+    // otherwise) for the scatter, so each group is matched once.  (A load, its
+    // wait and a match per group and walk: 31 us of a 12,345-slot box's build,
+    // 22 now; the matches of one box on one CU bound it.)
     const int S = ((n + BS_WAVES - 1) / BS_WAVES + 63) & ~63;
     const int s0 = min(w * S, n), s1 = min(s0 + S, n);
-    for (int g = s0; g < s1; g += 64) {
-        const int i = g + lane;
-        const bool valid = i < s1;
-        const int c = valid ? cell_of(A.r[B.part_off + i], B) : 0;
-        const uint64_t m = match_cell(c, valid);
-        if (valid && (m & lanes_below()) == 0) cnt[w][c] += (unsigned short)__popcll(m);
+    const int coff = A.box_coff[b];
+    constexpr int AHEAD = 4;
+#pragma unroll 1
+    for (int g = s0; g < s1; g += 64 * AHEAD) {
+        double2 r[AHEAD];
+#pragma unroll
+        for (int q = 0; q < AHEAD; ++q) r[q] = A.r[B.part_off + min(g + q * 64 + lane, n - 1)];
+#pragma unroll
+        for (int q = 0; q < AHEAD; ++q) {
+            const int i = g + q * 64 + lane;
+            const bool valid = i < s1;
+            const int c = valid ? cell_of(r[q], B) : 0;
+            const uint64_t m = match_cell(c, valid);
+            const int rank = __popcll(m & lanes_below()), num = rank == 0 ? __popcll(m) : 0;
+            if (valid) {
+                if (num) cnt[w][c] += (unsigned short)num;
+                A.keys_in[coff + i] = (unsigned)(c | (rank << BS_CELL_BITS) | (num << 16));
+            }
+        }
     }
     __syncthreads();
     // start[c] = slots in cells below c; cnt[w][c] becomes the count of cell
-    // c in the slices of waves below w
-    const int per = (C + BS_THREADS - 1) / BS_THREADS;
-    const int c0 = min(tid * per, C), c1 = min(c0 + per, C);
-    int sum = 0;
-    for (int c = c0; c < c1; ++c)
-        for (int v = 0; v < BS_WAVES; ++v) sum += cnt[v][c];
-    part[tid] = sum;
-    __syncthreads();
-    for (int off = 1; off < BS_THREADS; off <<= 1) {  // inclusive scan
-        const int x = tid >= off ? part[tid - off] : 0;
-        __syncthreads();
-        part[tid] += x;
-        __syncthreads();
-    }
-    int run = part[tid] - sum;
-    for (int c = c0; c < c1; ++c) {
-        start[c] = run;
-        int acc = 0;
-        for (int v = 0; v < BS_WAVES; ++v) {
-            const int x = cnt[v][c];
-            cnt[v][c] = (unsigned short)acc;
-            acc += x;
+    // c in the slices of waves below w.  One cell a thread (C <= BS_THREADS):
+    // shuffle scans within the waves, then over the wave totals.
+    {
+        static_assert(BS_MAX_CELLS <= BS_THREADS, "one cell a thread");
+        int sum = 0;
+        if (tid < C)
+            for (int v = 0; v < BS_WAVES; ++v) {
+                const int x = cnt[v][tid];
+                cnt[v][tid] = (unsigned short)sum;
+                sum += x;
+            }
+        int run = sum;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int x = __shfl_up(run, off);
+            if (lane >= off) run += x;
         }
-        run += acc;
+        if (lane == 63) part[w] = run;
+        __syncthreads();
+        int below = 0;
+        for (int v = 0; v < w; ++v) below += part[v];
+        if (tid < C) start[tid] = below + run - sum;
+        if (tid == 0) start[C] = n;
     }
-    if (tid == 0) start[C] = n;
     __syncthreads();
     // stable scatter: compact positions of the sorted order
-    const int coff = A.box_coff[b];
-    for (int g = s0; g < s1; g += 64) {
-        const int i = g + lane;
-        const bool valid = i < s1;
-        const int c = valid ? cell_of(A.r[B.part_off + i], B) : 0;
-        const uint64_t m = match_cell(c, valid);
-        const int rank = __popcll(m & lanes_below());
-        if (valid) {
-            const int pos = start[c] + cnt[w][c] + rank;
-            A.vals[coff + pos] = (unsigned)(coff + i);
-            A.keys[coff + pos] = (unsigned)(B.key_base + c);
+#pragma unroll 1
+    for (int g = s0; g < s1; g += 64 * AHEAD) {
+        unsigned k[AHEAD];
+#pragma unroll
+        for (int q = 0; q < AHEAD; ++q) k[q] = A.keys_in[coff + min(g + q * 64 + lane, n - 1)];
+#pragma unroll
+        for (int q = 0; q < AHEAD; ++q) {
+            const int i = g + q * 64 + lane, c = (int)k[q] & (BS_MAX_CELLS - 1);
+            if (i < s1) {
+                const int pos = start[c] + cnt[w][c] + (int)((k[q] >> BS_CELL_BITS) & 63u);
+                A.vals[coff + pos] = (unsigned)(coff + i);
+                A.keys[coff + pos] = (unsigned)(B.key_base + c);
+                // (after the group's lanes have read their counters: one
+                // wave's LDS accesses keep their order)
+                if (k[q] >> 16) cnt[w][c] += (unsigned short)(k[q] >> 16);
+            }
         }
-        if (valid && rank == 0) cnt[w][c] += (unsigned short)__popcll(m);
     }
     for (int c = tid; c <= C; c += BS_THREADS) A.cell_start[B.key_base + c] = B.part_off + start[c];
 }
@@ -2783,33 +2806,61 @@ __global__ __launch_bounds__(NT) void k_set_u(ArenaView A, int box, const double
     A.up[s] = u;
 }
 
-// out3 = (sum m v^2/2, sum m u, total) over one box's state.
-__global__ __launch_bounds__(NT) void k_energy_now(ArenaView A, int box, double *__restrict__ out3)
+// Block sums (sum m v^2/2, sum m u) of one box's state, part[block], and from
+// them the box's totals out3 = (kinetic, thermal, sum).  A block takes 1,024
+// slots in four strided loads a thread; the second launch adds the block sums
+// in a fixed order.  (One block over the whole box read it at the rate of one
+// CU: 286 us at 262,144 slots, 1,158 us at 1,048,576.)
+static constexpr int EN_SLOTS = 4 * NT;
+
+__device__ __forceinline__ void block_sum2(double &a, double &b)
+{
+    __shared__ double wa[NT / 64], wb[NT / 64];
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+        a += __shfl_xor(a, off);
+        b += __shfl_xor(b, off);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        wa[threadIdx.x >> 6] = a;
+        wb[threadIdx.x >> 6] = b;
+    }
+    __syncthreads();
+    a = (wa[0] + wa[1]) + (wa[2] + wa[3]);
+    b = (wb[0] + wb[1]) + (wb[2] + wb[3]);
+}
+
+__global__ __launch_bounds__(NT) void k_energy_blocks(ArenaView A, int box, double2 *__restrict__ part)
 {
     const BoxDesc &B = A.boxes[box];
+    const int i0 = (int)blockIdx.x * EN_SLOTS + threadIdx.x;
     double ke = 0.0, ue = 0.0;
-    for (int i = threadIdx.x; i < B.n; i += NT) {
-        const int s = B.part_off + i;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int i = i0 + q * NT, s = B.part_off + (i < B.n ? i : 0);
         const double2 v = A.v[s];
-        const double m = A.m[s];
+        const double m = i < B.n ? A.m[s] : 0.0;
         ke += m * (0.5 * (v.x * v.x + v.y * v.y));
         ue += m * A.u[s];
     }
-    __shared__ double rk[NT], ru[NT];
-    rk[threadIdx.x] = ke;
-    ru[threadIdx.x] = ue;
-    __syncthreads();
-    for (int off = NT / 2; off > 0; off >>= 1) {
-        if (threadIdx.x < off) {
-            rk[threadIdx.x] += rk[threadIdx.x + off];
-            ru[threadIdx.x] += ru[threadIdx.x + off];
-        }
-        __syncthreads();
+    block_sum2(ke, ue);
+    if (threadIdx.x == 0) part[blockIdx.x] = make_double2(ke, ue);
+}
+
+__global__ __launch_bounds__(NT) void k_energy_total(int nblocks, const double2 *__restrict__ part,
+                                                      double *__restrict__ out3)
+{
+    double ke = 0.0, ue = 0.0;
+    for (int i = threadIdx.x; i < nblocks; i += NT) {
+        const double2 p = part[i];
+        ke += p.x;
+        ue += p.y;
     }
+    block_sum2(ke, ue);
     if (threadIdx.x == 0) {
-        out3[0] = rk[0];
-        out3[1] = ru[0];
-        out3[2] = rk[0] + ru[0];
+        out3[0] = ke;
+        out3[1] = ue;
+        out3[2] = ke + ue;
     }
 }
 
@@ -3051,7 +3102,7 @@ void launch_box_sort(const ArenaView &A, int force_mask, int nbox, hipStream_t s
 }
 // one block sorts a box: beyond ~16k slots its sequential walk outlasts the
 // radix sort (measured on the served workload, boxes up to 40k slots)
-bool box_sort_fits(int ncells, int n) { return ncells <= BS_MAX_CELLS && n <= 16384; }
+bool box_sort_fits(int ncells, int n) { return ncells <= BS_MAX_CELLS && n <= BS_MAX_N; }
 void launch_build_lists(const ArenaView &A, int force_mask, int fp32, hipStream_t st)
 {
     hipLaunchKernelGGL(k_build_lists, tile_grid(A), dim3(NT), 0, st, A, force_mask, fp32);
@@ -3193,9 +3244,12 @@ void launch_set_u(const ArenaView &A, int box, int n, const double *T, double T0
 {
     hipLaunchKernelGGL(k_set_u, grid_for(n), dim3(NT), 0, st, A, box, T, T0);
 }
-void launch_energy_now(const ArenaView &A, int box, double *out3, hipStream_t st)
+int energy_blocks(int n) { return n > 0 ? (n + EN_SLOTS - 1) / EN_SLOTS : 1; }
+void launch_energy_now(const ArenaView &A, int box, int n, double2 *part, double *out, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_energy_now, dim3(1), dim3(NT), 0, st, A, box, out3);
+    const int nb = energy_blocks(n);
+    hipLaunchKernelGGL(k_energy_blocks, dim3(nb), dim3(NT), 0, st, A, box, part);
+    hipLaunchKernelGGL(k_energy_total, dim3(1), dim3(NT), 0, st, nb, part, out);
 }
 void launch_fp32_accumulate(long long n, const double *x, int unroll, double *out2, hipStream_t st)
 {

@@ -49,7 +49,9 @@ void launch_lucy(long long np, const double *r, const double *dx, double h, int 
                  double *dwdx, hipStream_t st);
 void launch_min_image(long long np, double *dr, double Lx, double Ly, hipStream_t st);
 void launch_set_u(const ArenaView &A, int box, int n, const double *T, double T0, hipStream_t st);
-void launch_energy_now(const ArenaView &A, int box, double *out3, hipStream_t st);
+// part: energy_blocks(n) block sums of the box's n slots
+int energy_blocks(int n);
+void launch_energy_now(const ArenaView &A, int box, int n, double2 *part, double *out3, hipStream_t st);
 void launch_fp32_accumulate(long long n, const double *x, int unroll, double *out2, hipStream_t st);
 // Device scratch of a rendering of n particles (n >= 1 counts; the arrays of
 // one call, nothing in them need be cleared): SPLASH_HEAD_BYTES of head, n
