@@ -256,6 +256,15 @@ struct Arena {
     double *h_stage = nullptr;  // pinned
     size_t h_stage_bytes = 0;
 
+    // host memory the device reads directly (tables and states of admitted
+    // boxes): two halves used in turn, each waited for before it is reused
+    static constexpr size_t FEED_HALF = (size_t)4 << 20;
+    char *h_feed = nullptr, *d_feed = nullptr;
+    hipEvent_t feed_done[2] = {nullptr, nullptr};
+    bool feed_used[2] = {false, false};
+    int feed_half = 0;
+    size_t feed_at = 0;
+
     // asynchronous snapshots: state copied on the device in stream order,
     // then to the host on a copy stream
     double *d_snap = nullptr;
@@ -402,7 +411,7 @@ struct Arena {
             hipMemset(Q, 0, z2) || hipMemset(acc, 0, z2) || hipMemset(udot, 0, z1) ||
             hipMemset(gradv, 0, sizeof(double4) * cap) || hipMemset(jq, 0, z2) || hipMemset(e, 0, z1) ||
             hipMemset(r_ref, 0, z2) || hipMemset(cnt, 0, sizeof(int2) * cap) || hipMemset(vt, 0, z2) ||
-            hipMemset(aco, 0, z2) || hipMemset(uco, 0, z1))
+            hipMemset(aco, 0, z2) || hipMemset(uco, 0, z1) || hipMemset(slot_box, 0xff, sizeof(int) * cap))
             return fail(SPH_ERR_HIP, "hipMemset failed");
         // the context stream does not synchronise with the null stream
         HIPCHK(hipDeviceSynchronize());
@@ -438,6 +447,12 @@ struct Arena {
         if (h_stage) (void)hipHostFree(h_stage);
         h_stage = nullptr;
         h_stage_bytes = 0;
+        if (h_feed) (void)hipHostFree(h_feed);
+        h_feed = d_feed = nullptr;
+        for (auto &e : feed_done) {
+            if (e) (void)hipEventDestroy(e);
+            e = nullptr;
+        }
         dfree(d_inv); dfree(d_cnt); dfree(d_off); dfree(d_grand); dfree(d_jbuf); dfree(d_iap);
         if (scan_tmp) (void)hipFree(scan_tmp);
         scan_tmp = nullptr;
@@ -597,30 +612,95 @@ struct Arena {
         return SPH_OK;
     }
 
-    // Bring the device's box table up to date: the range of entries that
-    // differ from what was last sent (adding a box to an arena changes one
-    // entry; the whole table of a large arena is a slow pageable copy).
-    int send_boxes()
+    // bytes (at most FEED_HALF) of host memory that launches enqueued from now
+    // on may read
+    int feed(size_t bytes, char **h, char **d)
     {
-        size_t lo = 0, hi = boxes.size();
-        if (sent.size() == hi) {
-            while (lo < hi && memcmp(&boxes[lo], &sent[lo], sizeof(BoxDesc)) == 0) ++lo;
-            while (hi > lo && memcmp(&boxes[hi - 1], &sent[hi - 1], sizeof(BoxDesc)) == 0) --hi;
-        } else if (sent.size() < hi) {
-            while (lo < sent.size() && memcmp(&boxes[lo], &sent[lo], sizeof(BoxDesc)) == 0) ++lo;
+        bytes = align256(bytes);
+        if (bytes > FEED_HALF) return fail(SPH_ERR_ARG, "feed request too large");
+        if (!h_feed) {
+            for (auto &e : feed_done) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+            char *p = nullptr;
+            if (hipHostMalloc((void **)&p, 2 * FEED_HALF, hipHostMallocDefault) != hipSuccess)
+                return fail(SPH_ERR_NOMEM, "hipHostMalloc failed");
+            if (hipHostGetDevicePointer((void **)&d_feed, p, 0) != hipSuccess) {
+                (void)hipHostFree(p);
+                return fail(SPH_ERR_HIP, "hipHostGetDevicePointer failed");
+            }
+            h_feed = p;
         }
-        if (lo >= hi) return SPH_OK;
-        sent.clear();  // until the copy is queued
-        HIPCHK(hipMemcpyAsync(d_boxes + lo, boxes.data() + lo, sizeof(BoxDesc) * (hi - lo), hipMemcpyHostToDevice,
-                              ctx->stream));
-        sent = boxes;
+        if (feed_at + bytes > FEED_HALF) {
+            HIPCHK(hipEventRecord(feed_done[feed_half], ctx->stream));
+            feed_used[feed_half] = true;
+            feed_half ^= 1;
+            feed_at = 0;
+            if (feed_used[feed_half]) HIPCHK(hipEventSynchronize(feed_done[feed_half]));
+        }
+        const size_t at = feed_half * FEED_HALF + feed_at;
+        feed_at += bytes;
+        *h = h_feed + at;
+        *d = d_feed + at;
         return SPH_OK;
     }
 
+    // Entries [lo, hi) of the box table that differ from what was last sent
+    // (adding a box to an arena changes one of them).
+    void changed_boxes(size_t &lo, size_t &hi) const
+    {
+        lo = 0;
+        hi = boxes.size();
+        const size_t both = std::min(sent.size(), hi);
+        while (lo < both && memcmp(&boxes[lo], &sent[lo], sizeof(BoxDesc)) == 0) ++lo;
+        if (sent.size() >= hi)
+            while (hi > lo && memcmp(&boxes[hi - 1], &sent[hi - 1], sizeof(BoxDesc)) == 0) --hi;
+    }
+
+    // Bring the device's box table up to date, with all: the segment table
+    // too, with dyn_b >= 0: box dyn_b's state h_dyn[dyn_b].  One launch that
+    // reads the entries from host memory (a pageable copy per table took most
+    // of an admission); copies where they do not fit its feed.
+    int send_tables(bool all, int dyn_b)
+    {
+        size_t lo, hi;
+        changed_boxes(lo, hi);
+        const size_t nb = sizeof(BoxDesc) * (hi - lo), ns = all ? sizeof(SegDesc) * segs.size() : 0;
+        const size_t nd = dyn_b >= 0 ? sizeof(BoxDyn) : 0;
+        if (nb + ns + nd == 0) return SPH_OK;
+        sent.clear();  // until the entries are queued
+        if (align256(nb) + align256(ns) + nd <= FEED_HALF) {
+            static_assert(sizeof(BoxDesc) % 4 == 0 && sizeof(SegDesc) % 4 == 0 && sizeof(BoxDyn) % 4 == 0, "words");
+            char *h, *d;
+            if (int rc = feed(align256(nb) + align256(ns) + nd, &h, &d)) return rc;
+            PutSpans P;
+            memset(&P, 0, sizeof(P));
+            auto span = [&](int q, void *dst, const void *src, size_t at, size_t bytes) {
+                memcpy(h + at, src, bytes);
+                P.dst[q] = (unsigned *)dst;
+                P.src[q] = (const unsigned *)(d + at);
+                P.words[q] = (int)(bytes / 4);
+            };
+            if (nb) span(0, d_boxes + lo, boxes.data() + lo, 0, nb);
+            if (ns) span(1, d_segs, segs.data(), align256(nb), ns);
+            if (nd) span(2, d_dyn + dyn_b, h_dyn + dyn_b, align256(nb) + align256(ns), nd);
+            launch_put(P, ctx->stream);
+            HIPCHK(hipGetLastError());
+        } else {
+            if (nb) HIPCHK(hipMemcpyAsync(d_boxes + lo, boxes.data() + lo, nb, hipMemcpyHostToDevice, ctx->stream));
+            if (ns) HIPCHK(hipMemcpyAsync(d_segs, segs.data(), ns, hipMemcpyHostToDevice, ctx->stream));
+            if (nd) HIPCHK(hipMemcpyAsync(d_dyn + dyn_b, h_dyn + dyn_b, nd, hipMemcpyHostToDevice, ctx->stream));
+        }
+        if (nd) host_dyn_ok = false;
+        sent = boxes;
+        return SPH_OK;
+    }
+    int send_boxes() { return send_tables(false, -1); }
+
     // Recompute key bases in slot order, the high-water mark, and upload the
-    // box and segment tables.  own_terms false: a box's terms are those of one
-    // evaluation, not of its steps (sph_rates).
-    int relayout(bool own_terms = true)
+    // box and segment tables (and box dyn_b's state, when given).  own_terms
+    // false: a box's terms are those of one evaluation, not of its steps
+    // (sph_rates).  Slot owners are set where slots change hands (add_box,
+    // remove_box).
+    int relayout(bool own_terms = true, int dyn_b = -1, const BoxDyn *D = nullptr)
     {
         int key = 0;
         hwm = 0;
@@ -665,12 +745,8 @@ struct Arena {
             invalidate_graph();
         }
         if (ensure_tables((int)boxes.size())) return SPH_ERR_NOMEM;
-        if (int rc = send_boxes()) return rc;
-        HIPCHK(hipMemcpyAsync(d_segs, segs.data(), sizeof(SegDesc) * segs.size(), hipMemcpyHostToDevice,
-                              ctx->stream));
-        launch_slot_box(view(), ctx->stream);
-        // copies from pageable host memory are staged before hipMemcpyAsync
-        // returns, so the tables may change right away; no wait
+        if (D) h_dyn[dyn_b] = *D;
+        if (int rc = send_tables(true, dyn_b)) return rc;
         // the slot count, key count and segment count are baked into
         // captured launches
         check_graph_sig();
@@ -1071,7 +1147,8 @@ struct Arena {
     }
 
     // ---- boxes -------------------------------------------------------------
-    int add_box(int64_t n, const sph_params *prm, int *box_out);
+    int add_box(int64_t n, const sph_params *prm, int *box_out, const BoxDyn &D, double T0 = 0.0,
+                const double *r = nullptr, const double *v = nullptr, const double *m = nullptr);
     int remove_box(int b);
     int upload(int b, int field, const double *host, int ncomp);
     int download(int b, int field, double *host, int ncomp);
@@ -1149,13 +1226,27 @@ int list_entries_for(const sph_params *p, int64_t n)
     return std::max(64, std::min(l, 4096));
 }
 
-int Arena::add_box(int64_t n, const sph_params *prm, int *box_out)
+// The common mass of m[0 .. n) when all are equal, positive and finite, else 0
+// (the passes then skip the per-neighbour mass fetch).
+double common_mass(const double *m, int64_t n)
+{
+    bool uni = n > 0 && m[0] > 0.0 && std::isfinite(m[0]);
+    for (int64_t i = 1; uni && i < n; ++i) uni = m[i] == m[0];
+    return uni ? m[0] : 0.0;
+}
+
+// A new box of n particles in state D at initial temperature T0; r, v, m
+// (all or none) its particles' state.
+int Arena::add_box(int64_t n, const sph_params *prm, int *box_out, const BoxDyn &D, double T0, const double *r,
+                   const double *v, const double *m)
 {
     if (n <= 0 || n > cap) return fail(SPH_ERR_ARG, "box size out of range");
     BoxDesc B;
     if (int rc = fill_desc(prm, n, B)) return rc;
     if (prm->precision != precision) return fail(SPH_ERR_ARG, "box precision differs from the arena's");
     B.build16 = list_bits == 16 ? 1 : 0;
+    B.T0 = T0;
+    if (m) B.munif = common_mass(m, n);
     {
         // mean neighbours within r_cut + skin at the box's number density:
         // a box whose mean alone takes over half the list entries is refused
@@ -1190,12 +1281,24 @@ int Arena::add_box(int64_t n, const sph_params *prm, int *box_out)
     if (fs.len > n) ns.push_back(SegDesc{fs.off + (int)n, fs.len - (int)n, -1, 0});
     ns.insert(ns.end(), segs.begin() + si + 1, segs.end());
     segs.swap(ns);
-    if (int rc = relayout()) return rc;
-    BoxDyn D;
-    memset(&D, 0, sizeof(D));
-    D.state = BOX_DONE;
-    if (int rc = write_dyn(b, D)) return rc;
-    launch_init_slots(view(), boxes[b].part_off, (int)n, ctx->stream);
+    if (int rc = relayout(true, b, &D)) return rc;
+    const int off = boxes[b].part_off;
+    if (!r) {
+        launch_assign_slots(view(), off, (int)n, b, 0, nullptr, ctx->stream);
+    } else {
+        // the particles' state through the feed, in pieces that fit half of it
+        const int64_t most = (int64_t)(FEED_HALF / 2 / (5 * sizeof(double)));
+        for (int64_t i = 0; i < n; i += most) {
+            const size_t k = (size_t)std::min(most, n - i);
+            char *h, *d;
+            if (int rc = feed(5 * sizeof(double) * k, &h, &d)) return rc;
+            double *p = (double *)h;
+            memcpy(p, r + 2 * i, sizeof(double) * 2 * k);
+            memcpy(p + 2 * k, v + 2 * i, sizeof(double) * 2 * k);
+            memcpy(p + 4 * k, m + i, sizeof(double) * k);
+            launch_assign_slots(view(), off + (int)i, (int)k, b, (int)i, (const double *)d, ctx->stream);
+        }
+    }
     HIPCHK(hipGetLastError());
     *box_out = b;
     return SPH_OK;
@@ -1204,6 +1307,9 @@ int Arena::add_box(int64_t n, const sph_params *prm, int *box_out)
 int Arena::remove_box(int b)
 {
     if (b < 0 || b >= (int)boxes.size() || !box_live[b]) return fail(SPH_ERR_ARG, "no such box");
+    // (the view of the layout the box lies in: its slots are in use)
+    launch_assign_slots(view(), boxes[b].part_off, boxes[b].n, -1, 0, nullptr, ctx->stream);
+    HIPCHK(hipGetLastError());
     for (auto &sg : segs)
         if (sg.box == b) sg.box = -1;
     // merge adjacent free segments
@@ -1218,8 +1324,7 @@ int Arena::remove_box(int b)
     BoxDyn D;
     memset(&D, 0, sizeof(D));
     D.state = BOX_FREE;
-    if (int rc = write_dyn(b, D)) return rc;
-    return relayout();
+    return relayout(true, b, &D);
 }
 
 int Arena::upload(int b, int field, const double *host, int ncomp)
@@ -1234,9 +1339,7 @@ int Arena::upload(int b, int field, const double *host, int ncomp)
     if (field == 2) {
         // equal masses (every configuration of the reference's drivers):
         // the density pass then skips the per-neighbour mass fetch
-        bool uni = n > 0 && host[0] > 0.0 && std::isfinite(host[0]);
-        for (int i = 1; uni && i < n; ++i) uni = host[i] == host[0];
-        boxes[b].munif = uni ? host[0] : 0.0;
+        boxes[b].munif = common_mass(host, n);
         if (int rc = send_boxes()) return rc;
     }
     // the pageable source is staged before the copy call returns and the
@@ -1359,7 +1462,10 @@ int sph_box_create(sph_ctx *ctx, int64_t n, const sph_params *prm, sph_box **out
     bx->ar.keep_host_dyn = true;
     bx->prm = *prm;
     int rc = bx->ar.alloc((int)n, prm->precision, list_entries_for(prm, n));
-    if (!rc) rc = bx->ar.add_box(n, prm, &bx->b);
+    BoxDyn D;
+    memset(&D, 0, sizeof(D));
+    D.state = BOX_DONE;
+    if (!rc) rc = bx->ar.add_box(n, prm, &bx->b, D);
     if (!rc) rc = bx->ar.prepare_graphs();  // no capture inside a later sph_step
     if (rc) {
         std::string keep = g_err;
@@ -1440,9 +1546,38 @@ int sph_box_download(sph_box *box, double *r, double *v, double *u, double *rho,
     struct F { double *dst; int field, nc; } fs[] = {
         {r, 0, 2}, {v, 1, 2}, {u, 3, 1}, {rho, 4, 1}, {rho_lr, 5, 1}, {T, 6, 1}, {p, 7, 1},
         {pco, 8, 1}, {acc, 9, 2}, {udot, 10, 1}, {gradv, 11, 4}, {jq, 12, 2}, {P, 13, 4}};
+    // the fields together through pinned memory: one copy and one wait (each
+    // field's own pageable copy and wait: 1.6 ms of nine fields of 65,536
+    // particles); fields past DOWNLOAD_PINNED bytes one by one
+    Arena &A = box->ar;
+    const size_t n = (size_t)A.boxes[box->b].n;
+    size_t total = 0;
+    for (auto &f : fs)
+        if (f.dst) total += sizeof(double) * n * f.nc;
+    static constexpr size_t DOWNLOAD_PINNED = (size_t)16 << 20;
+    if (total <= DOWNLOAD_PINNED) {
+        if (A.stage(total) || A.host_stage(total)) return SPH_ERR_NOMEM;
+        const ArenaView V = A.view();
+        size_t at = 0;
+        for (auto &f : fs)
+            if (f.dst) {
+                launch_download(V, box->b, (int)n, f.field, A.d_stage + at, A.ctx->stream);
+                at += n * f.nc;
+            }
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(A.h_stage, A.d_stage, total, hipMemcpyDeviceToHost, A.ctx->stream));
+        HIPCHK(hipStreamSynchronize(A.ctx->stream));
+        at = 0;
+        for (auto &f : fs)
+            if (f.dst) {
+                memcpy(f.dst, A.h_stage + at, sizeof(double) * n * f.nc);
+                at += n * f.nc;
+            }
+        return SPH_OK;
+    }
     for (auto &f : fs)
         if (f.dst)
-            if (int rc = box->ar.download(box->b, f.field, f.dst, f.nc)) return rc;
+            if (int rc = A.download(box->b, f.field, f.dst, f.nc)) return rc;
     return SPH_OK;
 }
 
@@ -1459,10 +1594,10 @@ int sph_nlist_build(sph_box *box, int64_t cap, int64_t *iap, int64_t *nip_out)
     A.sched_kept = false;  // lists rebuilt outside a run's schedule
     A.mark(T_PAIRS, true);
     if (int rc = A.build_now(MASK_ALL)) return rc;
-    if (!A.d_inv) {
-        if (dalloc(&A.d_inv, A.cap) || dalloc(&A.d_cnt, A.cap) || dalloc(&A.d_off, A.cap) ||
-            dalloc(&A.d_grand, 1))
-            return SPH_ERR_NOMEM;
+    if (!A.d_inv && dalloc(&A.d_inv, A.cap)) return SPH_ERR_NOMEM;
+    if (!A.scan_tmp) {  // d_inv may be there from a separations call
+        dfree(A.d_cnt); dfree(A.d_off); dfree(A.d_grand);
+        if (dalloc(&A.d_cnt, A.cap) || dalloc(&A.d_off, A.cap) || dalloc(&A.d_grand, 1)) return SPH_ERR_NOMEM;
         A.scan_tmp_bytes = exscan_temp_bytes(A.cap);
         if (dalloc((char **)&A.scan_tmp, A.scan_tmp_bytes)) return SPH_ERR_NOMEM;
     }
@@ -1890,20 +2025,12 @@ int sph_arena_add(sph_arena *ar, int64_t n, const sph_params *prm, const double 
         if (!(x >= 0.0 && x < prm->Lx && y >= 0.0 && y < prm->Ly))
             return fail(SPH_ERR_ARG, "position outside [0, L)");
     }
-    int b = -1;
-    if (int rc = A.add_box(n, prm, &b)) return rc;
-    A.boxes[b].T0 = T0;
-    if (int rc = A.send_boxes()) return rc;
-    if (int rc = A.upload(b, 0, r, 2)) return rc;
-    if (int rc = A.upload(b, 1, v, 2)) return rc;
-    if (int rc = A.upload(b, 2, m, 1)) return rc;
     BoxDyn D;
     memset(&D, 0, sizeof(D));
     D.state = BOX_INIT;
     D.nsteps = nsteps;
-    if (int rc = A.write_dyn(b, D)) return rc;
-    *box_id = b;
-    return SPH_OK;
+    A.sched_kept = false;
+    return A.add_box(n, prm, box_id, D, T0, r, v, m);
 }
 
 int sph_arena_step(sph_arena *ar, int64_t nsteps)
@@ -1948,21 +2075,21 @@ int sph_arena_result(sph_arena *ar, int box_id, double *r, double *v, double *u,
     Arena &A = ar->ar;
     if (box_id < 0 || box_id >= (int)A.boxes.size() || !A.box_live[box_id]) return fail(SPH_ERR_ARG, "no such box");
     HIPCHK(hipSetDevice(A.ctx->device));
-    // r, v, u, rho packed into the device staging buffer, one copy to pinned
-    // host memory and one wait (with the box states) for the four fields
+    // r, v, u, rho and the box states written to pinned host memory by the
+    // device itself, one wait for all
     const int n = A.boxes[box_id].n;
     const size_t nd = (size_t)n;
-    if (A.stage(sizeof(double) * 6 * nd)) return SPH_ERR_NOMEM;
-    if (A.host_stage(sizeof(double) * 6 * nd)) return SPH_ERR_NOMEM;
-    double *d = A.d_stage;
-    const ArenaView V = A.view();
-    launch_download(V, box_id, n, 0, d, A.ctx->stream);
-    launch_download(V, box_id, n, 1, d + 2 * nd, A.ctx->stream);
-    launch_download(V, box_id, n, 3, d + 4 * nd, A.ctx->stream);
-    launch_download(V, box_id, n, 4, d + 5 * nd, A.ctx->stream);
+    const size_t dyn_bytes = sizeof(BoxDyn) * A.boxes.size();
+    if (A.host_stage(sizeof(double) * 6 * nd + dyn_bytes)) return SPH_ERR_NOMEM;
+    if (!A.d_inv && dalloc(&A.d_inv, A.cap)) return SPH_ERR_NOMEM;
+    double *dst = nullptr;
+    HIPCHK(hipHostGetDevicePointer((void **)&dst, A.h_stage, 0));
+    launch_inverse(A.id, A.boxes[box_id].part_off, n, A.d_inv, A.ctx->stream);
+    launch_fetch(A.view(), n, A.d_inv, dst, (int)(dyn_bytes / 4), A.ctx->stream);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(A.h_stage, d, sizeof(double) * 6 * nd, hipMemcpyDeviceToHost, A.ctx->stream));
-    if (int rc = A.read_dyn()) return rc;  // waits for the copy above too
+    HIPCHK(hipStreamSynchronize(A.ctx->stream));
+    memcpy((void *)A.h_dyn, A.h_stage + 6 * nd, dyn_bytes);
+    if (int rc = A.release_held()) return rc;
     const double *h = A.h_stage;
     if (r) memcpy(r, h, sizeof(double) * 2 * nd);
     if (v) memcpy(v, h + 2 * nd, sizeof(double) * 2 * nd);

@@ -666,20 +666,6 @@ __device__ __forceinline__ int building_box(const ArenaView &A, int s, int force
     return (b >= 0 && building(A.dyn[b], force_mask)) ? b : -1;
 }
 
-// Slot owners, written when the layout changes (free slots: -1).
-__global__ __launch_bounds__(NT) void k_slot_box(ArenaView A)
-{
-    const int s = blockIdx.x * NT + threadIdx.x;
-    if (s >= A.n) return;
-    int lo = 0, hi = A.nseg - 1;
-    while (lo < hi) {  // last segment with off <= s
-        const int mid = (lo + hi + 1) >> 1;
-        if (A.segs[mid].off <= s) lo = mid;
-        else hi = mid - 1;
-    }
-    A.slot_box[s] = A.segs[lo].box;
-}
-
 // key = box key base + current cell (row major) at the slot's compact
 // position.
 // The build kernels run over the building tiles of the plan
@@ -2606,14 +2592,54 @@ __global__ __launch_bounds__(NT) void k_upload(ArenaView A, int off, int n, int 
     }
 }
 
-__global__ __launch_bounds__(NT) void k_init_slots(ArenaView A, int off, int n)
+// Slots [off, off + n) become box b's (-1: free), in caller order; with src
+// (r[n][2], v[n][2], m[n] of the caller's particles i0 on, in memory the
+// device reads directly) they also take that state.
+__global__ __launch_bounds__(NT) void k_assign_slots(ArenaView A, int off, int n, int b, int i0,
+                                                      const double *__restrict__ src)
 {
     const int i = blockIdx.x * NT + threadIdx.x;
     if (i >= n) return;
     const int s = off + i;
-    A.id[s] = i;
+    A.slot_box[s] = b;
+    if (b < 0) return;
+    A.id[s] = i0 + i;
     A.acc[s] = make_double2(0.0, 0.0);
     A.udot[s] = 0.0;
+    if (!src) return;
+    const double2 *r = (const double2 *)src, *v = r + n;
+    const double *m = (const double *)(v + n);
+    A.r[s] = r[i];
+    const double2 vi = v[i];
+    A.v[s] = vi;
+    A.vp[s] = vi;
+    A.m[s] = m[i];
+}
+
+// Copies up to three spans of words (the changed table entries of a relayout).
+__global__ __launch_bounds__(NT) void k_put(PutSpans P)
+{
+    for (int q = 0; q < 3; ++q)
+        for (int w = blockIdx.x * NT + threadIdx.x; w < P.words[q]; w += gridDim.x * NT) P.dst[q][w] = P.src[q][w];
+}
+
+// One box's r, v, u, rho in caller order (inv: slot of a caller index), one
+// after the other in dst, then the words of all box states: dst is host
+// memory, written in order (a copy per field and one of the states, each a
+// launch and a wait of its own, took 65 us a box).
+__global__ __launch_bounds__(NT) void k_fetch(ArenaView A, int n, const int *__restrict__ inv, double *__restrict__ dst,
+                                               int dyn_words)
+{
+    const int k = blockIdx.x * NT + threadIdx.x;
+    if (k < n) {
+        const int s = inv[k];
+        ((double2 *)dst)[k] = A.r[s];
+        ((double2 *)dst)[n + k] = A.v[s];
+        dst[4 * (size_t)n + k] = A.u[s];
+        dst[5 * (size_t)n + k] = A.rho[s].x;
+    }
+    unsigned *d = (unsigned *)(dst + 6 * (size_t)n);
+    for (int w = k; w < dyn_words; w += gridDim.x * NT) d[w] = ((const unsigned *)A.dyn)[w];
 }
 
 __global__ __launch_bounds__(NT) void k_download(ArenaView A, int box, int field,
@@ -3071,10 +3097,6 @@ static inline int pass_block_of(const ArenaView &A)
     return (A.pass_block == 128 || A.pass_block == 512) ? A.pass_block : NT;
 }
 
-void launch_slot_box(const ArenaView &A, hipStream_t st)
-{
-    if (A.n > 0) hipLaunchKernelGGL(k_slot_box, grid_for(A.n), dim3(NT), 0, st, A);
-}
 void launch_build_plan(const ArenaView &A, int force_mask, hipStream_t st)
 {
     hipLaunchKernelGGL(k_build_plan, dim3(1), dim3(PLAN_THREADS), 0, st, A, force_mask);
@@ -3181,9 +3203,20 @@ void launch_upload(const ArenaView &A, int off, int n, int field, const double *
 {
     hipLaunchKernelGGL(k_upload, grid_for(n), dim3(NT), 0, st, A, off, n, field, src);
 }
-void launch_init_slots(const ArenaView &A, int off, int n, hipStream_t st)
+void launch_assign_slots(const ArenaView &A, int off, int n, int b, int i0, const double *src, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_init_slots, grid_for(n), dim3(NT), 0, st, A, off, n);
+    if (n > 0) hipLaunchKernelGGL(k_assign_slots, grid_for(n), dim3(NT), 0, st, A, off, n, b, i0, src);
+}
+void launch_put(const PutSpans &P, hipStream_t st)
+{
+    int most = 0;
+    for (int q = 0; q < 3; ++q) most = P.words[q] > most ? P.words[q] : most;
+    const int nb = (most + NT - 1) / NT;
+    if (most > 0) hipLaunchKernelGGL(k_put, dim3(nb < 64 ? nb : 64), dim3(NT), 0, st, P);
+}
+void launch_fetch(const ArenaView &A, int n, const int *inv, double *dst, int dyn_words, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_fetch, grid_for(n), dim3(NT), 0, st, A, n, inv, dst, dyn_words);
 }
 void launch_download(const ArenaView &A, int box, int n, int field, double *dst, hipStream_t st)
 {

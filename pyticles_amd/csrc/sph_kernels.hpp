@@ -11,9 +11,8 @@ constexpr int MASK_RUN = (1 << BOX_RUN);
 constexpr int MASK_INIT = (1 << BOX_INIT);
 constexpr int MASK_ALL = (1 << BOX_INIT) | (1 << BOX_RUN) | (1 << BOX_DONE);
 
-// build stage: slot owners (on a layout change), then plan, keys, sort,
-// permutation, cell starts and lists of the building boxes
-void launch_slot_box(const ArenaView &A, hipStream_t st);
+// build stage: plan, keys, sort, permutation, cell starts and lists of the
+// building boxes
 void launch_build_plan(const ArenaView &A, int force_mask, hipStream_t st);
 void launch_keys(const ArenaView &A, int force_mask, hipStream_t st);
 // cells != 0: also the cell starts from the sorted keys (radix-sort path)
@@ -35,7 +34,16 @@ void launch_rates(const ArenaView &A, int fp32, int state_mask, int unroll, int 
 void launch_leapfrog(const ArenaView &A, int fp32, hipStream_t st);
 void launch_box_step(const ArenaView &A, int nbox, hipStream_t st);
 void launch_upload(const ArenaView &A, int off, int n, int field, const double *src, hipStream_t st);
-void launch_init_slots(const ArenaView &A, int off, int n, hipStream_t st);
+// slots [off, off + n) to box b (-1: free); src: host-mapped r, v, m of the
+// caller's particles i0 .. i0 + n - 1, or null
+void launch_assign_slots(const ArenaView &A, int off, int n, int b, int i0, const double *src, hipStream_t st);
+struct PutSpans {
+    unsigned *dst[3];
+    const unsigned *src[3];
+    int words[3];
+};
+void launch_put(const PutSpans &P, hipStream_t st);
+void launch_fetch(const ArenaView &A, int n, const int *inv, double *dst, int dyn_words, hipStream_t st);
 void launch_download(const ArenaView &A, int box, int n, int field, double *dst, hipStream_t st);
 void launch_inverse(const int *ids, int off, int n, int *inv, hipStream_t st);
 void launch_pairs(const ArenaView &A, int box, int n, const int *inv, unsigned *count,

@@ -4,6 +4,7 @@ A Box owns one periodic 2-D system in HBM.  Every method is a C-ABI call
 into libpyticles_hip.so; host arrays are copied in and out only when asked.
 """
 import ctypes
+import math
 
 import numpy as np
 
@@ -186,7 +187,13 @@ class DeviceBox:
     def pairs(self, cap=None):
         """Every unordered pair (i<j) with rsq < rc^2 + tol^2, lexicographic."""
         if cap is None:
-            cap = max(64, 16 * self.n)
+            # a fifth over the mean count at the box's density, so that the
+            # first call seldom comes back for more (its search is then done
+            # twice); at least 16 a particle
+            p = self.prm
+            mean = 0.5 * math.pi * (p["rc"] ** 2 + p["tol"] ** 2) * self.n / (p["Lx"] * p["Ly"])
+            most = 0.5 * (self.n - 1)
+            cap = max(64, int(self.n * min(max(16.0, 1.2 * mean + 4.0), max(16.0, most))))
         while True:
             iap = np.empty((cap, 2), dtype=np.int64)
             nip = ctypes.c_int64()
@@ -195,7 +202,9 @@ class DeviceBox:
                 cap = int(nip.value)
                 continue
             _lib.check(rc)
-            return iap[: nip.value].copy()
+            # most of the rows are used: no second array for the few that are not
+            k = int(nip.value)
+            return iap[:k] if 3 * k >= 2 * cap else iap[:k].copy()
 
     def separations(self, iap):
         iap = np.ascontiguousarray(iap, dtype=np.int64)
