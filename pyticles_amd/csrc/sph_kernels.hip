@@ -936,6 +936,17 @@ __global__ __launch_bounds__(BS_THREADS) void k_box_sort(ArenaView A, int force_
 // slots never overflows while its cells hold fewer than (65,536 - n) / 2
 // slots each.  The candidate loop adds one constant per entry, as the
 // 32-bit form stores the slot itself.
+__device__ __forceinline__ int cell_base16(int s, int nb, int t0, int t1, bool &wrapped, bool &over)
+{
+    if (t1 <= t0) return 0;
+    const int dlo = t0 - s, dhi = t1 - 1 - s, dm = (dlo + dhi) >> 1;
+    int k = 0;  // the plain offsets when they fit, else the nearest modulo n
+    if (dlo < -32768 || dhi > 32767) k = 2 * dm > nb ? -nb : (2 * dm < -nb ? nb : 0);
+    if (dlo + k < -32768 || dhi + k > 32767) over = true;
+    if (k) wrapped = true;
+    return k - s;
+}
+
 template <bool SINGLE, bool L16>
 __device__ __forceinline__ void list_walk(const ArenaView &A, const BoxDesc &Bu, int s, double2 ri, int cell,
                                           unsigned *buf, int &ns, int &nl, bool &lost, bool &wrapped, bool &over)
@@ -957,19 +968,7 @@ __device__ __forceinline__ void list_walk(const ArenaView &A, const BoxDesc &Bu,
         else *(uint4 *)(list_base(A, s) + (size_t)q * LIST_ROW) = g;
     };
     auto ring = [&](int w0) { return make_uint4(buf[w0 * NT], buf[(w0 + 1) * NT], buf[(w0 + 2) * NT], buf[(w0 + 3) * NT]); };
-    // 16-bit base of the cell's candidates (0 in the 32-bit form)
-    auto base16 = [&](int t0, int t1) {
-        int ks = 0;
-        if (L16 && t1 > t0) {
-            const int dlo = t0 - s, dhi = t1 - 1 - s, dm = (dlo + dhi) >> 1;
-            int k = 0;  // the plain offsets when they fit, else the nearest modulo n
-            if (dlo < -32768 || dhi > 32767) k = 2 * dm > nb ? -nb : (2 * dm < -nb ? nb : 0);
-            if (dlo + k < -32768 || dhi + k > 32767) over = true;
-            if (k) wrapped = true;
-            ks = k - s;
-        }
-        return ks;
-    };
+    auto base16 = [&](int t0, int t1) { return L16 ? cell_base16(s, nb, t0, t1, wrapped, over) : 0; };
     // candidates t0 .. t1 - 1 at image offset (rx, ry) from r_i
     auto scan = [&](int t0, int t1, double rx, double ry, int ks) {
         for (int t = t0; t < t1; t += 4) {
@@ -1055,6 +1054,25 @@ __device__ __forceinline__ void list_walk(const ArenaView &A, const BoxDesc &Bu,
     }
 }
 
+// The sorted state of a building slot back into the state arrays, its build
+// position and FP32C record.
+template <class Box>
+__device__ __forceinline__ void take_sorted(const ArenaView &A, int s, const Box &B, int fp32, double2 ri, double2 vpi,
+                                            double2 ai)
+{
+    A.r[s] = ri;
+    A.v[s] = A.v_s[s];
+    A.vp[s] = vpi;
+    A.acc[s] = ai;
+    A.u[s] = A.u_s[s];
+    A.m[s] = A.m_s[s];
+    A.up[s] = A.up_s[s];
+    A.udot[s] = A.udot_s[s];
+    A.id[s] = A.id_s[s];
+    A.r_ref[s] = ri;
+    if (fp32) fix_rec(ri, vpi, B, A.rf[s], A.rlo[s]);
+}
+
 // Neighbour list of a building slot: every other slot of the 3x3 cell
 // stencil with r^2 < (r_cut + skin)^2, short entries (r^2 < (h + skin)^2)
 // from the front, the rest from the back.  The sorted state is copied back
@@ -1077,19 +1095,8 @@ __device__ __forceinline__ int build_slot(const ArenaView &A, int s, int force_m
     const BoxDesc &B = A.boxes[b];
     const double2 ri = A.r_s[s];
     const double2 vpi = A.vp_s[s], ai = A.acc_s[s];
-    const double mi = A.m_s[s];
-    A.r[s] = ri;
-    A.v[s] = A.v_s[s];
-    A.vp[s] = vpi;
-    A.acc[s] = ai;
-    A.u[s] = A.u_s[s];
-    A.m[s] = mi;
-    A.up[s] = A.up_s[s];
-    A.udot[s] = A.udot_s[s];
-    A.id[s] = A.id_s[s];
-    A.r_ref[s] = ri;
+    take_sorted(A, s, B, fp32, ri, vpi, ai);
     const int cell = A.pcell[s];
-    if (fp32) fix_rec(ri, vpi, B, A.rf[s], A.rlo[s]);
     int ns = 0, nl = 0;
     bool lost = false, wrapped = false, over = false;
     // Box constants wave-uniform (scalar registers); each stencil cell's
@@ -1116,6 +1123,138 @@ __device__ __forceinline__ int build_slot(const ArenaView &A, int s, int force_m
     v2 = vpi.x * vpi.x + vpi.y * vpi.y;
     a2 = ai.x * ai.x + ai.y * ai.y;
     return b;
+}
+
+// The same list by four lanes of a slot (sub 0 .. 3), for launches of few
+// waves: list_walk's serial chain of ~47 rounds at ~1,800 cycles each (one
+// wave a SIMD issues a dependent instruction every ~10 cycles) sets their
+// time, 36 us at 1,024 slots as at 65,536.  The lanes take the stencil's cells
+// in consecutive shares (3, 2, 2, 2 of nine).  A lane first tests its
+// candidates into bit masks, one short and one long a cell; the lanes' counts
+// then place its entries behind those of the lanes before it, so the entries
+// and their order are list_walk's, and every entry is stored to its place by
+// itself.  (With the chip full the scattered stores and the shares' spread
+// cost more than the chain.)  A cell of more than 64 slots (SERIAL, the slot's
+// first lane alone) takes neither masks nor shares.
+template <bool L16>
+__device__ __forceinline__ void list_shared(const ArenaView &A, const CBox &B, int s, int sub, double2 ri, int cell,
+                                            int &ns, int &nl, bool &lost, bool &wrapped, bool &over)
+{
+    const int lcap = A.lcap;
+    const double rnl2 = B.rnl2, hsk2 = B.hsk2, Lx = B.Lx, Ly = B.Ly, hLx = B.hLx, hLy = B.hLy;
+    const int ncx = B.ncx, ncy = B.ncy, sx = B.sx, sy = B.sy, nb = B.n;
+    const int *cs = A.cell_start + B.key_base;
+    const int cx = cell % ncx, cy = cell / ncx, wx = 2 * sx + 1, nq = wx * (2 * sy + 1);
+    const int q0 = nq == 9 ? (sub ? 2 * sub + 1 : 0) : min(sub, nq), q1 = nq == 9 ? 2 * sub + 3 : min(sub + 1, nq);
+    double rx, ry;  // r_i at the cell's image
+    auto cell_at = [&](int q, int &t0, int &t1) {
+        const int oy = q / wx, yr = cy + oy - sy, xr = cx + (q - oy * wx) - sx;
+        const int yy = yr < 0 ? yr + ncy : (yr >= ncy ? yr - ncy : yr);
+        const int xx = xr < 0 ? xr + ncx : (xr >= ncx ? xr - ncx : xr);
+        ry = ri.y - (yr < 0 ? -Ly : (yr >= ncy ? Ly : 0.0));
+        rx = ri.x - (xr < 0 ? -Lx : (xr >= ncx ? Lx : 0.0));
+        t0 = cs[yy * ncx + xx];
+        t1 = cs[yy * ncx + xx + 1];
+    };
+    auto dist2 = [&](double2 rj) {
+        double dx = rj.x - rx, dy = rj.y - ry;
+        if (sx == 0) {
+            dx = dx > hLx ? dx - Lx : dx;
+            dx = dx < -hLx ? dx + Lx : dx;
+        }
+        if (sy == 0) {
+            dy = dy > hLy ? dy - Ly : dy;
+            dy = dy < -hLy ? dy + Ly : dy;
+        }
+        return rsq_exact(dx, dy);
+    };
+    auto put = [&](int P, int t, int ks) {
+        if (L16) list_base16(A, s)[pos16(P)] = (unsigned short)(t + ks);
+        else list_base(A, s)[(size_t)(P / LIST_GROUP) * LIST_ROW + P % LIST_GROUP] = (unsigned)t;
+    };
+    auto base = [&](int t0, int t1) { return L16 ? cell_base16(s, nb, t0, t1, wrapped, over) : 0; };
+    uint64_t ms[3], ml[3];
+    int tb[3], kb[3], a = 0, l = 0;
+    bool big = false;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        ms[j] = ml[j] = 0;
+        tb[j] = kb[j] = 0;
+        if (q0 + j < q1) {
+            int t0, t1;
+            cell_at(q0 + j, t0, t1);
+            tb[j] = t0;
+            kb[j] = base(t0, t1);
+            big = big || t1 - t0 > 64;
+            const int te = min(t1, t0 + 64);
+            for (int t = t0; t < te; t += 4) {
+                double2 rj[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) rj[u] = at32(A.r_s, min(t + u, te - 1));
+                unsigned bs = 0, bl = 0;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const double r2 = dist2(rj[u]);
+                    const unsigned take = (unsigned)((int)(t + u < te) & (int)(r2 < rnl2) & (int)(t + u != s));
+                    const unsigned sh = (unsigned)(r2 < hsk2);
+                    bs |= (take & sh) << u;
+                    bl |= (take & (sh ^ 1u)) << u;
+                }
+                ms[j] |= (uint64_t)bs << (t - t0);
+                ml[j] |= (uint64_t)bl << (t - t0);
+            }
+            a += __popcll(ms[j]);
+            l += __popcll(ml[j]);
+        }
+    }
+    // flags of the four lanes, then their counts before this lane's
+    int fl = (wrapped ? 1 : 0) | (over ? 2 : 0) | (big ? 4 : 0);
+    fl |= __shfl_xor(fl, 1);
+    fl |= __shfl_xor(fl, 2);
+    wrapped = fl & 1;
+    over = (fl & 2) != 0;
+    if (fl & 4) {
+        ns = nl = 0;
+        if (sub == 0) {
+            for (int q = 0; q < nq; ++q) {
+                int t0, t1;
+                cell_at(q, t0, t1);
+                const int ks = base(t0, t1);
+                for (int t = t0; t < t1; ++t) {
+                    const double r2 = dist2(at32(A.r_s, t));
+                    if (!(r2 < rnl2) || t == s) continue;
+                    if (ns + nl >= lcap) {
+                        lost = true;
+                        break;
+                    }
+                    if (r2 < hsk2) put(ns++, t, ks);
+                    else put(lcap - 1 - nl++, t, ks);
+                }
+            }
+            if (lost) ns = nl = 0;
+        }
+        return;
+    }
+    int pa = 0, pl = 0;
+    ns = nl = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int x = lane_bcast<4>(a, i), y = lane_bcast<4>(l, i);
+        pa += i < sub ? x : 0;
+        pl += i < sub ? y : 0;
+        ns += x;
+        nl += y;
+    }
+    if (ns + nl > lcap) {
+        lost = true;
+        ns = nl = 0;
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        for (uint64_t m = ms[j]; m; m &= m - 1) put(pa++, tb[j] + __ffsll((long long)m) - 1, kb[j]);
+        for (uint64_t m = ml[j]; m; m &= m - 1) put(lcap - 1 - pl++, tb[j] + __ffsll((long long)m) - 1, kb[j]);
+    }
 }
 
 // The build's largest squared speed and acceleration per box, as step_tail
@@ -1171,6 +1310,50 @@ __global__ __launch_bounds__(NT) void k_build_lists(ArenaView A, int force_mask,
         const int b = build_slot(A, s, force_mask, fp32, lbuf + threadIdx.x, v2, a2);
         build_tail(A, s, b, v2, a2);
     });
+}
+
+// The shared form: one block per building tile, four lanes a slot; the first
+// wave takes the tile's maxima (build_tail) with a lane a slot.
+__global__ __launch_bounds__(NT) void k_build_shared(ArenaView A, int force_mask, int fp32)
+{
+    __shared__ double x2[2][64];
+    const int x = blockIdx.x & 7, local = blockIdx.x >> 3;
+    const int nbx = ((int)gridDim.x - x + 7) >> 3;  // blocks on this XCD (for_building_tiles)
+    const int T = A.plan_n[2];
+    const int k0 = (int)(((long long)T * x) >> 3), k1 = (int)(((long long)T * (x + 1)) >> 3);
+    const int sub = threadIdx.x & 3, i = threadIdx.x >> 2;
+    for (int k = k0 + local; k < k1; k += nbx) {
+        const int s0 = A.tile_list[k] * 64, s = s0 + i;
+        const int b = s < A.n ? building_box(A, s, force_mask) : -1;
+        double v2 = 0.0, a2 = 0.0;
+        per_box(b, [&](int bu) {
+            CBox &B = cbox(A, bu);
+            const double2 ri = A.r_s[s], vpi = A.vp_s[s], ai = A.acc_s[s];
+            const int cell = A.pcell[s];
+            if (sub == 0) take_sorted(A, s, B, fp32, ri, vpi, ai);
+            v2 = vpi.x * vpi.x + vpi.y * vpi.y;
+            a2 = ai.x * ai.x + ai.y * ai.y;
+            int ns = 0, nl = 0;
+            bool lost = false, wrapped = false, over = false;
+            if (B.build16) list_shared<true>(A, B, s, sub, ri, cell, ns, nl, lost, wrapped, over);
+            else list_shared<false>(A, B, s, sub, ri, cell, ns, nl, lost, wrapped, over);
+            if (sub != 0) return;
+            if (lost) flag_health(A.dyn, bu, HEALTH_LISTCAP);
+            if (over) A.dyn[bu].relist = 1;  // (build_slot)
+            if (s == B.part_off) A.dyn[bu].list16 = B.build16;
+            A.cnt[s] = make_int2(ns | (wrapped ? CNT_WRAP : 0), nl);
+        });
+        if (sub == 0) {
+            x2[0][i] = v2;
+            x2[1][i] = a2;
+        }
+        __syncthreads();
+        if (threadIdx.x < 64) {
+            const int sl = s0 + (int)threadIdx.x;
+            build_tail(A, sl, sl < A.n ? building_box(A, sl, force_mask) : -1, x2[0][threadIdx.x], x2[1][threadIdx.x]);
+        }
+        __syncthreads();
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -3125,9 +3308,24 @@ void launch_box_sort(const ArenaView &A, int force_mask, int nbox, hipStream_t s
 // one block sorts a box: beyond ~16k slots its sequential walk outlasts the
 // radix sort (measured on the served workload, boxes up to 40k slots)
 bool box_sort_fits(int ncells, int n) { return ncells <= BS_MAX_CELLS && n <= BS_MAX_N; }
+// The list kernel: four lanes a slot while a build leaves the chip's SIMDs
+// short of waves, one above.  Whole build stages with 4 / 1 lanes: 1,024 slots
+// 34.1 / 54.3 us, 12,345: 50.4 / 68.8, 65,536: 73.1 / 71.6, 98,304: 88.5 /
+// 80.1, 262,144: 171 / 117.  In an arena each box builds on its own schedule,
+// a sixth to an eighth of the slots a step: 96 boxes of 328,481 slots step in
+// 202 / 219 us, 40 of 178,118 in 158 / 178.  The same lists either way.
+static constexpr int SHARED_BUILD_SLOTS = 49152;
+static constexpr int ARENA_BUILD_PART = 8;
 void launch_build_lists(const ArenaView &A, int force_mask, int fp32, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_build_lists, tile_grid(A), dim3(NT), 0, st, A, force_mask, fp32);
+    const int building = A.one_box >= 0 ? A.n : A.n / ARENA_BUILD_PART;
+    if (building <= SHARED_BUILD_SLOTS) {
+        int nb = (A.n + 63) / 64;  // a block per tile, at least one per XCD
+        nb = ((nb < 2048 ? nb : 2048) + 7) / 8 * 8;
+        hipLaunchKernelGGL(k_build_shared, dim3(nb < 8 ? 8 : nb), dim3(NT), 0, st, A, force_mask, fp32);
+    } else {
+        hipLaunchKernelGGL(k_build_lists, tile_grid(A), dim3(NT), 0, st, A, force_mask, fp32);
+    }
 }
 // Lanes that share a slot's list in the pair passes.  One lane per slot
 // leaves the chip's 1024 SIMDs with less than two waves each up to ~100k
