@@ -1597,24 +1597,28 @@ int sph_nlist_build(sph_box *box, int64_t cap, int64_t *iap, int64_t *nip_out)
     if (!A.d_inv && dalloc(&A.d_inv, A.cap)) return SPH_ERR_NOMEM;
     if (!A.scan_tmp) {  // d_inv may be there from a separations call
         dfree(A.d_cnt); dfree(A.d_off); dfree(A.d_grand);
-        if (dalloc(&A.d_cnt, A.cap) || dalloc(&A.d_off, A.cap) || dalloc(&A.d_grand, 1)) return SPH_ERR_NOMEM;
+        if (dalloc(&A.d_cnt, A.cap) || dalloc(&A.d_off, A.cap) || dalloc(&A.d_grand, 2)) return SPH_ERR_NOMEM;
         A.scan_tmp_bytes = exscan_temp_bytes(A.cap);
         if (dalloc((char **)&A.scan_tmp, A.scan_tmp_bytes)) return SPH_ERR_NOMEM;
     }
     ArenaView V = A.view();
-    launch_inverse(A.id_s, A.boxes[box->b].part_off, n, A.d_inv, st);
-    launch_pairs(V, box->b, n, A.d_inv, A.d_cnt, nullptr, nullptr, 0, st);
-    exclusive_scan_u32(A.d_cnt, A.d_off, n, A.d_grand, A.scan_tmp, st);
-    unsigned grand = 0;
-    HIPCHK(hipMemcpyAsync(&grand, A.d_grand, sizeof(unsigned), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    const int64_t nip = grand;
-    if ((size_t)nip > A.jbuf_cap) {
+    auto room = [&](size_t words) {
+        if (words <= A.jbuf_cap) return (int)SPH_OK;
         dfree(A.d_jbuf);
         A.jbuf_cap = 0;
-        if (dalloc(&A.d_jbuf, (size_t)nip + 1)) return SPH_ERR_NOMEM;
-        A.jbuf_cap = (size_t)nip + 1;
-    }
+        if (dalloc(&A.d_jbuf, words)) return (int)SPH_ERR_NOMEM;
+        A.jbuf_cap = words;
+        return (int)SPH_OK;
+    };
+    const int row = pair_row();
+    if (int rc = room((size_t)n * row)) return rc;
+    unsigned *d_over = A.d_grand + 1;
+    launch_pairs(V, box->b, n, A.d_cnt, A.d_jbuf, d_over, st);
+    exclusive_scan_u32(A.d_cnt, A.d_off, n, A.d_grand, A.scan_tmp, st);
+    unsigned got[2] = {0, 0};  // pairs, and whether a particle has more than a row holds
+    HIPCHK(hipMemcpyAsync(got, A.d_grand, sizeof(got), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    const int64_t nip = got[0];
     const int64_t nout = std::min<int64_t>(nip, cap);
     if ((size_t)nout > A.iap_cap) {
         dfree(A.d_iap);
@@ -1622,8 +1626,12 @@ int sph_nlist_build(sph_box *box, int64_t cap, int64_t *iap, int64_t *nip_out)
         if (dalloc(&A.d_iap, 2 * (size_t)nout + 2)) return SPH_ERR_NOMEM;
         A.iap_cap = (size_t)nout;
     }
-    launch_pairs(V, box->b, n, A.d_inv, A.d_cnt, A.d_off, A.d_jbuf, 1, st);
-    launch_pairs_emit(n, A.d_off, A.d_cnt, A.d_jbuf, A.d_iap, (long long)nout, st);
+    if (got[1]) {
+        if (int rc = room((size_t)nip + 1)) return rc;
+        launch_inverse(A.id_s, A.boxes[box->b].part_off, n, A.d_inv, st);
+        launch_pairs_long(V, box->b, n, A.d_inv, A.d_off, A.d_jbuf, st);
+    }
+    launch_pairs_emit(n, A.d_off, A.d_cnt, A.d_jbuf, got[1] ? 0 : row, A.d_iap, (long long)nout, st);
     HIPCHK(hipGetLastError());
     if (nout > 0)
         HIPCHK(hipMemcpyAsync(iap, A.d_iap, sizeof(long long) * 2 * nout, hipMemcpyDeviceToHost, st));

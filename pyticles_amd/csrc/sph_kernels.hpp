@@ -46,9 +46,14 @@ void launch_put(const PutSpans &P, hipStream_t st);
 void launch_fetch(const ArenaView &A, int n, const int *inv, double *dst, int dyn_words, hipStream_t st);
 void launch_download(const ArenaView &A, int box, int n, int field, double *dst, hipStream_t st);
 void launch_inverse(const int *ids, int off, int n, int *inv, hipStream_t st);
-void launch_pairs(const ArenaView &A, int box, int n, const int *inv, unsigned *count,
-                  const unsigned *offs, int *jbuf, int pass, hipStream_t st);
-void launch_pairs_emit(int n, const unsigned *offs, const unsigned *count, const int *jbuf,
+// sorted partners of particle i in rows[i * pair_row()] on, their number in
+// count[i]; *over is set when one has more than a row holds (then
+// launch_pairs_long fills segments at offs instead)
+int pair_row();
+void launch_pairs(const ArenaView &A, int box, int n, unsigned *count, int *rows, unsigned *over, hipStream_t st);
+void launch_pairs_long(const ArenaView &A, int box, int n, const int *inv, const unsigned *offs, int *jbuf, hipStream_t st);
+// stride: pair_row() for rows, 0 for segments
+void launch_pairs_emit(int n, const unsigned *offs, const unsigned *count, const int *jbuf, int stride,
                        long long *iap, long long cap, hipStream_t st);
 void launch_separations(const ArenaView &A, int box, const int *inv, long long np,
                         const long long *iap, double *drij, double *rij, double *rsq, double *dv,
