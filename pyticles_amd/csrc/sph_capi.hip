@@ -1829,12 +1829,15 @@ int sph_gradients(sph_box *box)
 int sph_rates(sph_box *box, unsigned terms)
 {
     if (!box) return fail(SPH_ERR_ARG, "null box");
+    // an open run closes with the box's own terms, not with this evaluation's
+    if (int rc = settle(box)) return rc;
     Arena &A = box->ar;
+    HIPCHK(hipSetDevice(A.ctx->device));
     BoxDesc &B = A.boxes[box->b];
     const int keep = B.terms;
     B.terms = (int)(terms & SPH_ALL_TERMS);
-    if (int rc = A.relayout(false)) return rc;
-    int rc = eval_box(box, (terms & (SPH_VISCOSITY | SPH_CONDUCTION)) ? 1 : 0, 1);
+    int rc = A.relayout(false);
+    if (!rc) rc = eval_box(box, (terms & (SPH_VISCOSITY | SPH_CONDUCTION)) ? 1 : 0, 1);
     std::string msg = g_err;
     B.terms = keep;
     int rc2 = A.relayout();
