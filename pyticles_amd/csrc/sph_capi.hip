@@ -311,14 +311,19 @@ struct Arena {
     // replays the largest that fit: each graph launch costs ~1-2 us of idle
     // GPU between graphs)
     static constexpr int PLAIN_LOG2 = 3;
-    hipGraphExec_t graph[2][2 + PLAIN_LOG2] = {};  // per parity (the buffers a step starts from)
+    // One set per need_grad (steps without and with the gradient launch) and
+    // parity (the buffers a step starts from).
+    hipGraphExec_t graph[2][2][2 + PLAIN_LOG2] = {};
     // What the captured launches bake in: the view (pointers, slot, key and
     // segment counts), the box count, the sort path and the pass depths.  A
     // relayout that leaves it unchanged (a box's terms or constants changed:
-    // the kernels read those from the box table) keeps the graphs.
+    // the kernels read those from the box table) keeps the graphs, of both
+    // sets: a program that evaluates its forces one by one switches the terms
+    // several times a step (capturing anew at each switch took 2.1 ms of a
+    // sph_box_set_params, 4 us without).
     struct GraphSig {
         ArenaView view;
-        int nbox, small, unroll, unroll_rates, fuse_step, need_grad;
+        int nbox, small, unroll, unroll_rates, fuse_step;
     };
     GraphSig graph_sig;
     bool graph_sig_set = false;
@@ -510,16 +515,23 @@ struct Arena {
     void invalidate_graph()
     {
         graph_sig_set = false;
-        bool any = false;
-        for (auto &gp : graph)
-            for (auto g : gp) any = any || g;
-        if (!any) return;
+        if (!any_graph()) return;
         (void)hipStreamSynchronize(ctx->stream);  // no replay of them is in flight
-        for (auto &gp : graph)
-            for (auto &g : gp) {
-                if (g) (void)hipGraphExecDestroy(g);
-                g = nullptr;
-            }
+        for (auto &set : graph)
+            for (auto &gp : set)
+                for (auto &g : gp) {
+                    if (g) (void)hipGraphExecDestroy(g);
+                    g = nullptr;
+                }
+    }
+
+    bool any_graph() const
+    {
+        for (auto &set : graph)
+            for (auto &gp : set)
+                for (auto g : gp)
+                    if (g) return true;
+        return false;
     }
 
     GraphSig signature() const
@@ -538,7 +550,6 @@ struct Arena {
         sg.unroll = unroll;
         sg.unroll_rates = unroll_rates;
         sg.fuse_step = fuse_step;
-        sg.need_grad = need_grad ? 1 : 0;
         return sg;
     }
 
@@ -570,7 +581,7 @@ struct Arena {
     // without it (the buffers swapping between the captured steps).
     int capture_graph(int idx)
     {
-        hipGraphExec_t &g = graph[parity][idx];
+        hipGraphExec_t &g = graph[need_grad][parity][idx];
         if (g) return SPH_OK;
         check_graph_sig();
         const bool with_build = idx == 1;
@@ -923,10 +934,11 @@ struct Arena {
             const int idx = lg > 0 ? 1 + lg : (with_build ? 1 : 0);
             i += per;
             if (graphs) {
-                // single boxes capture at set-up (prepare_graphs); arenas
+                // single boxes capture at set-up (prepare_graphs) and here
+                // the set for other terms than those of the set-up; arenas
                 // capture here, at the first step after a relayout
                 if (int rc = capture_graph(idx)) return rc;
-                HIPCHK(hipGraphLaunch(graph[parity][idx], ctx->stream));
+                HIPCHK(hipGraphLaunch(graph[need_grad][parity][idx], ctx->stream));
                 if (per & 1) swap_state();
             } else {
                 enqueue_step(with_build);
@@ -1522,7 +1534,9 @@ int sph_box_set_params(sph_box *box, const sph_params *prm)
     box->ar.boxes[box->b] = B;
     box->prm = *prm;
     if (int rc = box->ar.relayout()) return rc;
-    return box->ar.prepare_graphs();
+    // kept graphs serve the new terms too, or steps with them capture their
+    // set (launch_steps): nothing is captured for terms that take no step
+    return box->ar.any_graph() ? (int)SPH_OK : box->ar.prepare_graphs();
 }
 
 static int check_positions(const sph_box *box, const double *r)
