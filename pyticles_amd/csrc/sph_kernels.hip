@@ -3111,9 +3111,11 @@ __global__ __launch_bounds__(NT) void k_energy_blocks(ArenaView A, int box, doub
     for (int q = 0; q < 4; ++q) {
         const int i = i0 + q * NT, s = B.part_off + (i < B.n ? i : 0);
         const double2 v = A.v[s];
-        const double m = i < B.n ? A.m[s] : 0.0;
-        ke += m * (0.5 * (v.x * v.x + v.y * v.y));
-        ue += m * A.u[s];
+        const double m = A.m[s], u = A.u[s];
+        if (i < B.n) {  // (a zero mass past the end would make a NaN of an infinity)
+            ke += m * (0.5 * (v.x * v.x + v.y * v.y));
+            ue += m * u;
+        }
     }
     block_sum2(ke, ue);
     if (threadIdx.x == 0) part[blockIdx.x] = make_double2(ke, ue);
