@@ -1134,8 +1134,14 @@ __device__ __forceinline__ int build_slot(const ArenaView &A, int s, int force_m
 // then place its entries behind those of the lanes before it, so the entries
 // and their order are list_walk's, and every entry is stored to its place by
 // itself.  (With the chip full the scattered stores and the shares' spread
-// cost more than the chain.)  A cell of more than 64 slots (SERIAL, the slot's
-// first lane alone) takes neither masks nor shares.
+// cost more than the chain.)
+//
+// A slot with a cell of more than 64 slots in its stencil takes its cells one
+// after the other instead, 64 candidates at a time, 16 a lane, placed as
+// above: single-cell boxes of 65 slots on and boxes of wide supports or dense
+// cells.  (Whole build stages, one-cell boxes of 100 / 169 slots: 28 / 31 us; one
+// candidate at a time by the slot's first lane took 74 / 101, list_walk's
+// kernel 40 / 54.)
 template <bool L16>
 __device__ __forceinline__ void list_shared(const ArenaView &A, const CBox &B, int s, int sub, double2 ri, int cell,
                                             int &ns, int &nl, bool &lost, bool &wrapped, bool &over)
@@ -1173,8 +1179,46 @@ __device__ __forceinline__ void list_shared(const ArenaView &A, const CBox &B, i
         else list_base(A, s)[(size_t)(P / LIST_GROUP) * LIST_ROW + P % LIST_GROUP] = (unsigned)t;
     };
     auto base = [&](int t0, int t1) { return L16 ? cell_base16(s, nb, t0, t1, wrapped, over) : 0; };
+    // candidates t0 .. te - 1 (at most 64) as masks of short and long entries
+    auto test = [&](int t0, int te, uint64_t &ms, uint64_t &ml) {
+        ms = ml = 0;
+        for (int t = t0; t < te; t += 4) {
+            double2 rj[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) rj[u] = at32(A.r_s, min(t + u, te - 1));
+            unsigned bs = 0, bl = 0;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const double r2 = dist2(rj[u]);
+                const unsigned take = (unsigned)((int)(t + u < te) & (int)(r2 < rnl2) & (int)(t + u != s));
+                const unsigned sh = (unsigned)(r2 < hsk2);
+                bs |= (take & sh) << u;
+                bl |= (take & (sh ^ 1u)) << u;
+            }
+            ms |= (uint64_t)bs << (t - t0);
+            ml |= (uint64_t)bl << (t - t0);
+        }
+    };
+    // the lanes' a short and l long entries behind those placed so far: where
+    // this lane's begin, and the new totals in ns, nl
+    auto places = [&](int a, int l, int &pa, int &pl) {
+        pa = ns;
+        pl = nl;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int x = lane_bcast<4>(a, i), y = lane_bcast<4>(l, i);
+            pa += i < sub ? x : 0;
+            pl += i < sub ? y : 0;
+            ns += x;
+            nl += y;
+        }
+    };
+    auto store = [&](uint64_t ms, uint64_t ml, int t, int ks, int &pa, int &pl) {
+        for (; ms; ms &= ms - 1) put(pa++, t + __ffsll((long long)ms) - 1, ks);
+        for (; ml; ml &= ml - 1) put(lcap - 1 - pl++, t + __ffsll((long long)ml) - 1, ks);
+    };
     uint64_t ms[3], ml[3];
-    int tb[3], kb[3], a = 0, l = 0;
+    int tb[3], kb[3], a = 0, l = 0, pa, pl;
     bool big = false;
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
@@ -1186,75 +1230,39 @@ __device__ __forceinline__ void list_shared(const ArenaView &A, const CBox &B, i
             tb[j] = t0;
             kb[j] = base(t0, t1);
             big = big || t1 - t0 > 64;
-            const int te = min(t1, t0 + 64);
-            for (int t = t0; t < te; t += 4) {
-                double2 rj[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) rj[u] = at32(A.r_s, min(t + u, te - 1));
-                unsigned bs = 0, bl = 0;
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const double r2 = dist2(rj[u]);
-                    const unsigned take = (unsigned)((int)(t + u < te) & (int)(r2 < rnl2) & (int)(t + u != s));
-                    const unsigned sh = (unsigned)(r2 < hsk2);
-                    bs |= (take & sh) << u;
-                    bl |= (take & (sh ^ 1u)) << u;
-                }
-                ms[j] |= (uint64_t)bs << (t - t0);
-                ml[j] |= (uint64_t)bl << (t - t0);
-            }
+            test(t0, big ? t0 : t1, ms[j], ml[j]);
             a += __popcll(ms[j]);
             l += __popcll(ml[j]);
         }
     }
-    // flags of the four lanes, then their counts before this lane's
+    // flags of the four lanes
     int fl = (wrapped ? 1 : 0) | (over ? 2 : 0) | (big ? 4 : 0);
     fl |= __shfl_xor(fl, 1);
     fl |= __shfl_xor(fl, 2);
     wrapped = fl & 1;
     over = (fl & 2) != 0;
-    if (fl & 4) {
-        ns = nl = 0;
-        if (sub == 0) {
-            for (int q = 0; q < nq; ++q) {
-                int t0, t1;
-                cell_at(q, t0, t1);
-                const int ks = base(t0, t1);
-                for (int t = t0; t < t1; ++t) {
-                    const double r2 = dist2(at32(A.r_s, t));
-                    if (!(r2 < rnl2) || t == s) continue;
-                    if (ns + nl >= lcap) {
-                        lost = true;
-                        break;
-                    }
-                    if (r2 < hsk2) put(ns++, t, ks);
-                    else put(lcap - 1 - nl++, t, ks);
-                }
-            }
-            if (lost) ns = nl = 0;
-        }
-        return;
-    }
-    int pa = 0, pl = 0;
     ns = nl = 0;
+    if (fl & 4) {
+        for (int q = 0; q < nq && !lost; ++q) {
+            int t0, t1;
+            cell_at(q, t0, t1);
+            const int ks = base(t0, t1);
+            for (int t = t0; t < t1 && !lost; t += 64) {
+                const int tl = t + 16 * sub;
+                test(tl, min(t1, tl + 16), ms[0], ml[0]);
+                places(__popcll(ms[0]), __popcll(ml[0]), pa, pl);
+                lost = ns + nl > lcap;
+                if (!lost) store(ms[0], ml[0], tl, ks, pa, pl);
+            }
+        }
+    } else {
+        places(a, l, pa, pl);
+        lost = ns + nl > lcap;
+        if (!lost)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int x = lane_bcast<4>(a, i), y = lane_bcast<4>(l, i);
-        pa += i < sub ? x : 0;
-        pl += i < sub ? y : 0;
-        ns += x;
-        nl += y;
+            for (int j = 0; j < 3; ++j) store(ms[j], ml[j], tb[j], kb[j], pa, pl);
     }
-    if (ns + nl > lcap) {
-        lost = true;
-        ns = nl = 0;
-        return;
-    }
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-        for (uint64_t m = ms[j]; m; m &= m - 1) put(pa++, tb[j] + __ffsll((long long)m) - 1, kb[j]);
-        for (uint64_t m = ml[j]; m; m &= m - 1) put(lcap - 1 - pl++, tb[j] + __ffsll((long long)m) - 1, kb[j]);
-    }
+    if (lost) ns = nl = 0;
 }
 
 // The build's largest squared speed and acceleration per box, as step_tail
