@@ -330,6 +330,7 @@ struct Arena {
     int use_graph = 1;
     int always_build = 0;  // arenas: build stage every step (per-box schedule on device)
     int one_box = -1;          // the box owning every slot in use, or -1 (set by relayout)
+    int largest = 0;           // slots of the largest live box (set by relayout)
     int sums = SUMS_MIXED;     // the live boxes' summation orders (set by relayout)
     bool small_boxes = false;  // all live boxes fit the per-box sort (set by relayout)
     int unroll = 0;        // list entries in flight per lane in the pair passes (0 = default)
@@ -362,6 +363,7 @@ struct Arena {
         A.cap = cap;
         A.lcap = lcap;
         A.one_box = one_box;
+        A.largest = largest;
         A.sums = sums;
         A.pass_block = pass_block;
         return A;
@@ -731,9 +733,11 @@ struct Arena {
         nkeys = key;
         // every live box small enough for the per-box sort: no global sort
         small_boxes = true;
+        largest = 0;
         bool any_groups = false, any_plain = false, any_grad = false;
         for (size_t i = 0; i < boxes.size(); ++i) {
             if (!box_live[i]) continue;
+            largest = std::max(largest, boxes[i].n);
             if (!box_sort_fits(boxes[i].ncx * boxes[i].ncy, boxes[i].n)) small_boxes = false;
             (boxes[i].n > SUM_GROUP_MAX ? any_plain : any_groups) = true;
             any_grad = any_grad || (boxes[i].terms & (int)(SPH_VISCOSITY | SPH_CONDUCTION));

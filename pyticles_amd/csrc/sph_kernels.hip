@@ -3385,13 +3385,16 @@ bool box_sort_fits(int ncells, int n) { return ncells <= BS_MAX_CELLS && n <= BS
 // short of waves, one above.  Whole build stages with 4 / 1 lanes: 1,024 slots
 // 34.1 / 54.3 us, 12,345: 50.4 / 68.8, 65,536: 73.1 / 71.6, 98,304: 88.5 /
 // 80.1, 262,144: 171 / 117.  In an arena each box builds on its own schedule,
-// a sixth to an eighth of the slots a step: 96 boxes of 328,481 slots step in
-// 202 / 219 us, 40 of 178,118 in 158 / 178.  The same lists either way.
+// a sixth to an eighth of the slots in use a step where its boxes are many
+// (96 boxes of 328,481 slots step in 202 / 219 us, 40 of 178,118 in 158 / 178),
+// its largest box at once where they are few (two of 150,000: 182 / 180, three
+// of 100,000: 169 / 167, one of 262,144 beside a freed range: 150.5 / 147).
+// The same lists either way.
 static constexpr int SHARED_BUILD_SLOTS = 49152;
 static constexpr int ARENA_BUILD_PART = 8;
 void launch_build_lists(const ArenaView &A, int force_mask, int fp32, hipStream_t st)
 {
-    const int building = A.one_box >= 0 ? A.n : A.n / ARENA_BUILD_PART;
+    const int part = A.n / ARENA_BUILD_PART, building = A.largest > part ? A.largest : part;
     if (building <= SHARED_BUILD_SLOTS) {
         int nb = (A.n + 63) / 64;  // a block per tile, at least one per XCD
         nb = ((nb < 2048 ? nb : 2048) + 7) / 8 * 8;
