@@ -133,7 +133,6 @@ struct sph_ctx {
     void render_trim()
     {
         if (render_bytes <= RENDER_KEEP) return;
-        (void)hipStreamSynchronize(stream);
         dfree(d_render);
         render_bytes = 0;
     }
@@ -2315,10 +2314,15 @@ int sph_splash_map_2d(sph_ctx *ctx, int64_t n, const double *r, const double *m,
     std::lock_guard<std::mutex> lk(ctx->render_mu);  // calls of several threads take turns
     if (ctx->render_space(in_b + xy_b + z_b + SPLASH_HEAD_BYTES + 2 * rec_b + 5 * key_b + cs_b + tmp_b))
         return SPH_ERR_NOMEM;
-    struct Trim {
+    struct Finish {  // on every path out: no copy from or to the caller's arrays is left in flight
         sph_ctx *c;
-        ~Trim() { c->render_trim(); }
-    } trim{ctx};
+        bool waited;
+        ~Finish()
+        {
+            if (!waited) (void)hipStreamSynchronize(c->stream);
+            c->render_trim();
+        }
+    } finish{ctx, false};
     char *at = ctx->d_render;
     auto take = [&](size_t b) {
         char *p = at;
@@ -2351,6 +2355,7 @@ int sph_splash_map_2d(sph_ctx *ctx, int64_t n, const double *r, const double *m,
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(Z, d_Z, sizeof(double) * np, hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
+    finish.waited = true;
     return SPH_OK;
 }
 
