@@ -1637,7 +1637,7 @@ int sph_nlist_build(sph_box *box, int64_t cap, int64_t *iap, int64_t *nip_out)
     if (!A.d_inv && dalloc(&A.d_inv, A.cap)) return SPH_ERR_NOMEM;
     if (!A.scan_tmp) {  // d_inv may be there from a separations call
         dfree(A.d_cnt); dfree(A.d_off); dfree(A.d_grand);
-        if (dalloc(&A.d_cnt, A.cap) || dalloc(&A.d_off, A.cap) || dalloc(&A.d_grand, 2)) return SPH_ERR_NOMEM;
+        if (dalloc(&A.d_cnt, A.cap) || dalloc(&A.d_off, A.cap) || dalloc(&A.d_grand, 3)) return SPH_ERR_NOMEM;
         A.scan_tmp_bytes = exscan_temp_bytes(A.cap);
         if (dalloc((char **)&A.scan_tmp, A.scan_tmp_bytes)) return SPH_ERR_NOMEM;
     }
@@ -1655,9 +1655,13 @@ int sph_nlist_build(sph_box *box, int64_t cap, int64_t *iap, int64_t *nip_out)
     unsigned *d_over = A.d_grand + 1;
     launch_pairs(V, box->b, n, A.d_cnt, A.d_jbuf, d_over, st);
     exclusive_scan_u32(A.d_cnt, A.d_off, n, A.d_grand, A.scan_tmp, st);
-    unsigned got[2] = {0, 0};  // pairs, and whether a particle has more than a row holds
+    // (more particles than can all be partners in under 2^32 pairs)
+    if ((long long)n * (n - 1) / 2 > 0xffffffffll) launch_offsets_wrap(n, A.d_off, A.d_grand, d_over + 1, st);
+    // pairs, whether a particle has more than a row holds, whether the count passed 32 bits
+    unsigned got[3] = {0, 0, 0};
     HIPCHK(hipMemcpyAsync(got, A.d_grand, sizeof(got), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
+    if (got[2]) return fail(SPH_ERR_ARG, "more than 2^32 - 1 pairs: reduce the list cutoff");
     const int64_t nip = got[0];
     const int64_t nout = std::min<int64_t>(nip, cap);
     if ((size_t)nout > A.iap_cap) {

@@ -2982,7 +2982,17 @@ __global__ __launch_bounds__(NT) void k_pairs_long(ArenaView A, int box, const i
     }
 }
 
-__global__ void k_clear_word(unsigned *w) { *w = 0u; }
+__global__ void k_clear_words(unsigned *w) { w[0] = w[1] = 0u; }
+
+// Whether the offsets of the n counts, or their sum *grand, passed 32 bits
+// (one count does not, so an offset that wrapped lies below the one before).
+__global__ __launch_bounds__(NT) void k_offsets_wrap(int n, const unsigned *__restrict__ offs,
+                                                      const unsigned *__restrict__ grand,
+                                                      unsigned *__restrict__ wrapped)
+{
+    const int i = blockIdx.x * NT + threadIdx.x;
+    if (i < n && (i + 1 < n ? offs[i + 1] : *grand) < offs[i]) *wrapped = 1u;
+}
 
 // The j-lists (rows of PAIR_ROW, or with stride 0 segments at offs) to int64
 // iap[k][2], first cap pairs.  A block writes the consecutive pairs of its 64
@@ -2999,8 +3009,8 @@ __global__ __launch_bounds__(NT) void k_pairs_emit(int n, const unsigned *__rest
     if (threadIdx.x < EMIT_N && i < n) end[threadIdx.x] = offs[i] + count[i];
     __syncthreads();
     const unsigned o0 = offs[i0], o1 = end[last];
-    for (unsigned k = o0 + threadIdx.x; k < o1; k += NT) {
-        if ((long long)k >= cap) break;
+    for (long long k = (long long)o0 + threadIdx.x; k < (long long)o1; k += NT) {  // (o1 may lie at the end of 32 bits)
+        if (k >= cap) break;
         int lo = 0, hi = last;  // first particle whose pairs end past k
         while (lo < hi) {
             const int mid = (lo + hi) >> 1;
@@ -3008,7 +3018,7 @@ __global__ __launch_bounds__(NT) void k_pairs_emit(int n, const unsigned *__rest
             else lo = mid + 1;
         }
         const unsigned first = lo > 0 ? end[lo - 1] : o0;
-        const int j = stride ? jbuf[(size_t)(i0 + lo) * stride + (k - first)] : jbuf[k];
+        const int j = stride ? jbuf[(long long)(i0 + lo) * stride + (k - first)] : jbuf[k];
         ((longlong2 *)iap)[k] = make_longlong2(i0 + lo, j);
     }
 }
@@ -3503,8 +3513,12 @@ void launch_inverse(const int *ids, int off, int n, int *inv, hipStream_t st)
 int pair_row() { return PAIR_ROW; }
 void launch_pairs(const ArenaView &A, int box, int n, unsigned *count, int *rows, unsigned *over, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_clear_word, dim3(1), dim3(1), 0, st, over);
+    hipLaunchKernelGGL(k_clear_words, dim3(1), dim3(1), 0, st, over);
     hipLaunchKernelGGL(k_pairs, grid_for_bs(n, PAIR_NT), dim3(PAIR_NT), 0, st, A, box, count, rows, over);
+}
+void launch_offsets_wrap(int n, const unsigned *offs, const unsigned *grand, unsigned *wrapped, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_offsets_wrap, grid_for(n), dim3(NT), 0, st, n, offs, grand, wrapped);
 }
 void launch_pairs_long(const ArenaView &A, int box, int n, const int *inv, const unsigned *offs, int *jbuf, hipStream_t st)
 {

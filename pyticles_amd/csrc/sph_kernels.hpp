@@ -47,9 +47,11 @@ void launch_fetch(const ArenaView &A, int n, const int *inv, double *dst, int dy
 void launch_download(const ArenaView &A, int box, int n, int field, double *dst, hipStream_t st);
 void launch_inverse(const int *ids, int off, int n, int *inv, hipStream_t st);
 // sorted partners of particle i in rows[i * pair_row()] on, their number in
-// count[i]; *over is set when one has more than a row holds (then
-// launch_pairs_long fills segments at offs instead)
+// count[i]; over[0] is set when one has more than a row holds (then
+// launch_pairs_long fills segments at offs instead), over[1] is cleared for
+// launch_offsets_wrap, which sets it when the counts' sum passed 32 bits
 int pair_row();
+void launch_offsets_wrap(int n, const unsigned *offs, const unsigned *grand, unsigned *wrapped, hipStream_t st);
 void launch_pairs(const ArenaView &A, int box, int n, unsigned *count, int *rows, unsigned *over, hipStream_t st);
 void launch_pairs_long(const ArenaView &A, int box, int n, const int *inv, const unsigned *offs, int *jbuf, hipStream_t st);
 // stride: pair_row() for rows, 0 for segments
