@@ -278,7 +278,10 @@ int sph_box_set_graph(sph_box *box, int on);
 /* Launch schedule of the pair passes: list entries whose loads are in
  * flight per lane (1, 2 or 4; 0 = the precision's default).  Chosen by the
  * autotuner (pyticles_amd/autotune.py); any value gives the same results up
- * to summation order.  No counterpart in the reference. */
+ * to summation order.  Up to 98,304 slots in use two or four lanes share a
+ * slot's list at the depths 0, 4 and in the FP64 form 2; the others give a
+ * list one lane at any size, which is slower there.  No counterpart in the
+ * reference. */
 int sph_arena_set_schedule(sph_arena *ar, int unroll);
 int sph_box_set_schedule(sph_box *box, int unroll);
 /* The same for the rate pass alone (0 = as the other passes): its walk keeps
@@ -288,7 +291,10 @@ int sph_box_set_schedule(sph_box *box, int unroll);
 int sph_arena_set_rates_unroll(sph_arena *ar, int unroll);
 int sph_box_set_rates_unroll(sph_box *box, int unroll);
 /* Work-items per block of the three pair passes: 128, 256 or 512 (0 = the
- * default 256).  A launch schedule the autotuner picks per workload class;
+ * default 256).  It applies where one lane walks a slot's list: above 98,304
+ * slots in use, and at the depths (sph_*_set_schedule) that do not share
+ * lists, 1 and in the FP32C form 2.  Passes that share lists always take
+ * blocks of 256.  A launch schedule the autotuner picks per workload class;
  * results do not depend on it.  No counterpart in the reference. */
 int sph_arena_set_pass_block(sph_arena *ar, int block);
 int sph_box_set_pass_block(sph_box *box, int block);

@@ -85,8 +85,9 @@ class Arena:
     def set_schedule(self, unroll, rates_unroll=0, block=0, list_bits=0, fused=1):
         """List entries in flight per lane in the pair passes (1, 2, 4; 0 =
         default), in the rate pass alone (0 = the same), the pair passes'
-        block size (128, 256, 512; 0 = 256), the list entry width (16,
-        32; 0 = leave it) and whether the leapfrog step runs inside the rate
+        block size (128, 256, 512; 0 = 256; passes whose lists are shared by
+        lanes, up to 98,304 slots at the default depth, always take 256), the
+        list entry width (16, 32; 0 = leave it) and whether the leapfrog step runs inside the rate
         pass (1) or as a launch of its own (0).  unroll may be a schedule
         dict from autotune.schedule_for."""
         if isinstance(unroll, dict):

@@ -13,7 +13,9 @@ rounding; the list entry width not even that):
             for batched boxes); tuned after the other two
     block   work-items per block of the three pair passes (128, 256 or
             512): how the slots, in cell order, are dealt to the XCDs and
-            CUs
+            CUs.  Passes whose lists are shared by lanes (up to 98,304
+            slots at unroll 4, FP64 also 2) always take 256: there the
+            candidates time the same launches
     list_bits
             neighbour-list entry width (16: slot offsets, half the list
             bytes, one 16-byte load per eight entries; 32: slots); same

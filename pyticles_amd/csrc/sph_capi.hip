@@ -333,7 +333,7 @@ struct Arena {
     int sums = SUMS_MIXED;     // the live boxes' summation orders (set by relayout)
     bool small_boxes = false;  // all live boxes fit the per-box sort (set by relayout)
     int unroll = 0;        // list entries in flight per lane in the pair passes (0 = default)
-    int pass_block = 256;  // work-items per block of the pair passes (128, 256, 512)
+    int pass_block = 256;  // work-items per block of the pair passes (128, 256, 512) where one lane walks a list
     int unroll_rates = 0;  // the same for the rate pass alone (0 = unroll)
     int fuse_step = 1;     // the leapfrog step inside the rate pass (0: a launch of its own)
     int rates_unroll() const { return unroll_rates ? unroll_rates : unroll; }

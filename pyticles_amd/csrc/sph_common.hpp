@@ -208,7 +208,7 @@ struct ArenaView {
     int one_box;         // the box that owns every slot in use, or -1 (several, or free slots)
     int largest;         // slots of the largest live box
     int sums;            // summation orders of the live boxes (SUMS_*)
-    int pass_block;      // work-items per block of the pair passes (128, 256 or 512)
+    int pass_block;      // work-items per block of the pair passes (128, 256 or 512) where one lane walks a list
 };
 
 // Cell grid of the splash rendering: cells at least as wide as the largest

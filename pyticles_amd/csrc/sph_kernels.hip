@@ -2898,7 +2898,12 @@ __global__ __launch_bounds__(NT) void k_inverse(const int *__restrict__ ids, int
 //
 // (Over caller indices, a search each to count and to store and an insertion
 // sort in global memory, 27 dependent accesses an entry in the worst case, the
-// two searches took 330 us at 20,011 particles; this one 81 us.)
+// two searches took 330 us at 20,011 particles on a jittered lattice; this one
+// 81 us.  A list cutoff of 4 gives 26 partners a particle, 44 at most on that
+// lattice and 53 after 400 steps; of uniformly random positions some exceed a
+// row, and the export then takes the two searches' time: 0.83 ms a call of
+// 20,011 particles without its download, as before, where rows alone take
+// 0.20.)
 static constexpr int PAIR_ROW = 56;
 static constexpr int PAIR_NT = 64;
 
@@ -3282,8 +3287,10 @@ __host__ __device__ inline int splash_block_bits(int li) { return li == 3 ? 4 : 
 // (100 us along pixel rows with cells one cutoff wide, two divisions and a
 // correctly rounded root per pair in reach); what bounds it now is the FP64
 // arithmetic of the pairs some lane of a wave has in reach.  The root is
-// sqrt_pair's and the partial sums keep the total's error at the level of the
-// running sum it replaces (3.29e-16 against 3.35e-16 in long double).
+// sqrt_pair's and 1 / h is rounded once more than a quotient; the partial sums
+// make up for it: against extended precision the field is 3.38e-16 off, with
+// correctly rounded roots and quotients and one running sum a pixel 3.45e-16
+// (tests/test_gpu_render_error.py).
 __global__ __launch_bounds__(NT) void k_splash_pixels(long long tiles, int li, int nx, int ny,
                                                        const double *__restrict__ x,
                                                        const double *__restrict__ y,
