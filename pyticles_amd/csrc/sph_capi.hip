@@ -1274,13 +1274,62 @@ int list_entries_for(const sph_params *p, int64_t n)
     return std::max(64, std::min(l, 4096));
 }
 
+typedef double v2d __attribute__((vector_size(16)));
+typedef long long v2l __attribute__((vector_size(16)));
+
 // The common mass of m[0 .. n) when all are equal, positive and finite, else 0
 // (the passes then skip the per-neighbour mass fetch).
 double common_mass(const double *m, int64_t n)
 {
-    bool uni = n > 0 && m[0] > 0.0 && std::isfinite(m[0]);
-    for (int64_t i = 1; uni && i < n; ++i) uni = m[i] == m[0];
-    return uni ? m[0] : 0.0;
+    if (!(n > 0 && m[0] > 0.0 && std::isfinite(m[0]))) return 0.0;
+    const v2d first = {m[0], m[0]};
+    for (int64_t i = 0; i < n; i += 256) {
+        const int64_t end = std::min<int64_t>(i + 256, n);
+        v2l eq0 = {-1, -1}, eq1 = {-1, -1};
+        int64_t k = i;
+        for (; k + 3 < end; k += 4) {
+            v2d p, q;
+            memcpy(&p, m + k, sizeof(p));
+            memcpy(&q, m + k + 2, sizeof(q));
+            eq0 &= p == first;
+            eq1 &= q == first;
+        }
+        bool same = true;
+        for (; k < end; ++k) same = same && m[k] == m[0];
+        eq0 &= eq1;
+        if (!same || !(eq0[0] & eq0[1])) return 0.0;
+    }
+    return m[0];
+}
+
+// First of n positions outside [0, Lx) x [0, Ly), or n.  Two positions at a
+// time, a branch every 256 (one by one the check took 200 of an upload's
+// 274 us at 300,000 positions).
+int64_t first_outside(const double *r, int64_t n, double Lx, double Ly)
+{
+    const v2d L = {Lx, Ly}, zero = {0.0, 0.0};
+    for (int64_t i = 0; i < n; i += 256) {
+        const int64_t end = std::min<int64_t>(i + 256, n);
+        v2l in0 = {-1, -1}, in1 = {-1, -1};
+        int64_t k = i;
+        for (; k + 1 < end; k += 2) {
+            v2d p, q;
+            memcpy(&p, r + 2 * k, sizeof(p));
+            memcpy(&q, r + 2 * k + 2, sizeof(q));
+            in0 &= (p >= zero) & (p < L);  // (false for NaN)
+            in1 &= (q >= zero) & (q < L);
+        }
+        if (k < end) {
+            v2d p;
+            memcpy(&p, r + 2 * k, sizeof(p));
+            in0 &= (p >= zero) & (p < L);
+        }
+        in0 &= in1;
+        if (in0[0] & in0[1]) continue;
+        for (k = i;; ++k)
+            if (!(r[2 * k] >= 0.0 && r[2 * k] < Lx && r[2 * k + 1] >= 0.0 && r[2 * k + 1] < Ly)) return k;
+    }
+    return n;
 }
 
 // A new box of n particles in state D at initial temperature T0; r, v, m
@@ -1545,13 +1594,10 @@ int sph_box_set_params(sph_box *box, const sph_params *prm)
 static int check_positions(const sph_box *box, const double *r)
 {
     const int n = box->ar.boxes[box->b].n;
-    const double Lx = box->prm.Lx, Ly = box->prm.Ly;
-    for (int i = 0; i < n; ++i) {
-        const double x = r[2 * i], y = r[2 * i + 1];
-        if (!(x >= 0.0 && x < Lx && y >= 0.0 && y < Ly))
-            return fail(SPH_ERR_ARG, "position of particle " + std::to_string(i) +
-                                         " lies outside [0, L); wrap positions into the periodic box first");
-    }
+    const int64_t i = first_outside(r, n, box->prm.Lx, box->prm.Ly);
+    if (i < n)
+        return fail(SPH_ERR_ARG, "position of particle " + std::to_string(i) +
+                                     " lies outside [0, L); wrap positions into the periodic box first");
     return SPH_OK;
 }
 
@@ -2077,11 +2123,7 @@ int sph_arena_add(sph_arena *ar, int64_t n, const sph_params *prm, const double 
     if (!ar || !prm || !r || !v || !m || !box_id || nsteps < 0) return fail(SPH_ERR_ARG, "invalid argument");
     Arena &A = ar->ar;
     HIPCHK(hipSetDevice(A.ctx->device));
-    for (int64_t i = 0; i < n; ++i) {
-        const double x = r[2 * i], y = r[2 * i + 1];
-        if (!(x >= 0.0 && x < prm->Lx && y >= 0.0 && y < prm->Ly))
-            return fail(SPH_ERR_ARG, "position outside [0, L)");
-    }
+    if (first_outside(r, n, prm->Lx, prm->Ly) < n) return fail(SPH_ERR_ARG, "position outside [0, L)");
     BoxDyn D;
     memset(&D, 0, sizeof(D));
     D.state = BOX_INIT;
