@@ -137,6 +137,94 @@ struct sph_ctx {
         render_bytes = 0;
     }
 
+    // Pinned host memory that the boxes and arenas of this context share (they
+    // share its stream), allocated once: a box that pinned its own paid for it
+    // at its first download and its end (1 MB: 0.2-0.5 ms each time), and an
+    // arena for the first touch of its pages (1.5 us each).
+    //
+    // The feed: memory the device reads directly (tables and states of
+    // admitted boxes), two halves used in turn, each waited for before it is
+    // reused.  feed_mu is held from feed() until the launch that reads the
+    // bytes is queued.
+    static constexpr size_t FEED_HALF = (size_t)512 << 10;
+    std::mutex feed_mu;
+    char *h_feed = nullptr, *d_feed = nullptr;
+    hipEvent_t feed_done[2] = {nullptr, nullptr};
+    bool feed_used[2] = {false, false};
+    int feed_half = 0;
+    size_t feed_at = 0;
+
+    // bytes (at most FEED_HALF) of host memory that launches queued from now
+    // on may read
+    int feed(size_t bytes, char **h, char **d)
+    {
+        bytes = align256(bytes);
+        if (bytes > FEED_HALF) return fail(SPH_ERR_ARG, "feed request too large");
+        if (!h_feed) {
+            for (auto &e : feed_done)
+                if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+            char *p = nullptr;
+            if (hipHostMalloc((void **)&p, 2 * FEED_HALF, hipHostMallocDefault) != hipSuccess)
+                return fail(SPH_ERR_NOMEM, "hipHostMalloc failed");
+            if (hipHostGetDevicePointer((void **)&d_feed, p, 0) != hipSuccess) {
+                (void)hipHostFree(p);
+                return fail(SPH_ERR_HIP, "hipHostGetDevicePointer failed");
+            }
+            h_feed = p;
+        }
+        if (feed_at + bytes > FEED_HALF) {
+            HIPCHK(hipEventRecord(feed_done[feed_half], stream));
+            feed_used[feed_half] = true;
+            feed_half ^= 1;
+            feed_at = 0;
+            if (feed_used[feed_half]) HIPCHK(hipEventSynchronize(feed_done[feed_half]));
+        }
+        const size_t at = feed_half * FEED_HALF + feed_at;
+        feed_at += bytes;
+        *h = h_feed + at;
+        *d = d_feed + at;
+        return SPH_OK;
+    }
+
+    // Two halves through which downloads pass (Arena::to_host, under down_mu).
+    static constexpr size_t DOWN_HALF = (size_t)64 << 10;  // words
+    hipEvent_t down_done[2] = {nullptr, nullptr};
+    std::mutex down_mu;
+    double *h_down = nullptr, *d_down = nullptr;
+
+    int down_open()
+    {
+        if (h_down) return SPH_OK;
+        for (auto &e : down_done)
+            if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        if (hipHostMalloc((void **)&h_down, 2 * DOWN_HALF * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+            h_down = nullptr;
+            return fail(SPH_ERR_NOMEM, "hipHostMalloc failed");
+        }
+        if (hipHostGetDevicePointer((void **)&d_down, h_down, 0) != hipSuccess) {
+            (void)hipHostFree(h_down);
+            h_down = nullptr;
+            return fail(SPH_ERR_HIP, "hipHostGetDevicePointer failed");
+        }
+        return SPH_OK;
+    }
+
+    void release_pinned()
+    {
+        if (h_feed) (void)hipHostFree(h_feed);
+        h_feed = d_feed = nullptr;
+        for (auto &e : feed_done) {
+            if (e) (void)hipEventDestroy(e);
+            e = nullptr;
+        }
+        if (h_down) (void)hipHostFree(h_down);
+        h_down = d_down = nullptr;
+        for (auto &e : down_done) {
+            if (e) (void)hipEventDestroy(e);
+            e = nullptr;
+        }
+    }
+
     int scratch(size_t bytes)
     {
         if (bytes <= scratch_bytes) return SPH_OK;
@@ -254,15 +342,6 @@ struct Arena {
     size_t stage_bytes = 0;
     double *h_stage = nullptr;  // pinned
     size_t h_stage_bytes = 0;
-
-    // host memory the device reads directly (tables and states of admitted
-    // boxes): two halves used in turn, each waited for before it is reused
-    static constexpr size_t FEED_HALF = (size_t)4 << 20;
-    char *h_feed = nullptr, *d_feed = nullptr;
-    hipEvent_t feed_done[2] = {nullptr, nullptr};
-    bool feed_used[2] = {false, false};
-    int feed_half = 0;
-    size_t feed_at = 0;
 
     // asynchronous snapshots: state copied on the device in stream order,
     // then to the host on a copy stream
@@ -453,12 +532,6 @@ struct Arena {
         if (h_stage) (void)hipHostFree(h_stage);
         h_stage = nullptr;
         h_stage_bytes = 0;
-        if (h_feed) (void)hipHostFree(h_feed);
-        h_feed = d_feed = nullptr;
-        for (auto &e : feed_done) {
-            if (e) (void)hipEventDestroy(e);
-            e = nullptr;
-        }
         dfree(d_inv); dfree(d_cnt); dfree(d_off); dfree(d_grand); dfree(d_jbuf); dfree(d_iap);
         if (scan_tmp) (void)hipFree(scan_tmp);
         scan_tmp = nullptr;
@@ -624,37 +697,6 @@ struct Arena {
         return SPH_OK;
     }
 
-    // bytes (at most FEED_HALF) of host memory that launches enqueued from now
-    // on may read
-    int feed(size_t bytes, char **h, char **d)
-    {
-        bytes = align256(bytes);
-        if (bytes > FEED_HALF) return fail(SPH_ERR_ARG, "feed request too large");
-        if (!h_feed) {
-            for (auto &e : feed_done) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-            char *p = nullptr;
-            if (hipHostMalloc((void **)&p, 2 * FEED_HALF, hipHostMallocDefault) != hipSuccess)
-                return fail(SPH_ERR_NOMEM, "hipHostMalloc failed");
-            if (hipHostGetDevicePointer((void **)&d_feed, p, 0) != hipSuccess) {
-                (void)hipHostFree(p);
-                return fail(SPH_ERR_HIP, "hipHostGetDevicePointer failed");
-            }
-            h_feed = p;
-        }
-        if (feed_at + bytes > FEED_HALF) {
-            HIPCHK(hipEventRecord(feed_done[feed_half], ctx->stream));
-            feed_used[feed_half] = true;
-            feed_half ^= 1;
-            feed_at = 0;
-            if (feed_used[feed_half]) HIPCHK(hipEventSynchronize(feed_done[feed_half]));
-        }
-        const size_t at = feed_half * FEED_HALF + feed_at;
-        feed_at += bytes;
-        *h = h_feed + at;
-        *d = d_feed + at;
-        return SPH_OK;
-    }
-
     // Entries [lo, hi) of the box table that differ from what was last sent
     // (adding a box to an arena changes one of them).
     void changed_boxes(size_t &lo, size_t &hi) const
@@ -679,10 +721,11 @@ struct Arena {
         const size_t nd = dyn_b >= 0 ? sizeof(BoxDyn) : 0;
         if (nb + ns + nd == 0) return SPH_OK;
         sent.clear();  // until the entries are queued
-        if (align256(nb) + align256(ns) + nd <= FEED_HALF) {
+        if (align256(nb) + align256(ns) + nd <= sph_ctx::FEED_HALF) {
             static_assert(sizeof(BoxDesc) % 4 == 0 && sizeof(SegDesc) % 4 == 0 && sizeof(BoxDyn) % 4 == 0, "words");
             char *h, *d;
-            if (int rc = feed(align256(nb) + align256(ns) + nd, &h, &d)) return rc;
+            std::lock_guard<std::mutex> lk(ctx->feed_mu);
+            if (int rc = ctx->feed(align256(nb) + align256(ns) + nd, &h, &d)) return rc;
             PutSpans P;
             memset(&P, 0, sizeof(P));
             auto span = [&](int q, void *dst, const void *src, size_t at, size_t bytes) {
@@ -767,7 +810,7 @@ struct Arena {
         return SPH_OK;
     }
 
-    // pinned host staging for combined downloads
+    // pinned host memory that arena results are written to
     int host_stage(size_t bytes)
     {
         if (bytes <= h_stage_bytes) return SPH_OK;
@@ -781,28 +824,30 @@ struct Arena {
     }
 
     // `total` 8-byte words at src to the host's pieces, one behind another,
-    // through two pinned halves in turn: one is filled while the host empties
-    // the other (nine fields of 65,536 particles: 1.22 ms; 1.39 copied whole,
-    // then emptied).  Pinning costs about 0.25 ms a megabyte: a buffer of
-    // those fields' size took 2.6 ms of a first download
+    // through the context's two pinned halves in turn: the device fills one
+    // (launch_to_host) while the host empties the other
     struct Piece { void *dst; size_t words; };
     int to_host(const void *src, const Piece *piece, int pieces)
     {
-        static constexpr size_t HALF = (size_t)64 << 10;  // words
+        constexpr size_t HALF = sph_ctx::DOWN_HALF;
         size_t total = 0;
         for (int p = 0; p < pieces; p++) total += piece[p].words;
-        if (host_stage(sizeof(double) * std::min(total, 2 * HALF))) return SPH_ERR_NOMEM;
+        if (total == 0) return SPH_OK;
+        std::lock_guard<std::mutex> lk(ctx->down_mu);  // downloads of several threads take turns
+        if (int rc = ctx->down_open()) return rc;
         hipStream_t st = ctx->stream;
         auto fetch = [&](size_t lo) {  // words [lo, lo+HALF)
             if (lo >= total) return hipSuccess;
-            return hipMemcpyAsync(h_stage + (lo / HALF & 1) * HALF, (const double *)src + lo,
-                                  sizeof(double) * std::min(HALF, total - lo), hipMemcpyDeviceToHost, st);
+            const size_t half = lo / HALF & 1;
+            launch_to_host(std::min(HALF, total - lo), (const double *)src + lo, ctx->d_down + half * HALF, st);
+            const hipError_t e = hipGetLastError();
+            return e != hipSuccess ? e : hipEventRecord(ctx->down_done[half], st);
         };
         HIPCHK(fetch(0));
+        HIPCHK(fetch(HALF));
         for (size_t lo = 0; lo < total; lo += HALF) {
-            HIPCHK(hipStreamSynchronize(st));
-            HIPCHK(fetch(lo + HALF));
-            const double *half = h_stage + (lo / HALF & 1) * HALF;
+            HIPCHK(hipEventSynchronize(ctx->down_done[lo / HALF & 1]));
+            const double *half = ctx->h_down + (lo / HALF & 1) * HALF;
             const size_t hi = std::min(lo + HALF, total);
             size_t at = 0;  // the piece's first word
             for (int p = 0; p < pieces; p++) {
@@ -810,6 +855,7 @@ struct Arena {
                 if (x < y) memcpy((double *)piece[p].dst + (x - at), half + (x - lo), sizeof(double) * (y - x));
                 at = end;
             }
+            HIPCHK(fetch(lo + 2 * HALF));
         }
         return SPH_OK;
     }
@@ -1384,11 +1430,12 @@ int Arena::add_box(int64_t n, const sph_params *prm, int *box_out, const BoxDyn 
         launch_assign_slots(view(), off, (int)n, b, 0, nullptr, ctx->stream);
     } else {
         // the particles' state through the feed, in pieces that fit half of it
-        const int64_t most = (int64_t)(FEED_HALF / 2 / (5 * sizeof(double)));
+        const int64_t most = (int64_t)(sph_ctx::FEED_HALF / 2 / (5 * sizeof(double)));
         for (int64_t i = 0; i < n; i += most) {
             const size_t k = (size_t)std::min(most, n - i);
             char *h, *d;
-            if (int rc = feed(5 * sizeof(double) * k, &h, &d)) return rc;
+            std::lock_guard<std::mutex> lk(ctx->feed_mu);
+            if (int rc = ctx->feed(5 * sizeof(double) * k, &h, &d)) return rc;
             double *p = (double *)h;
             memcpy(p, r + 2 * i, sizeof(double) * 2 * k);
             memcpy(p + 2 * k, v + 2 * i, sizeof(double) * 2 * k);
@@ -1522,6 +1569,7 @@ int sph_ctx_destroy(sph_ctx *ctx)
     (void)hipStreamSynchronize(ctx->stream);
     dfree(ctx->d_scratch);
     dfree(ctx->d_render);
+    ctx->release_pinned();
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return SPH_OK;
@@ -2178,18 +2226,29 @@ int sph_arena_result(sph_arena *ar, int box_id, double *r, double *v, double *u,
     // device itself, one wait for all
     const int n = A.boxes[box_id].n;
     const size_t nd = (size_t)n;
-    const size_t dyn_bytes = sizeof(BoxDyn) * A.boxes.size();
-    if (A.host_stage(sizeof(double) * 6 * nd + dyn_bytes)) return SPH_ERR_NOMEM;
+    // (the context's halves, or pinned memory of the arena's own where they
+    // are too small)
+    const size_t dyn_bytes = sizeof(BoxDyn) * A.boxes.size(), bytes = sizeof(double) * 6 * nd + dyn_bytes;
     if (!A.d_inv && dalloc(&A.d_inv, A.cap)) return SPH_ERR_NOMEM;
+    std::unique_lock<std::mutex> lk(A.ctx->down_mu, std::defer_lock);
     double *dst = nullptr;
-    HIPCHK(hipHostGetDevicePointer((void **)&dst, A.h_stage, 0));
+    const double *h = nullptr;
+    if (bytes <= sizeof(double) * 2 * sph_ctx::DOWN_HALF) {
+        lk.lock();
+        if (int rc = A.ctx->down_open()) return rc;
+        dst = A.ctx->d_down;
+        h = A.ctx->h_down;
+    } else {
+        if (A.host_stage(bytes)) return SPH_ERR_NOMEM;
+        HIPCHK(hipHostGetDevicePointer((void **)&dst, A.h_stage, 0));
+        h = A.h_stage;
+    }
     launch_inverse(A.id, A.boxes[box_id].part_off, n, A.d_inv, A.ctx->stream);
     launch_fetch(A.view(), n, A.d_inv, dst, (int)(dyn_bytes / 4), A.ctx->stream);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(A.ctx->stream));
-    memcpy((void *)A.h_dyn, A.h_stage + 6 * nd, dyn_bytes);
+    memcpy((void *)A.h_dyn, h + 6 * nd, dyn_bytes);
     if (int rc = A.release_held()) return rc;
-    const double *h = A.h_stage;
     if (r) memcpy(r, h, sizeof(double) * 2 * nd);
     if (v) memcpy(v, h + 2 * nd, sizeof(double) * 2 * nd);
     if (u) memcpy(u, h + 4 * nd, sizeof(double) * nd);

@@ -43,6 +43,7 @@ struct PutSpans {
     int words[3];
 };
 void launch_put(const PutSpans &P, hipStream_t st);
+void launch_to_host(size_t n, const double *src, double *dst, hipStream_t st);
 void launch_fetch(const ArenaView &A, int n, const int *inv, double *dst, int dyn_words, hipStream_t st);
 void launch_download(const ArenaView &A, int box, int n, int field, double *dst, hipStream_t st);
 void launch_inverse(const int *ids, int off, int n, int *inv, hipStream_t st);
