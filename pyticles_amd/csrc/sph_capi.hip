@@ -350,7 +350,6 @@ struct Arena {
     hipStream_t copy_stream = nullptr;
     hipEvent_t ev_snap_ready = nullptr, ev_snap_done = nullptr;
     bool snap_pending = false;
-    double *d_e3 = nullptr;
 
     // pair export buffers
     int *d_inv = nullptr;
@@ -480,7 +479,6 @@ struct Arena {
         rc |= dalloc(&k_alt, cap); rc |= dalloc(&v_alt, cap);
         sort_tmp_bytes = radix_sort_temp_bytes(cap);
         rc |= dalloc((char **)&sort_tmp, sort_tmp_bytes);
-        rc |= dalloc(&d_e3, 3);
         rc |= dalloc(&plan_n, 4);
         rc |= dalloc(&tile_list, (size_t)(cap + 63) / 64 + 1);
         rc |= dalloc(&wdisp, (size_t)(cap + 63) / 64);
@@ -528,7 +526,7 @@ struct Arena {
         copy_stream = nullptr;
         dfree(d_snap);
         snap_cap = 0;
-        dfree(cell_start); dfree(d_boxes); dfree(d_dyn); dfree(d_segs); dfree(d_stage); dfree(d_e3);
+        dfree(cell_start); dfree(d_boxes); dfree(d_dyn); dfree(d_segs); dfree(d_stage);
         if (h_stage) (void)hipHostFree(h_stage);
         h_stage = nullptr;
         h_stage_bytes = 0;
@@ -2044,12 +2042,14 @@ int sph_energy(sph_box *box, double *ke, double *ue, double *etot)
     if (int rc = settle(box)) return rc;
     Arena &A = box->ar;
     HIPCHK(hipSetDevice(A.ctx->device));
-    double out[3];
     const int n = A.boxes[box->b].n;
     if (A.stage(sizeof(double2) * (size_t)energy_blocks(n))) return SPH_ERR_NOMEM;
-    launch_energy_now(A.view(), box->b, n, (double2 *)A.d_stage, A.d_e3, A.ctx->stream);
+    // the totals go to the context's pinned memory by themselves
+    std::lock_guard<std::mutex> lk(A.ctx->down_mu);
+    if (int rc = A.ctx->down_open()) return rc;
+    const double *out = A.ctx->h_down;
+    launch_energy_now(A.view(), box->b, n, (double2 *)A.d_stage, A.ctx->d_down, A.ctx->stream);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(out, A.d_e3, sizeof(out), hipMemcpyDeviceToHost, A.ctx->stream));
     HIPCHK(hipStreamSynchronize(A.ctx->stream));
     if (ke) *ke = out[0];
     if (ue) *ue = out[1];

@@ -3123,8 +3123,10 @@ __global__ __launch_bounds__(NT) void k_set_u(ArenaView A, int box, const double
 // them the box's totals out3 = (kinetic, thermal, sum).  A block takes 1,024
 // slots in four strided loads a thread; the second launch adds the block sums
 // in a fixed order.  (One block over the whole box read it at the rate of one
-// CU: 286 us at 262,144 slots, 1,158 us at 1,048,576.)
+// CU: 286 us at 262,144 slots, 1,158 us at 1,048,576.)  Boxes of up to EN_ONE
+// slots take one block and no second launch.
 static constexpr int EN_SLOTS = 4 * NT;
+static constexpr int EN_ONE = 4 * EN_SLOTS;
 
 __device__ __forceinline__ void block_sum2(double &a, double &b)
 {
@@ -3143,13 +3145,15 @@ __device__ __forceinline__ void block_sum2(double &a, double &b)
     b = (wb[0] + wb[1]) + (wb[2] + wb[3]);
 }
 
-__global__ __launch_bounds__(NT) void k_energy_blocks(ArenaView A, int box, double2 *__restrict__ part)
+// (rounds of EN_SLOTS slots a block; the only block writes the totals itself)
+__global__ __launch_bounds__(NT) void k_energy_blocks(ArenaView A, int box, int rounds, double2 *__restrict__ part,
+                                                       double *__restrict__ out3)
 {
     const BoxDesc &B = A.boxes[box];
-    const int i0 = (int)blockIdx.x * EN_SLOTS + threadIdx.x;
+    const int i0 = (int)blockIdx.x * rounds * EN_SLOTS + threadIdx.x;
     double ke = 0.0, ue = 0.0;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
+#pragma unroll 4
+    for (int q = 0; q < 4 * rounds; ++q) {
         const int i = i0 + q * NT, s = B.part_off + (i < B.n ? i : 0);
         const double2 v = A.v[s];
         const double m = A.m[s], u = A.u[s];
@@ -3159,7 +3163,14 @@ __global__ __launch_bounds__(NT) void k_energy_blocks(ArenaView A, int box, doub
         }
     }
     block_sum2(ke, ue);
-    if (threadIdx.x == 0) part[blockIdx.x] = make_double2(ke, ue);
+    if (threadIdx.x != 0) return;
+    if (gridDim.x > 1) {
+        part[blockIdx.x] = make_double2(ke, ue);
+    } else {
+        out3[0] = ke;
+        out3[1] = ue;
+        out3[2] = ke + ue;
+    }
 }
 
 __global__ __launch_bounds__(NT) void k_energy_total(int nblocks, const double2 *__restrict__ part,
@@ -3603,12 +3614,13 @@ void launch_set_u(const ArenaView &A, int box, int n, const double *T, double T0
 {
     hipLaunchKernelGGL(k_set_u, grid_for(n), dim3(NT), 0, st, A, box, T, T0);
 }
-int energy_blocks(int n) { return n > 0 ? (n + EN_SLOTS - 1) / EN_SLOTS : 1; }
+int energy_blocks(int n) { return n > EN_ONE ? (n + EN_SLOTS - 1) / EN_SLOTS : 1; }
 void launch_energy_now(const ArenaView &A, int box, int n, double2 *part, double *out, hipStream_t st)
 {
     const int nb = energy_blocks(n);
-    hipLaunchKernelGGL(k_energy_blocks, dim3(nb), dim3(NT), 0, st, A, box, part);
-    hipLaunchKernelGGL(k_energy_total, dim3(1), dim3(NT), 0, st, nb, part, out);
+    const int rounds = nb > 1 ? 1 : (n + EN_SLOTS - 1) / EN_SLOTS;
+    hipLaunchKernelGGL(k_energy_blocks, dim3(nb), dim3(NT), 0, st, A, box, rounds, part, out);
+    if (nb > 1) hipLaunchKernelGGL(k_energy_total, dim3(1), dim3(NT), 0, st, nb, part, out);
 }
 void launch_fp32_accumulate(long long n, const double *x, int unroll, double *out2, hipStream_t st)
 {

@@ -12,7 +12,7 @@ from pyticles_amd.device import DeviceBox
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 63, 1023, 1024, 1025, 1100])
+@pytest.mark.parametrize("n", [1, 63, 1023, 1024, 1025, 1100, 4096, 4097])
 @pytest.mark.parametrize("big", [math.inf, -math.inf])
 def test_infinite_energy(n, big):
     L = max(8.0, math.sqrt(n))
