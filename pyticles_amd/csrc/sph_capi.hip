@@ -661,7 +661,7 @@ struct Arena {
         hipGraph_t gr;
         HIPCHK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
         for (int j = 0; j < per; ++j) {
-            enqueue_step(with_build, j > 0, j == per - 1);
+            enqueue_step(with_build, j > 0 && !has_tail(per, j - 1), has_tail(per, j));
             swap_state();
         }
         if (per & 1) swap_state();  // nothing ran: back to the buffers that hold the state
@@ -963,19 +963,24 @@ struct Arena {
 
     // A chunk graph's steps but the last need no k_box_step: plain steps of a
     // single box build, review and capture nothing (the review lies in the
-    // last step before a build, the captures in a run's first step, launched
-    // by itself here, and its last one), so all it would do is to count the
-    // step; the next step's density pass, which reads no step count, does that
-    // (one launch less: FP64 1,024 slots 30.6 -> 29.2 us a step, 262,144
-    // slots 102.3 -> 100.3).
+    // last step before a build, the captures in a run's first step and its
+    // last one), so all it would do is to count the step; the next step's
+    // density pass, which reads no step count, does that (one launch less: FP64 1,024 slots 30.6 -> 29.2 us a step, 262,144
+    // slots 102.3 -> 100.3).  Chunks of up to 2^FIRST_LOG2 steps keep their
+    // first step's, so that a run may start with one: its first step as a
+    // launch of its own made short runs slower (one step of 7 particles, two
+    // evaluations: 54 -> 58 us).
+    static constexpr int FIRST_LOG2 = 2;
+    static bool has_tail(int per, int j) { return j == per - 1 || (j == 0 && per <= 1 << FIRST_LOG2); }
     int launch_steps(int64_t count, bool with_build)
     {
         host_dyn_ok = false;  // until every step is launched
         const bool graphs = use_graph && !ctx->timing;
         for (int64_t i = 0; i < count;) {
             int lg = 0;  // runs of plain steps: the largest chunk graph that fits
-            if (graphs && !with_build && !run_first)
-                while (lg < PLAIN_LOG2 && (int64_t)2 << lg <= count - i) ++lg;
+            const int most = run_first ? FIRST_LOG2 : PLAIN_LOG2;
+            if (graphs && !with_build)
+                while (lg < most && (int64_t)2 << lg <= count - i) ++lg;
             run_first = false;
             const int per = 1 << lg;
             const int idx = lg > 0 ? 1 + lg : (with_build ? 1 : 0);
