@@ -1802,21 +1802,38 @@ int sph_separations(sph_box *box, int64_t nip, const int64_t *iap, double *drij,
     const size_t bytes = sizeof(long long) * 2 * nip + sizeof(double) * 6 * nip;
     if (A.stage(bytes)) return SPH_ERR_NOMEM;
     long long *d_iap = (long long *)A.d_stage;
-    double *o = (double *)(d_iap + 2 * nip);
-    double *d_drij = drij ? o : nullptr;
-    double *d_dv = dv ? o + 2 * nip : nullptr;
-    double *d_rij = rij ? o + 4 * nip : nullptr;
-    double *d_rsq = rsq ? o + 5 * nip : nullptr;
-    HIPCHK(hipMemcpyAsync(d_iap, iap, sizeof(long long) * 2 * nip, hipMemcpyHostToDevice, st));
-    launch_inverse(A.id, A.boxes[box->b].part_off, n, A.d_inv, st);
-    launch_separations(A.view(), box->b, A.d_inv, nip, d_iap, d_drij, d_rij, d_rsq, d_dv, st);
-    HIPCHK(hipGetLastError());
+    // (the asked ones one behind another: one download)
+    double *const o = (double *)(d_iap + 2 * nip), *end = o;
+    Arena::Piece piece[4];
+    int pieces = 0;
+    auto out = [&](double *host, size_t words) -> double * {
+        if (!host) return nullptr;
+        piece[pieces++] = {host, words};
+        end += words;
+        return end - words;
+    };
     const size_t k = (size_t)nip;
-    const struct { double *src; Arena::Piece to; } out[] = {
-        {d_drij, {drij, 2 * k}}, {d_dv, {dv, 2 * k}}, {d_rij, {rij, k}}, {d_rsq, {rsq, k}}};
-    for (auto &c : out)
-        if (c.src)
-            if (int rc = A.to_host(c.src, &c.to, 1)) return rc;
+    double *d_drij = out(drij, 2 * k), *d_dv = out(dv, 2 * k), *d_rij = out(rij, k), *d_rsq = out(rsq, k);
+    {
+        // pairs that fit the feed are read from there (a pageable copy of
+        // 125 KB took 45 us longer now and then), more are copied
+        const size_t iap_bytes = sizeof(long long) * 2 * k;
+        std::unique_lock<std::mutex> lk(A.ctx->feed_mu, std::defer_lock);
+        const long long *src = d_iap;
+        if (iap_bytes <= sph_ctx::FEED_HALF) {
+            lk.lock();
+            char *fh, *fd;
+            if (int rc = A.ctx->feed(iap_bytes, &fh, &fd)) return rc;
+            memcpy(fh, iap, iap_bytes);
+            src = (const long long *)fd;
+        } else {
+            HIPCHK(hipMemcpyAsync(d_iap, iap, iap_bytes, hipMemcpyHostToDevice, st));
+        }
+        launch_inverse(A.id, A.boxes[box->b].part_off, n, A.d_inv, st);
+        launch_separations(A.view(), box->b, A.d_inv, nip, src, d_drij, d_rij, d_rsq, d_dv, st);
+        HIPCHK(hipGetLastError());
+    }
+    if (int rc = A.to_host(o, piece, pieces)) return rc;
     HIPCHK(hipStreamSynchronize(st));
     return SPH_OK;
 }
