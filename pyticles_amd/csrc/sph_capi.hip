@@ -2399,7 +2399,9 @@ static constexpr int64_t SPLASH_FINE_CELLS = 65536;
 // (xmax, ymax) as interpolate.py:79 uses them.
 // Its cells are the coarsest a rendering takes; the device refines them to
 // the particles' reach (splash_fine) up to max_cells: about one particle a
-// cell, at most 65,536 (two passes of the cell sort).
+// cell, at most 65,536 (two passes of the cell sort), 256 of few particles
+// (one pass: a call of 1,000 particles, cutoff 2, on 1 x 300 pixels 125 -> 108
+// us with the launch that SPLASH_FEW saves too).
 static int splash_grid(const double *bounds, double cutoff, int64_t n, SplashGrid &G)
 {
     memset(&G, 0, sizeof(G));
@@ -2411,7 +2413,7 @@ static int splash_grid(const double *bounds, double cutoff, int64_t n, SplashGri
     G.ncx = G.ncx < 3 ? 1 : std::min(G.ncx, 4096);
     G.ncy = G.ncy < 3 ? 1 : std::min(G.ncy, 4096);
     G.cwx = Lx / G.ncx; G.cwy = Ly / G.ncy;
-    const int64_t fine = std::min<int64_t>(std::max<int64_t>(n, 256), SPLASH_FINE_CELLS);
+    const int64_t fine = n <= SPLASH_FEW ? 256 : std::min<int64_t>(n, SPLASH_FINE_CELLS);
     G.max_cells = (int)std::max<int64_t>((int64_t)G.ncx * G.ncy, fine);
     return SPH_OK;
 }

@@ -3254,7 +3254,10 @@ __global__ __launch_bounds__(NT) void k_splash_prep(long long n, const double *_
                                                      const double *__restrict__ part, SplashGrid *grid,
                                                      double4 *__restrict__ rec, unsigned *__restrict__ keys)
 {
-    double hm = n > 0 ? part[threadIdx.x & (SPLASH_HB - 1)] : 0.0;
+    double hm = 0.0;  // (of few particles, part = null: every wave looks at all)
+    if (part) hm = part[threadIdx.x & (SPLASH_HB - 1)];
+    else
+        for (long long t = threadIdx.x & 63; t < n; t += 64) hm = fmax(hm, h[t]);
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) hm = fmax(hm, __shfl_xor(hm, off));
     const SplashGrid G = splash_fine(C, hm);
@@ -3586,7 +3589,8 @@ void launch_splash(long long n, const double *r, const double *m, const double *
     double *part = (double *)W.head;
     SplashGrid *grid = (SplashGrid *)((char *)W.head + sizeof(double) * SPLASH_HB);
     static_assert(sizeof(double) * SPLASH_HB + sizeof(SplashGrid) <= SPLASH_HEAD_BYTES, "splash head");
-    if (n > 0) hipLaunchKernelGGL(k_splash_hmax, dim3(SPLASH_HB), dim3(NT), 0, st, n, h, part);
+    if (n <= SPLASH_FEW) part = nullptr;
+    else hipLaunchKernelGGL(k_splash_hmax, dim3(SPLASH_HB), dim3(NT), 0, st, n, h, part);
     hipLaunchKernelGGL(k_splash_prep, grid_for(n), dim3(NT), 0, st, n, r, m, rho, a, h, C, part, grid, W.rec, W.keys);
     if (n > 0) {
         int bits = 1;  // of the largest key the grid may have

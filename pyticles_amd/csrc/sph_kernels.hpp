@@ -74,6 +74,9 @@ void launch_fp32_accumulate(long long n, const double *x, int unroll, double *ou
 // records twice, n keys and values, the sort's counters and C.max_cells + 1
 // cell starts.
 constexpr size_t SPLASH_HEAD_BYTES = 1024;
+// Up to this many particles a rendering takes no launch for their largest
+// smoothing length and at most 256 cells (one pass of the cell sort).
+constexpr int64_t SPLASH_FEW = 1024;
 struct SplashScratch {
     void *head;
     double4 *rec, *rec_sorted;
