@@ -137,6 +137,11 @@ struct sph_ctx {
         render_bytes = 0;
     }
 
+    // Step graphs are captured on a stream of their own: a launch that another
+    // thread makes on the context's stream meanwhile is not captured with them.
+    std::mutex capture_mu;
+    hipStream_t capture_stream = nullptr;
+
     // Pinned host memory that the boxes and arenas of this context share (they
     // share its stream), allocated once: a box that pinned its own paid for it
     // at its first download and its end (1 MB: 0.2-0.5 ms each time), and an
@@ -659,13 +664,16 @@ struct Arena {
         const bool with_build = idx == 1;
         const int per = idx >= 2 ? 1 << (idx - 1) : 1;
         hipGraph_t gr;
-        HIPCHK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
+        std::lock_guard<std::mutex> lk(ctx->capture_mu);
+        if (!ctx->capture_stream) HIPCHK(hipStreamCreateWithFlags(&ctx->capture_stream, hipStreamNonBlocking));
+        const hipStream_t st = ctx->capture_stream;
+        HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
         for (int j = 0; j < per; ++j) {
-            enqueue_step(with_build, j > 0 && !has_tail(per, j - 1), has_tail(per, j));
+            enqueue_step(st, with_build, j > 0 && !has_tail(per, j - 1), has_tail(per, j));
             swap_state();
         }
         if (per & 1) swap_state();  // nothing ran: back to the buffers that hold the state
-        HIPCHK(hipStreamEndCapture(ctx->stream, &gr));
+        HIPCHK(hipStreamEndCapture(st, &gr));
         hipError_t e1 = hipGraphInstantiate(&g, gr, nullptr, nullptr, 0);
         (void)hipGraphDestroy(gr);
         if (e1 != hipSuccess) {
@@ -907,10 +915,9 @@ struct Arena {
     // ---- passes ----------------------------------------------------------
     // Cell order and neighbour lists of every box that builds in this launch
     // (see building() in the kernels); the others keep their order.
-    void enqueue_build(int force_mask)
+    void enqueue_build(hipStream_t st, int force_mask)
     {
         host_dyn_ok = false;  // the build stage writes box states
-        hipStream_t st = ctx->stream;
         ArenaView A = view();
         if (hwm == 0) return;
         // the sort runs over the M building slots (M read on the device);
@@ -932,14 +939,13 @@ struct Arena {
     //
     // advance: the step before this one left its bookkeeping to this one's
     // density pass (tail = false there): see launch_steps.
-    void enqueue_step(bool with_build, bool advance = false, bool tail = true)
+    void enqueue_step(hipStream_t st, bool with_build, bool advance = false, bool tail = true)
     {
-        hipStream_t st = ctx->stream;
         ArenaView A = view();
         const int f = fp32() ? 1 : 0;
         if (with_build) {
             mark(T_SORT, true);
-            enqueue_build(0);
+            enqueue_build(st, 0);
             mark(T_SORT, false);
         }
         mark(T_DENS, true);
@@ -993,7 +999,7 @@ struct Arena {
                 HIPCHK(hipGraphLaunch(graph[need_grad][parity][idx], ctx->stream));
                 if (per & 1) swap_state();
             } else {
-                enqueue_step(with_build);
+                enqueue_step(ctx->stream, with_build);
                 swap_state();
             }
         }
@@ -1226,7 +1232,7 @@ struct Arena {
     {
         for (int held = 0;;) {
             const int64_t rel = released;
-            enqueue_build(force_mask);
+            enqueue_build(ctx->stream, force_mask);
             HIPCHK(hipGetLastError());
             if (int rc = read_dyn()) return rc;
             if (released == rel) return SPH_OK;
@@ -1573,6 +1579,7 @@ int sph_ctx_destroy(sph_ctx *ctx)
     dfree(ctx->d_scratch);
     dfree(ctx->d_render);
     ctx->release_pinned();
+    if (ctx->capture_stream) (void)hipStreamDestroy(ctx->capture_stream);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return SPH_OK;
@@ -2130,7 +2137,7 @@ int sph_box_time_pass(sph_box *box, int pass, int reps, double *us_per_launch)
             if (pass == 0) launch_density(V, f, MASK_ALL, A.unroll, st);
             else if (pass == 1) launch_grad(V, f, MASK_ALL, 0, A.unroll, st);
             else if (pass == 2) launch_rates(V, f, MASK_ALL, A.rates_unroll(), 0, st);
-            else A.enqueue_build(MASK_ALL);
+            else A.enqueue_build(st, MASK_ALL);
         }
         e = hipGetLastError();
     }
