@@ -376,7 +376,6 @@ struct Arena {
     // runs with an unbounded step count, so no step is its closing one
     bool open_run = false;
     int64_t open_plain = 0;  // next steps known not to build
-    bool run_first = false;  // the next step launched is a run's first
     bool need_grad = true;   // some live box has viscosity or conduction (set by relayout)
     // the single box's lists are still valid for its state: its last run
     // ended without a health bit and no upload, parameter change, relayout
@@ -669,7 +668,7 @@ struct Arena {
         const hipStream_t st = ctx->capture_stream;
         HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
         for (int j = 0; j < per; ++j) {
-            enqueue_step(st, with_build, j > 0 && !has_tail(per, j - 1), has_tail(per, j));
+            enqueue_step(st, with_build, j > 0, j == per - 1);
             swap_state();
         }
         if (per & 1) swap_state();  // nothing ran: back to the buffers that hold the state
@@ -968,26 +967,20 @@ struct Arena {
     }
 
     // A chunk graph's steps but the last need no k_box_step: plain steps of a
-    // single box build, review and capture nothing (the review lies in the
-    // last step before a build, the captures in a run's first step and its
-    // last one), so all it would do is to count the step; the next step's
-    // density pass, which reads no step count, does that (one launch less: FP64 1,024 slots 30.6 -> 29.2 us a step, 262,144
-    // slots 102.3 -> 100.3).  Chunks of up to 2^FIRST_LOG2 steps keep their
-    // first step's, so that a run may start with one: its first step as a
-    // launch of its own made short runs slower (one step of 7 particles, two
-    // evaluations: 54 -> 58 us).
-    static constexpr int FIRST_LOG2 = 2;
-    static bool has_tail(int per, int j) { return j == per - 1 || (j == 0 && per <= 1 << FIRST_LOG2); }
+    // single box build nothing, the review lies in the last step before a
+    // build, and the one at the chunk's end takes the energies of a run's first
+    // step (step_tail keeps them apart) and its last one.  All the others would
+    // do is to count the step; the next step's density pass, which reads no
+    // step count, does that (one launch less: FP64 1,024 slots 30.6 -> 29.2 us
+    // a step, 262,144 slots 102.3 -> 100.3).
     int launch_steps(int64_t count, bool with_build)
     {
         host_dyn_ok = false;  // until every step is launched
         const bool graphs = use_graph && !ctx->timing;
         for (int64_t i = 0; i < count;) {
             int lg = 0;  // runs of plain steps: the largest chunk graph that fits
-            const int most = run_first ? FIRST_LOG2 : PLAIN_LOG2;
             if (graphs && !with_build)
-                while (lg < most && (int64_t)2 << lg <= count - i) ++lg;
-            run_first = false;
+                while (lg < PLAIN_LOG2 && (int64_t)2 << lg <= count - i) ++lg;
             const int per = 1 << lg;
             const int idx = lg > 0 ? 1 + lg : (with_build ? 1 : 0);
             i += per;
@@ -1028,7 +1021,6 @@ struct Arena {
     int run_start(int b, int64_t nsteps, BoxDyn &D, int64_t &plain)
     {
         memset(&D, 0, sizeof(D));
-        run_first = true;
         D.state = BOX_RUN;
         D.k = 0;
         D.nsteps = nsteps;

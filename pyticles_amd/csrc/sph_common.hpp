@@ -112,6 +112,8 @@ struct BoxDyn {
     int relist;     // a build met a neighbour offset beyond 16 bits: the box holds
                     // (no pass, integration or bookkeeping) until the runtime has
                     // switched it to 32-bit entries and cleared this
+    int cap0;       // E0 of this run is taken (k_box_step)
+    int pad;
 };
 
 // Segment of the slot space: a box or a free range, sorted by offset.
@@ -149,7 +151,8 @@ struct ArenaView {
     unsigned *rlo_nx;
     double *u, *m, *up, *udot;
     int *id;
-    // sorted scratch written by the permutation of a build
+    // sorted scratch written by the permutation of a build; between builds
+    // udot_s and up_s hold the energies of a run's first step (integrate_slot)
     double2 *r_s, *v_s, *vp_s, *acc_s;
     double *u_s, *m_s, *up_s, *udot_s;
     int *id_s;
@@ -193,7 +196,7 @@ struct ArenaView {
     double2 *wbuild;     // per 64-slot wave wholly inside one building box: its largest
                          // squared predicted speed and acceleration, stored at the build
     double *wenergy;     // per 64-slot wave wholly inside one box: the sum of its slots'
-                         // energies, stored on the box's first and last step
+                         // energies, stored on the box's last step (its first step's: up_s)
     // boxes
     const BoxDesc *boxes;
     BoxDyn *dyn;

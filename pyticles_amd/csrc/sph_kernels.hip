@@ -2320,9 +2320,14 @@ __device__ __forceinline__ void rates32_walk(const ArenaView &A, const BoxF &F, 
 // Leapfrog step of slot s of running box b with this evaluation's rates
 // (a, ud); returns the squared displacement since the box's last build (-1
 // at the closing half kick, which moves nothing).  On the box's first and
-// last step, cap is set and e holds the slot's energy.
+// last step, cap says which (CAP_*) and e holds the slot's energy, also stored
+// per slot: the first step's apart, in a build's scratch arrays (udot_s and,
+// per wave, up_s), so that a chunk of steps without a build may end before
+// k_box_step takes it, the last one's sums beside it.
+enum : int { CAP_NONE = 0, CAP_FIRST, CAP_LAST };
+
 __device__ __forceinline__ double integrate_slot(const ArenaView &A, int fp32, int s, int b, const CBox &B, const CDyn &D,
-                                                 double2 a, double ud, double &e, bool &cap)
+                                                 double2 a, double ud, double &e, int &cap)
 {
     const int64_t k = D.k, K = D.nsteps;
     const double kick = (k == 0 || k == K) ? 0.5 * B.dt : B.dt;
@@ -2330,8 +2335,8 @@ __device__ __forceinline__ double integrate_slot(const ArenaView &A, int fp32, i
     const double u = A.u[s], m = A.m[s];
     if (k == 0) {
         e = m * (0.5 * (v.x * v.x + v.y * v.y) + u);
-        A.e[s] = e;
-        cap = true;
+        A.udot_s[s] = e;
+        cap = CAP_FIRST;
     }
     const double vx = v.x + kick * a.x, vy = v.y + kick * a.y;
     const double un = u + kick * ud;
@@ -2340,8 +2345,8 @@ __device__ __forceinline__ double integrate_slot(const ArenaView &A, int fp32, i
     const double2 r = A.r[s];
     if (k == K) {
         e = m * (0.5 * (vx * vx + vy * vy) + un);
-        A.e[s] = e;
-        cap = true;
+        (k == 0 ? A.udot_s : A.e)[s] = e;
+        cap = k == 0 ? CAP_FIRST : CAP_LAST;
         A.r_nx[s] = r;
         A.vp_nx[s] = make_double2(vx, vy);
         A.up[s] = un;
@@ -2408,7 +2413,8 @@ __device__ __forceinline__ bool list_review(const Dyn &D)
 __device__ __forceinline__ void step_tail(const ArenaView &A, int fp32, int s, int b, double2 a, double ud)
 {
     double d2 = 0.0, e = 0.0;
-    bool review = false, cap = false;
+    bool review = false;
+    int cap = CAP_NONE;
     per_box(b, [&](int bu) {
         CDyn &D = cdyn(A, bu);
         if (takes_part(D, 1 << BOX_RUN)) {
@@ -2423,11 +2429,11 @@ __device__ __forceinline__ void step_tail(const ArenaView &A, int fp32, int s, i
     const bool whole = bfirst >= 0 && bfirst == __shfl(b, 63);  // wholly inside one box
     // a box's first or last step: a whole wave's energy sum (fixed shuffle
     // order, every lane the same total) for k_box_step; the box's lanes in
-    // shared waves it sums from e itself
-    if (whole && __ballot(cap) != 0ull) {
+    // shared waves it sums from the slots' energies itself
+    if (whole && __ballot(cap != CAP_NONE) != 0ull) {
 #pragma unroll
         for (int off = 32; off >= 1; off >>= 1) e += __shfl_xor(e, off);
-        if (lane == 0) A.wenergy[s >> 6] = e;
+        if (lane == 0) (cap == CAP_FIRST ? A.up_s : A.wenergy)[s >> 6] = e;
     }
     uint64_t pending = __ballot(review);
     if (pending == 0ull) return;
@@ -2648,7 +2654,8 @@ __global__ __launch_bounds__(NT_BOX) void k_box_step(ArenaView A, int nbox)
     }
     const int state = D.state;
     const int64_t k = D.k, K = D.nsteps;
-    const bool capture = state == BOX_RUN && (k == 0 || k == K);
+    // the run's first step, in this launch or an earlier one of its chunk, and its last
+    const bool first = state == BOX_RUN && !D.cap0, last = state == BOX_RUN && k == K && k != 0;
     const bool review = list_review(D);
     const bool built = building(D, 0);
     __shared__ double red[NT_BOX];
@@ -2693,40 +2700,45 @@ __global__ __launch_bounds__(NT_BOX) void k_box_step(ArenaView A, int nbox)
         dmax2 = fmax(red[0], __longlong_as_double((long long)D.dmax2));
         __syncthreads();  // red is reused below
     }
-    if (capture) {
-        // the step pass's sums of the box's whole waves (wenergy), then the
-        // box's slots in waves it shares (at most 63 at each end)
+    // an energy capture: the step pass's sums of the box's whole waves, then the
+    // box's slots in waves it shares (at most 63 at each end); thread 0's result
+    auto total = [&](const double *wave, const double *slot) {
         const BoxDesc &B = A.boxes[b];
-        const int w0 = (B.part_off + 63) >> 6, w1 = ((B.part_off + B.n) >> 6) - 1;
+        const int s0 = B.part_off, s1 = B.part_off + B.n;
+        const int w0 = (s0 + 63) >> 6, w1 = (s1 >> 6) - 1;
         double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
         int w = w0 + (int)threadIdx.x;
         for (; w + 3 * NT_BOX <= w1; w += 4 * NT_BOX) {
-            a0 += A.wenergy[w];
-            a1 += A.wenergy[w + NT_BOX];
-            a2 += A.wenergy[w + 2 * NT_BOX];
-            a3 += A.wenergy[w + 3 * NT_BOX];
+            a0 += wave[w];
+            a1 += wave[w + NT_BOX];
+            a2 += wave[w + 2 * NT_BOX];
+            a3 += wave[w + 3 * NT_BOX];
         }
-        for (; w <= w1; w += NT_BOX) a0 += A.wenergy[w];
+        for (; w <= w1; w += NT_BOX) a0 += wave[w];
         red[threadIdx.x] = (a0 + a1) + (a2 + a3);
         __syncthreads();
         for (int off = NT_BOX / 2; off > 0; off >>= 1) {
             if (threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
             __syncthreads();
         }
-    }
+        const double whole = red[0];
+        __syncthreads();  // red may be reused
+        double ends = 0.0;
+        if (threadIdx.x == 0) {
+            const int h1 = min(((s0 + 63) >> 6) << 6, s1), t0 = max((s1 >> 6) << 6, h1);
+            for (int s = s0; s < h1; ++s) ends += slot[s];
+            for (int s = t0; s < s1; ++s) ends += slot[s];
+        }
+        return whole + ends;
+    };
+    const double E0 = first ? total(A.up_s, A.udot_s) : 0.0, E1 = last ? total(A.wenergy, A.e) : 0.0;
     __syncthreads();  // every thread has read D before thread 0 updates it
     if (threadIdx.x != 0) return;
-    if (capture) {
-        const BoxDesc &B = A.boxes[b];
-        const int s0 = B.part_off, s1 = B.part_off + B.n;
-        const int h1 = min(((s0 + 63) >> 6) << 6, s1), t0 = max((s1 >> 6) << 6, h1);
-        double ends = 0.0;
-        for (int s = s0; s < h1; ++s) ends += A.e[s];
-        for (int s = t0; s < s1; ++s) ends += A.e[s];
-        const double tot = red[0] + ends;
-        if (k == 0) D.E0 = tot;
-        else D.E1 = tot;
+    if (first) {
+        D.E0 = E0;
+        D.cap0 = 1;
     }
+    if (last) D.E1 = E1;
     if (built) {
         D.vlast = sqrt(vmax2);
         D.alast = sqrt(amax2);
