@@ -1794,8 +1794,9 @@ int sph_separations(sph_box *box, int64_t nip, const int64_t *iap, double *drij,
     hipStream_t st = A.ctx->stream;
     HIPCHK(hipSetDevice(A.ctx->device));
     const int n = A.boxes[box->b].n;
-    for (int64_t k = 0; k < 2 * nip; ++k)
-        if (iap[k] < 0 || iap[k] >= n) return fail(SPH_ERR_ARG, "pair index out of range");
+    uint64_t outside = 0;  // its top bit: of an index below 0 or above n - 1
+    for (int64_t k = 0; k < 2 * nip; ++k) outside |= (uint64_t)iap[k] | ((uint64_t)(n - 1) - (uint64_t)iap[k]);
+    if (outside >> 63) return fail(SPH_ERR_ARG, "pair index out of range");
     if (!A.d_inv && dalloc(&A.d_inv, A.cap)) return SPH_ERR_NOMEM;
     // device layout: iap (2*nip int64) then up to 6*nip doubles of outputs
     const size_t bytes = sizeof(long long) * 2 * nip + sizeof(double) * 6 * nip;

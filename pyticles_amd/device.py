@@ -207,6 +207,15 @@ class DeviceBox:
             k = int(nip.value)
             return iap[:k] if 3 * k >= 2 * cap else iap[:k].copy()
 
+    def pairs_into(self, iap):
+        """The pairs of pairs() into the rows of iap (C-contiguous int64
+        [cap, 2]) as far as they fit; returns their number."""
+        nip = ctypes.c_int64()
+        rc = _lib.lib.sph_nlist_build(self._h, iap.shape[0], _lib.i64ptr(iap), ctypes.byref(nip))
+        if rc != _lib.SPH_ERR_CAP:
+            _lib.check(rc)
+        return int(nip.value)
+
     def separations(self, iap):
         iap = np.ascontiguousarray(iap, dtype=np.int64)
         nip = iap.shape[0]
@@ -214,9 +223,14 @@ class DeviceBox:
         dv = np.empty((nip, 2))
         rij = np.empty(nip)
         rsq = np.empty(nip)
-        _lib.check(_lib.lib.sph_separations(self._h, nip, _lib.i64ptr(iap), _lib.dptr(drij), _lib.dptr(rij),
-                                            _lib.dptr(rsq), _lib.dptr(dv)))
+        self.separations_into(iap, drij, rij, rsq, dv)
         return drij, rij, rsq, dv
+
+    def separations_into(self, iap, drij, rij, rsq, dv):
+        """Separations of the pairs iap (C-contiguous int64 [nip, 2]) into
+        C-contiguous float64 arrays of nip rows; None leaves one out."""
+        _lib.check(_lib.lib.sph_separations(self._h, iap.shape[0], _lib.i64ptr(iap), _lib.dptr(drij),
+                                            _lib.dptr(rij), _lib.dptr(rsq), _lib.dptr(dv)))
 
 
 class PinnedState:

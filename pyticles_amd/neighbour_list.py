@@ -80,11 +80,24 @@ class NeighbourList:
         if ni == 0:
             return
         dev = self._device()
+        if self._takes_device_output():
+            dev.separations_into(self.iap[:ni], self.drij, self.rij, self.rsq, self.dv)
+            return
         drij, rij, rsq, dv = dev.separations(self.iap[:ni])
         self.drij[:ni, :2] = drij
         self.rij[:ni] = rij
         self.rsq[:ni] = rsq
         self.dv[:ni, :2] = dv
+
+    def _takes_device_output(self):
+        """Whether the list's arrays are as NeighbourList makes them (a program
+        may have put others in their place), so that the device call can fill
+        them itself."""
+        cap = self.iap.shape[0]
+        return all(type(a) is np.ndarray and a.dtype == t and a.shape == s and a.flags.c_contiguous and a.flags.writeable
+                   for a, t, s in ((self.iap, np.int64, (cap, 2)), (self.drij, np.float64, (cap, 2)),
+                                   (self.dv, np.float64, (cap, 2)), (self.rij, np.float64, (cap,)),
+                                   (self.rsq, np.float64, (cap,))))
 
     def find_pair(self, i, j):
         """Index k of pair (i, j), or -1."""
@@ -131,6 +144,18 @@ class VerletList(NeighbourList):
             self.nip = 0
             return
         dev = self._device()
+        if self._takes_device_output():
+            # straight into the list's own arrays (new ones a call, copied
+            # over, cost page faults: 3 to 5 ms of 20,011 particles' list,
+            # with the state of the allocator)
+            ni = dev.pairs_into(self.iap)
+            if ni > self.iap.shape[0]:
+                _bind.ensure_pair_capacity(self, ni)
+                ni = dev.pairs_into(self.iap)
+            self.nip = ni
+            if ni:
+                dev.separations_into(self.iap[:ni], self.drij, None, self.rsq, self.dv)
+            return
         iap = dev.pairs()
         self._store_pairs(iap)
         ni = self.nip
