@@ -139,6 +139,7 @@ struct sph_ctx {
 
     // Step graphs are captured on a stream of their own: a launch that another
     // thread makes on the context's stream meanwhile is not captured with them.
+    // (Made with the context: a stream's queue takes 3 ms.)
     std::mutex capture_mu;
     hipStream_t capture_stream = nullptr;
 
@@ -664,7 +665,6 @@ struct Arena {
         const int per = idx >= 2 ? 1 << (idx - 1) : 1;
         hipGraph_t gr;
         std::lock_guard<std::mutex> lk(ctx->capture_mu);
-        if (!ctx->capture_stream) HIPCHK(hipStreamCreateWithFlags(&ctx->capture_stream, hipStreamNonBlocking));
         const hipStream_t st = ctx->capture_stream;
         HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
         for (int j = 0; j < per; ++j) {
@@ -1555,6 +1555,10 @@ int sph_ctx_create(int device, sph_ctx **out)
     sph_ctx *c = new sph_ctx();
     c->device = device;
     hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
+    if (e == hipSuccess) {
+        e = hipStreamCreateWithFlags(&c->capture_stream, hipStreamNonBlocking);
+        if (e != hipSuccess) (void)hipStreamDestroy(c->stream);
+    }
     if (e != hipSuccess) {
         delete c;
         return fail(SPH_ERR_HIP, std::string("hipStreamCreate: ") + hipGetErrorString(e));
@@ -1571,7 +1575,7 @@ int sph_ctx_destroy(sph_ctx *ctx)
     dfree(ctx->d_scratch);
     dfree(ctx->d_render);
     ctx->release_pinned();
-    if (ctx->capture_stream) (void)hipStreamDestroy(ctx->capture_stream);
+    (void)hipStreamDestroy(ctx->capture_stream);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return SPH_OK;
