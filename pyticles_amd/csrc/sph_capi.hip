@@ -1373,7 +1373,7 @@ int64_t first_outside(const double *r, int64_t n, double Lx, double Ly)
         }
         in0 &= in1;
         if (in0[0] & in0[1]) continue;
-        for (k = i;; ++k)
+        for (k = i; k < end; ++k)
             if (!(r[2 * k] >= 0.0 && r[2 * k] < Lx && r[2 * k + 1] >= 0.0 && r[2 * k + 1] < Ly)) return k;
     }
     return n;

@@ -2829,7 +2829,7 @@ __global__ __launch_bounds__(NT) void k_put(PutSpans P)
 // n words to host memory, in order, by 16-byte stores where both sides are
 // aligned to them.  (The copy engines took 24 us for 512 KB and its wait, 19
 // for 32 KB, this 22 and 14.  Right after large allocations or frees their
-// queues hold the driver's clears: 32 MB in 8.0 ms, through the runtime's
+// queues hold memory clears: 32 MB in 8.0 ms, through the runtime's
 // pageable path 5.9; this 1.8 at any time.)
 static constexpr size_t TO_HOST_BLOCKS = 64;
 
